@@ -35,6 +35,7 @@
 // (instance, voxel, face, palette index, steps) bit-exact with the CPU oracle.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstddef>
 
@@ -949,46 +950,91 @@ __host__ __device__ __forceinline__ uint32_t* slot_counters(uint32_t* counters, 
     return counters + slot * kParts * kPartStride;
 }
 
-// Each wave takes 64 consecutive items of a part from that part's counter (fetch + p *
-// kPartStride) until the part is exhausted, starting with part blockIdx.x % kParts and then
-// taking the others in turn.  range(p, &first, &count): part p's items are first + [0, count);
-// body(p, item).  `gone` (LDS, zero at start) marks the parts the block has seen exhausted, so
-// only one wave per block spends an atomic on finding that out.
-template <typename Range, typename Body>
-__device__ __forceinline__ void for_each_item(uint32_t* fetch, uint32_t* gone, Range&& range, Body&& body) {
+// Parts and the work a launch hands out without atomics.  Workgroup b belongs to part
+// b % kParts; with own = 1 the waves of part p start on the part's first tiles, one each
+// (wave i of the part on tile i), and only the tiles past those come from the part's counter.
+// A launch whose waves cover its items so needs no atomics at all, where every workgroup would
+// find each of the 8 counters exhausted before it ends: k_render0 on a 320 x 240 frame (1200 tiles)
+// 92 -> 59 us, k_secondary on a 640 x 480 frame's sun rays 81 -> 36 us.
+// own = 0 where the launch's workgroups may not all be resident at once (several streams): a tile
+// kept for a workgroup that starts late would be traced when everything else is done.
+// One part's share, in LDS (registers are what the traversal kernels are short of):
+struct Part {
+    uint32_t first;   // its first item, or (k_secondary) its number of bounce rays
+    uint32_t count;   // its items
+    uint32_t kept;    // items kept for its waves
+    uint32_t left;    // what its counter hands out: tiles (k_secondary: items)
+};
+struct Parts {
+    Part part[kParts];
+    uint32_t gone;    // parts whose counter this workgroup has seen exhausted
+};
+// (threads p < kParts, each for part p, before the workgroup's first barrier; unit: items per
+// counter step)
+__device__ __forceinline__ void put_part(Parts& P, uint32_t first, uint32_t count, uint32_t own, uint32_t unit) {
+    const uint32_t p = threadIdx.x;
+    const uint32_t kept = own ? (gridDim.x + kParts - 1u - p) / kParts * (uint32_t)kBlock : 0u;
+    P.part[p] = Part{first, count, kept, count > kept ? (count - kept + unit - 1u) / unit : 0u};
+    if (p == 0) P.gone = 0u;
+}
+// This wave's index among the waves of its part.
+__device__ __forceinline__ uint32_t part_wave() {
+    return blockIdx.x / kParts * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u);
+}
+// The parts with entries left to hand out, as far as this workgroup knows (wave-uniform).
+__device__ __forceinline__ uint32_t open_parts(const Parts& P) {
     const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t open = (uint32_t)__ballot(lane < kParts && P.part[lane % kParts].left > 0u);
+    return __builtin_amdgcn_readfirstlane(
+        open & ~__hip_atomic_load(&P.gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+// The first part at or after p0 with its bit set in `open`.
+__device__ __forceinline__ uint32_t next_part(uint32_t open) {
     const uint32_t p0 = blockIdx.x % kParts;
-    for (uint32_t k = 0; k < kParts; ++k) {
-        const uint32_t p = (p0 + k) % kParts;
-        uint32_t first = 0, count = 0;
-        range(p, &first, &count);
-        const uint32_t tiles = (count + 63u) / 64u;
-        for (;;) {
-            if (__hip_atomic_load(gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & (1u << p)) break;
-            uint32_t t = tiles;
-            if (tiles > 0 && lane == 0) t = atomicAdd(fetch + p * kPartStride, 1u);
-            t = __shfl(t, 0, 64);
-            if (t >= tiles) {
-                if (lane == 0) __hip_atomic_fetch_or(gone, 1u << p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                break;
+    return (p0 + (uint32_t)__ffs((int)((open | (open << kParts)) >> p0)) - 1u) % kParts;
+}
+// Part p's counter has passed its end: no other wave of the workgroup asks it again.  (Reading all
+// eight counters here instead, to skip every empty part at once, cost 0.1 ms a launch: their lines
+// are then shared by all XCDs while the atomics still run.)
+__device__ __forceinline__ void mark_gone(Parts& P, uint32_t p) {
+    if ((threadIdx.x & 63u) == 0) __hip_atomic_fetch_or(&P.gone, 1u << p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Each wave takes 64 consecutive items of a part at a time until all parts are exhausted: its own
+// tile first, then tiles of its part from that part's counter (fetch + p * kPartStride), then of
+// the others in turn.  body(item): part p's items are P.part[p].first + [0, count).
+template <typename Body>
+__device__ __forceinline__ void for_each_item(uint32_t* fetch, Parts& P, uint32_t own, Body&& body) {
+    const uint32_t lane = threadIdx.x & 63u;
+    bool start = own != 0u;
+    for (;;) {
+        uint32_t p = blockIdx.x % kParts, i;
+        if (start) {
+            start = false;
+            i = 64u * part_wave();
+        } else {
+            const uint32_t open = open_parts(P);
+            if (open == 0u) break;
+            p = next_part(open);
+            uint32_t t = 0;
+            if (lane == 0) t = atomicAdd(fetch + p * kPartStride, 1u);
+            t = __builtin_amdgcn_readfirstlane(t);
+            if (t >= P.part[p].left) {
+                mark_gone(P, p);
+                continue;
             }
-            const uint32_t i = t * 64u + lane;
-            if (i < count) body(p, first + i);
+            i = P.part[p].kept + 64u * t;
         }
+        i += lane;
+        if (i < P.part[p].count) body(P.part[p].first + i);
     }
 }
 
-// Items [0, nwork) in kParts contiguous ranges of whole 64-item tiles.
-__device__ __forceinline__ void static_part(uint32_t nwork, uint32_t p, uint32_t* first, uint32_t* count) {
-    const uint32_t tiles = (nwork + 63u) / 64u;
+// Items [0, nwork) in kParts contiguous ranges of whole 64-item tiles (threads p < kParts).
+__device__ __forceinline__ void put_static_part(Parts& P, uint32_t nwork, uint32_t own) {
+    const uint32_t tiles = (nwork + 63u) / 64u, p = threadIdx.x;
     const uint32_t t0 = (uint32_t)((uint64_t)tiles * p / kParts), t1 = (uint32_t)((uint64_t)tiles * (p + 1u) / kParts);
-    *first = t0 * 64u;
-    *count = min(t1 * 64u, nwork) - min(t0 * 64u, nwork);
-}
-
-// Slots used in segment p of a queue (its counter can pass seg_cap, see append_slot).
-__device__ __forceinline__ uint32_t queue_count(uint32_t* q, uint32_t p, uint32_t cap) {
-    return min(q[p * kPartStride], cap);
+    put_part(P, t0 * 64u, min(t1 * 64u, nwork) - min(t0 * 64u, nwork), own, 64u);
 }
 
 // Wave-aggregated append to queue counters q (segments of `cap` slots): the wave's appending
@@ -1151,21 +1197,18 @@ struct TileMap {
 
 template <bool ST, bool DEEP>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_primary(const ReqGPU* __restrict__ reqs, const BatchGPU* __restrict__ B,
-                                                    const float* __restrict__ srgb_dec, WF wf,
+                                                    const float* __restrict__ srgb_dec, WF wf, uint32_t own,
                                                     unsigned long long* stats) {
     __shared__ uint32_t smem[(kStackLds + 16) * kBlock];
     __shared__ BvhNode tree_lds[kLdsNodes];
     const Lds stk{&smem[threadIdx.x]}, mslot{&smem[kStackLds * kBlock + threadIdx.x]};
-    __shared__ uint32_t gone;
-    if (threadIdx.x == 0) gone = 0u;
+    __shared__ Parts parts;
+    const uint32_t nreq = B->nreq;
+    if (threadIdx.x < kParts) put_static_part(parts, B->work_base[nreq], own);
     const TreeLds tree = stage_tree(reqs, B, tree_lds);
     __syncthreads();
     Ctr<ST> ctr;
-    const uint32_t nreq = B->nreq;
-    const uint32_t nwork = B->work_base[nreq];
-    for_each_item(slot_counters(wf.counters, 2), &gone,
-                  [&](uint32_t p, uint32_t* first, uint32_t* count) { static_part(nwork, p, first, count); },
-                  [&](uint32_t, uint32_t w) {
+    for_each_item(slot_counters(wf.counters, 2), parts, own, [&](uint32_t w) {
         // the 64 items of a wave share a request (work ranges are 64-aligned)
         const uint32_t r = __builtin_amdgcn_readfirstlane(find_req(B->work_base, nreq, w));
         const ReqGPU& Rq = reqs[r];
@@ -1270,26 +1313,30 @@ constexpr uint32_t kPoolLow = 8;
 template <bool ST, bool DEEP, bool ONE>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_secondary(
     const ReqGPU* __restrict__ reqs, const BatchGPU* __restrict__ B, const float* __restrict__ srgb_dec, WF wf,
-    uint32_t q, uint32_t depth, uint32_t in_idx, uint32_t out_idx, uint32_t fetch_idx, uint32_t bounce,
+    uint32_t q, uint32_t depth, uint32_t in_idx, uint32_t out_idx, uint32_t fetch_idx, uint32_t bounce, uint32_t own,
     unsigned long long* stats) {
     __shared__ uint32_t smem[(kStackLds + 16) * kBlock];
     __shared__ BvhNode tree_lds[kLdsNodes];
     const Lds stk_lds{&smem[threadIdx.x]}, mslot{&smem[kStackLds * kBlock + threadIdx.x]};
-    __shared__ uint32_t gone;
-    if (threadIdx.x == 0) gone = 0u;
+    // part p: the bounce rays of segment p of this depth's queue, then the rays of its sun list (the
+    // queue is complete, so its counts are read once)
+    __shared__ Parts parts;
+    const uint32_t cap = wf.seg_cap;
+    if (threadIdx.x < kParts) {
+        const uint32_t at = threadIdx.x * kPartStride;
+        const uint32_t cb = slot_counters(wf.counters, in_idx)[at], cs = slot_counters(wf.counters, sun_slot(in_idx))[at];
+        const uint32_t nb = bounce ? min(cb, cap) : 0u;
+        put_part(parts, nb, nb + min(cs, cap), own, 1u);
+    }
     const TreeLds tree = stage_tree(reqs, B, tree_lds);
     __syncthreads();
     Ctr<ST> ctr;
-    uint32_t* const qin = slot_counters(wf.counters, in_idx);
-    uint32_t* const qsun = slot_counters(wf.counters, sun_slot(in_idx));
     uint32_t* const fetch = slot_counters(wf.counters, fetch_idx);
-    const uint32_t cap = wf.seg_cap;
     const uint32_t nq = 1u - q;
     const uint32_t nreq = B->nreq;
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64u - lane));
-    const uint32_t p0 = blockIdx.x % kParts;
-    uint32_t kp = 0;   // parts this wave has found exhausted, in the order p0, p0 + 1, ... (uniform)
+    bool start = own != 0u, more = true;   // more: the parts may hold items yet (uniform)
 
     // per-lane item and ray state
     bool busy = false, walking = false, is_bounce = false;
@@ -1312,40 +1359,41 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
         // -- take items for the idle lanes (consecutive items of one part in lane order) --
         const uint64_t idle = __ballot(!busy);
         bool fresh = false;
-        uint32_t item = 0, ipart = 0, inb_count = 0;
-        if (idle != 0ull && kp < kParts) {
+        uint32_t item = 0, ipart = 0;
+        if (idle != 0ull && more) {
             const uint32_t need = (uint32_t)__popcll(idle);
             const uint32_t rank = (uint32_t)__popcll(idle & below);
             uint32_t placed = 0;
-            while (placed < need && kp < kParts) {
-                const uint32_t p = (p0 + kp) % kParts;
-                const bool g = (__hip_atomic_load(&gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & (1u << p)) != 0u;
-                uint32_t take = 0, base = 0, nb_p = 0;
-                if (!g) {
-                    // (both counts loaded before either is used: one round trip)
-                    const uint32_t cb = qin[p * kPartStride], cs = qsun[p * kPartStride];
-                    nb_p = bounce ? min(cb, cap) : 0u;
-                    const uint32_t count = nb_p + min(cs, cap);
-                    if (lane == 0 && count > 0) base = atomicAdd(fetch + p * kPartStride, need - placed);
-                    base = __shfl(base, 0, 64);
-                    take = base < count ? min(count - base, need - placed) : 0u;
+            while (placed < need) {
+                uint32_t p = blockIdx.x % kParts, base, end;
+                const bool kept = start;
+                if (kept) {   // the tile kept for this wave
+                    start = false;
+                    base = 64u * part_wave();
+                    end = parts.part[p].count;
+                } else {
+                    const uint32_t open = open_parts(parts);
+                    more = open != 0u;
+                    if (!more) break;
+                    p = next_part(open);
+                    base = 0;
+                    if (lane == 0) base = atomicAdd(fetch + p * kPartStride, need - placed);
+                    base = __builtin_amdgcn_readfirstlane(base) + parts.part[p].kept;
+                    end = parts.part[p].count;
                 }
+                const uint32_t take = base < end ? min(end - base, need - placed) : 0u;
                 if (!busy && rank >= placed && rank < placed + take) {
                     fresh = true;
                     item = base + (rank - placed);
                     ipart = p;
-                    inb_count = nb_p;
                 }
                 placed += take;
-                if (placed < need) {   // part p has no items left
-                    if (lane == 0 && !g) __hip_atomic_fetch_or(&gone, 1u << p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    ++kp;
-                }
+                if (!kept && placed < need) mark_gone(parts, p);
             }
         }
         // -- set up the new items' rays: the origin walk first --
         if (fresh) {
-            const uint32_t nb = inb_count;   // bounce items of part ipart (read at the refill)
+            const uint32_t nb = parts.part[ipart].first;   // bounce items of part ipart
             is_bounce = item < nb;
             const uint32_t slot = is_bounce ? ipart * cap + item : wf.sun[q][ipart * cap + (item - nb)];
             const QueueRec sf = get_rec(&wf.rec[q][slot]);
@@ -1402,7 +1450,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
         for (;;) {
             if (walking) walking = box_walk_step<ST>(W, ctr, mslot);
             const uint32_t nw = (uint32_t)__popcll(__ballot(walking));
-            if (nw == 0u || (nw < kPoolLow && kp < kParts)) break;
+            if (nw == 0u || (nw < kPoolLow && more)) break;
         }
         // -- lanes whose walk ended: keep its hit, then the next instance or the ray's end --
         bool fin = false;
@@ -1622,16 +1670,16 @@ __global__ void k_zero_counters(uint32_t* c) {
 template <bool ST, bool DEEP>
 __global__ __launch_bounds__(kBlock) void k_render0(const FrameGPU F, const SceneGPU S, const float* __restrict__ srgb_dec,
                                                     HitRecord* __restrict__ hits, float4* __restrict__ rad,
-                                                    uint32_t* fetch, uint32_t nwork, unsigned long long* stats) {
+                                                    uint32_t* fetch, uint32_t nwork, uint32_t own,
+                                                    unsigned long long* stats) {
     __shared__ uint32_t smem[(kStackLds + 16) * kBlock];
     const Lds stk{&smem[threadIdx.x]}, mslot{&smem[kStackLds * kBlock + threadIdx.x]};
-    __shared__ uint32_t gone;
-    if (threadIdx.x == 0) gone = 0u;
+    __shared__ Parts parts;
+    if (threadIdx.x < kParts) put_static_part(parts, nwork, own);
     __syncthreads();
     Ctr<ST> ctr;
     const uint32_t spp = F.spp ? F.spp : 1u;
-    for_each_item(fetch, &gone, [&](uint32_t p, uint32_t* first, uint32_t* count) { static_part(nwork, p, first, count); },
-                  [&](uint32_t, uint32_t w) {
+    for_each_item(fetch, parts, own, [&](uint32_t w) {
         uint32_t px, py, s0;
         if (!work_pixel(F, w, 1u, &px, &py, &s0)) return;
         const uint32_t pix = py * F.width + px;
@@ -1812,7 +1860,15 @@ static int launch_batch(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long
                         uint8_t* kinds, uint32_t* nstages, hipStream_t s, hipEvent_t acc_after = nullptr,
                         bool with_acc = true, uint32_t blocks = 0, bool allow_one = true) {
     const uint32_t nblk = blocks ? blocks : g_persistent_blocks;
-    const dim3 grid(nblk), block(kBlock);
+    // Alone on the GPU (blocks = 0), every workgroup of a launch is resident, so its waves start on
+    // tiles of their own, and a launch has no more workgroups than its work has tiles for them: at
+    // most nwork items in the primary launch, one bounce and one sun ray of each in the others.  A
+    // captured launch sequence (nwork = 0 here) runs with any batch, so it keeps the full grid.
+    const uint32_t nwork = Bh.work_base[Bh.nreq], own = blocks == 0u && nwork != 0u ? 1u : 0u;
+    auto grid_of = [&](uint64_t items) {
+        return dim3(own ? (uint32_t)std::min<uint64_t>(nblk, (items + kBlock - 1) / kBlock) : nblk);
+    };
+    const dim3 grid = grid_of(nwork), grid2 = grid_of(2ull * nwork), block(kBlock);
     const ReqGPU* reqs = reinterpret_cast<const ReqGPU*>(wb.tables);
     const BatchGPU* B = reinterpret_cast<const BatchGPU*>(static_cast<const char*>(wb.tables) + sizeof(ReqGPU) * VT_MAX_BATCH);
     WF wf = to_wf(wb);
@@ -1828,18 +1884,19 @@ static int launch_batch(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long
     auto st_at = [&](uint32_t k) { return stats ? stats + (size_t)k * VT_STAT_COUNT : nullptr; };
     hipLaunchKernelGGL(k_zero_counters, dim3(kSlots * kParts / 256), dim3(256), 0, s, wb.counters);
     begin(VT_STAGE_PRIMARY);
-    hipLaunchKernelGGL((k_primary<ST, DEEP>), grid, block, 0, s, reqs, B, g_srgb_dec, wf, st_at(stage));
+    hipLaunchKernelGGL((k_primary<ST, DEEP>), grid, block, 0, s, reqs, B, g_srgb_dec, wf, own,
+                       st_at(stage));
     end();
     uint32_t fetch = 3, in_idx = 0;
     for (uint32_t d = 0; d <= Bh.max_bounces && fetch < kQueueCounters && kQueueCounters + d + 1 < kSlots; ++d) {
         const uint32_t out_idx = kQueueCounters + d + 1;
         begin(VT_STAGE_SECONDARY);
         if (allow_one && Bh.nreq == 1)
-            hipLaunchKernelGGL((k_secondary<ST, DEEP, true>), grid, block, 0, s, reqs, B, g_srgb_dec, wf, d & 1u, d,
-                               in_idx, out_idx, fetch, d < Bh.max_bounces ? 1u : 0u, st_at(stage));
+            hipLaunchKernelGGL((k_secondary<ST, DEEP, true>), grid2, block, 0, s, reqs, B, g_srgb_dec, wf, d & 1u, d,
+                               in_idx, out_idx, fetch, d < Bh.max_bounces ? 1u : 0u, own, st_at(stage));
         else
-            hipLaunchKernelGGL((k_secondary<ST, DEEP, false>), grid, block, 0, s, reqs, B, g_srgb_dec, wf, d & 1u, d,
-                               in_idx, out_idx, fetch, d < Bh.max_bounces ? 1u : 0u, st_at(stage));
+            hipLaunchKernelGGL((k_secondary<ST, DEEP, false>), grid2, block, 0, s, reqs, B, g_srgb_dec, wf, d & 1u, d,
+                               in_idx, out_idx, fetch, d < Bh.max_bounces ? 1u : 0u, own, st_at(stage));
         ++fetch;
         end();
         in_idx = out_idx;
@@ -1941,8 +1998,9 @@ static int launch_render0(const FrameGPU& F, const SceneGPU& S, HitRecord* hits,
     hipLaunchKernelGGL(k_zero_counters, dim3(kSlots * kParts / 256), dim3(256), 0, s, wb.counters);
     if (ev) hipEventRecord(ev[0], s);
     if (kinds) kinds[0] = VT_STAGE_RENDER0;
-    hipLaunchKernelGGL((k_render0<ST, DEEP>), dim3(g_persistent_blocks), dim3(kBlock), 0, s, F, S, g_srgb_dec, hits,
-                       rad, slot_counters(wb.counters, 2), tiles * 64u, stats);
+    const uint32_t grid = std::min(g_persistent_blocks, (tiles * 64u + kBlock - 1) / kBlock);
+    hipLaunchKernelGGL((k_render0<ST, DEEP>), dim3(grid), dim3(kBlock), 0, s, F, S, g_srgb_dec, hits, rad,
+                       slot_counters(wb.counters, 2), tiles * 64u, 1u, stats);
     if (ev) hipEventRecord(ev[1], s);
     if (nstages) *nstages = 1;
     return hipGetLastError() == hipSuccess ? 0 : -1;

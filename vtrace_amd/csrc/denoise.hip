@@ -29,9 +29,9 @@
 //                    through LDS in 32-wide K slices).  Both can pool their output (2x2
 //                    mean) in the epilogue and read the decoder's upsampled channels from
 //                    the lower level in their staging.
-//   k_conv3x3_wgrad  dW[co][tap][ci] = sum_p dY[p][co] X[p+tap][ci] over a chunk of pixels:
-//                    32-pixel tiles of dY and the shifted X are staged transposed in LDS so
-//                    both MFMA operands read 8 consecutive pixels; dbias in the same pass.
+//   k_conv3x3_wgrad  dW[co][tap][ci] = sum_p dY[p][co] X[p+tap][ci] over a chunk of pixel tiles,
+//                    all nine taps of a block of input channels in registers, the operands
+//                    transposed on the way out of LDS; dbias in the same pass.
 //   pooling, upsampling, feature, loss, Adam and weight-layout kernels are element-wise.
 #include <hip/hip_runtime.h>
 
@@ -51,9 +51,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kInCh = 16;       // input feature channels (10 used)
 constexpr int kOutCh = 3;
 constexpr int kLayers = 19;
-constexpr int kMaxWidth = 96;   // widest layer (LDS tile of the weight-gradient kernel)
+constexpr int kMaxWidth = 96;   // widest layer (accumulators of the weight-gradient kernel)
 constexpr uint32_t kConvPix = 128;
-constexpr uint32_t kPitch = 40;  // LDS row pitch (elements) of 32-pixel transposed tiles
 constexpr float kAlbedoEps = 0.01f;  // demodulation: irradiance = radiance / (albedo + eps)
 constexpr float kLogMax = 16.0f;     // clamp of the predicted log irradiance
 
@@ -650,99 +649,165 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3_res(ConvArgs a, uint32_t nt
 struct WGradArgs {
     const uint16_t* in;   // forward input, N x H x W x in_stride, channels [0, Cin)
     const uint16_t* g;    // gradient of the pre-activation output, N x H x W x g_stride (g_stride % 8 == 0)
-    float* part;          // [chunks][Cout][9 * Cin]
-    float* bpart;         // [chunks][Cout]
+    float* part;          // [chunks][Cout * 9 * Cin weights, then Cout biases]
     uint32_t in_stride, g_stride;
-    uint32_t N, H, W, Cin, Cout, chunk_px;
+    uint32_t N, H, W, Cin, Cout;
+    uint32_t ntx, nty, tiles;   // kWgX x kWgY pixel tiles: per row, per column, of the batch
+    uint32_t tiles_chunk;       // consecutive tiles of one workgroup
 };
 
-// grid (chunks, 9 taps, ceil(Cin / 32)); 256 threads.
-__global__ __launch_bounds__(256) void k_conv3x3_wgrad(WGradArgs a) {
-    __shared__ __align__(16) uint16_t gT[kMaxWidth][kPitch];
-    __shared__ __align__(16) uint16_t xT[32][kPitch];
-    const uint32_t chunk = blockIdx.x, tap = blockIdx.y, cib = blockIdx.z;
-    const int dy = (int)(tap / 3u) - 1, dx = (int)(tap % 3u) - 1;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t g = lane >> 4, r = lane & 15u;
-    const uint32_t HW = a.H * a.W, P = a.N * HW;
-    const uint32_t p_begin = chunk * a.chunk_px;
-    const uint32_t p_end = min(P, p_begin + a.chunk_px);
-    const uint32_t nco16 = (a.Cout + 15u) / 16u;
-    const uint32_t c_valid = min(32u, a.Cin - cib * 32u);
-    const uint32_t nci16 = (c_valid + 15u) / 16u;
-    const uint32_t ntiles = nco16 * nci16;  // <= 12 (Cout <= 96): <= 3 per wave
-    const uint32_t cout8 = (a.Cout + 7u) / 8u;
-    const bool do_bias = tap == 4u && cib == 0u;
-    f32x4 acc[3];
-#pragma unroll
-    for (int s = 0; s < 3; ++s) acc[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float bsum = 0.0f;
-    for (uint32_t p0 = p_begin; p0 < p_end; p0 += 32u) {
-        for (uint32_t idx = tid; idx < 32u * cout8; idx += 256u) {
-            const uint32_t j = idx / cout8, c8 = idx - j * cout8;
-            const uint32_t p = p0 + j;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if (p < p_end) v = *reinterpret_cast<const u32x4*>(a.g + (size_t)p * a.g_stride + c8 * 8u);
-#pragma unroll
-            for (int t = 0; t < 8; ++t) gT[c8 * 8u + (uint32_t)t][j] = (uint16_t)half16(v, t);
-        }
-        if (tid < 128u) {
-            const uint32_t j = tid >> 2, o = tid & 3u;
-            const uint32_t c = cib * 32u + o * 8u, p = p0 + j;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if (p < p_end && c < a.Cin) {
-                const uint32_t n = p / HW, rem = p - n * HW;
-                const int yy = (int)(rem / a.W) + dy, xx = (int)(rem % a.W) + dx;
-                if (yy >= 0 && yy < (int)a.H && xx >= 0 && xx < (int)a.W)
-                    v = *reinterpret_cast<const u32x4*>(a.in + (size_t)(n * HW + (uint32_t)yy * a.W + (uint32_t)xx) *
-                                                                   a.in_stride + c);
-            }
-#pragma unroll
-            for (int t = 0; t < 8; ++t) xT[o * 8u + (uint32_t)t][j] = (uint16_t)half16(v, t);
-        }
-        __syncthreads();
-        if (do_bias && tid < a.Cout)
-            for (int j = 0; j < 32; ++j) bsum += bf2f(gT[tid][j]);
-        uint32_t s = 0;
-        for (uint32_t ti = wave; ti < ntiles; ti += 4u, ++s) {
-            const uint32_t co16 = ti / nci16, c16 = ti - co16 * nci16;
-            const bf16x8 A = ld8(&gT[co16 * 16u + r][8u * g]);
-            const bf16x8 B = ld8(&xT[c16 * 16u + r][8u * g]);
-            if (s == 0) acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[0], 0, 0, 0);
-            else if (s == 1) acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[1], 0, 0, 0);
-            else acc[2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[2], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    const uint32_t K = 9u * a.Cin;
-    uint32_t s = 0;
-    for (uint32_t ti = wave; ti < ntiles; ti += 4u, ++s) {
-        const uint32_t co16 = ti / nci16, c16 = ti - co16 * nci16;
-        const uint32_t c = cib * 32u + c16 * 16u + r;
-        const f32x4 v = s == 0 ? acc[0] : (s == 1 ? acc[1] : acc[2]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t co = co16 * 16u + 4u * g + (uint32_t)i;
-            if (co < a.Cout && c < a.Cin) a.part[((size_t)chunk * a.Cout + co) * K + tap * a.Cin + c] = v[i];
-        }
-    }
-    if (do_bias && tid < a.Cout) a.bpart[(size_t)chunk * a.Cout + tid] = bsum;
+// dW[co][tap][ci] = sum_p dY[p][co] X[p + tap][ci] as a GEMM over pixels: rows co, columns ci, one
+// accumulator tile per tap.  A workgroup takes a chunk of kWgX x kWgY pixel tiles and 16 NCI of the
+// input channels and holds all nine taps' sums of all 16 NCO output channels in registers: wave w
+// the taps of row dy = w - 1 (three shifts in x share every dY fragment).  A tile of dY and of X with
+// a one-pixel halo is staged in LDS as it lies in memory (pixel by pixel); ds_read_b64_tr_b16
+// transposes on the way to the registers (16 lanes read 4 pixels x 16 channels, lane i gets channel i
+// of the 4 pixels), so a tap is an offset of whole LDS pixels and both tensors are read from memory
+// once for all taps.  The next tile is fetched into registers while the current one is multiplied.
+// A K step is 2 rows of 16 pixels: k = 8 g + 4 h + j is the pixel 4 (g & 1) + 8 h + j of row g >> 1,
+// the same for both operands.  LDS pixels lie an odd multiple of 32 B apart, so the 8 pixels that
+// half a wave reads are in different banks.
+// Bound by the matrix pipe and the staging together.  The form before (one tap and 32 input channels
+// per workgroup, the transpose by 2-byte LDS stores, dY read 9 Cin / 32 times) took 4.9 ms of a
+// 14.1 ms fine-tuning call (8 steps of 8 crops of 128 x 128); this one 1.2 ms.
+constexpr uint32_t kWgX = 16, kWgY = 4, kWgThreads = 192;
+constexpr uint32_t wg_pitch(uint32_t n16) { return 16u * (n16 | 1u); }
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// 16 channels x 8 pixels of an MFMA operand: pixels at p and p + 8 (LDS pixels of `pitch` elements)
+__device__ __forceinline__ bf16x8 ld_tr(const uint16_t* p, uint32_t pitch) {
+    typedef __attribute__((address_space(3))) s16x4 LdsS16x4;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4*)(p));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4*)(p + 8u * pitch));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// sum of the chunk partials in chunk order (deterministic): W part then bias part
-__global__ void k_wgrad_reduce(const float* __restrict__ part, const float* __restrict__ bpart, uint32_t chunks,
-                               uint32_t nw, uint32_t nb, float* __restrict__ gw, float* __restrict__ gb) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nw) {
-        float s = 0.0f;
-        for (uint32_t c = 0; c < chunks; ++c) s += part[(size_t)c * nw + i];
-        gw[i] = s;
-    } else if (i < nw + nb) {
-        const uint32_t j = i - nw;
-        float s = 0.0f;
-        for (uint32_t c = 0; c < chunks; ++c) s += bpart[(size_t)c * nb + j];
-        gb[j] = s;
+// grid (chunks, ceil(Cin / (16 NCI)))
+template <int NCO, int NCI>
+__global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_conv3x3_wgrad(WGradArgs a) {
+    constexpr uint32_t GP = wg_pitch(NCO), XP = wg_pitch(NCI), XW = kWgX + 2u, XH = kWgY + 2u;
+    constexpr uint32_t GCH = kWgX * kWgY * 2u * NCO, XCH = XW * XH * 2u * NCI;   // 16-byte chunks of a tile
+    constexpr uint32_t GB = (GCH + kWgThreads - 1u) / kWgThreads, XB = (XCH + kWgThreads - 1u) / kWgThreads;
+    __shared__ __align__(16) uint16_t gt[kWgX * kWgY * GP];
+    __shared__ __align__(16) uint16_t xt[XW * XH * XP];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // tap row: dy = wave - 1
+    const uint32_t ci0 = blockIdx.y * 16u * NCI;
+    const uint32_t cout8 = (a.Cout + 7u) & ~7u;
+    const uint32_t t1 = min(a.tiles, (blockIdx.x + 1u) * a.tiles_chunk);
+    u32x4 gpre[GB], xpre[XB];
+    auto fetch = [&](uint32_t t) {
+        const uint32_t tx = t % a.ntx, rest = t / a.ntx, ty = rest % a.nty, n = rest / a.nty;
+        const int x0 = (int)(tx * kWgX), y0 = (int)(ty * kWgY);
+        const size_t img = (size_t)n * a.H * a.W;
+#pragma unroll
+        for (uint32_t b = 0; b < GB; ++b) {
+            const uint32_t i = tid + kWgThreads * b, pix = i / (2u * NCO), c = 8u * (i % (2u * NCO));
+            const uint32_t x = (uint32_t)x0 + pix % kWgX, y = (uint32_t)y0 + pix / kWgX;
+            gpre[b] = u32x4{0u, 0u, 0u, 0u};
+            if (i < GCH && c < cout8 && x < a.W && y < a.H)
+                gpre[b] = *reinterpret_cast<const u32x4*>(a.g + (img + (size_t)y * a.W + x) * a.g_stride + c);
+        }
+#pragma unroll
+        for (uint32_t b = 0; b < XB; ++b) {
+            const uint32_t i = tid + kWgThreads * b, pix = i / (2u * NCI), c = ci0 + 8u * (i % (2u * NCI));
+            const int x = x0 + (int)(pix % XW) - 1, y = y0 + (int)(pix / XW) - 1;
+            xpre[b] = u32x4{0u, 0u, 0u, 0u};
+            if (i < XCH && c < a.Cin && x >= 0 && x < (int)a.W && y >= 0 && y < (int)a.H)
+                xpre[b] = *reinterpret_cast<const u32x4*>(a.in + (img + (size_t)y * a.W + (uint32_t)x) * a.in_stride + c);
+        }
+    };
+    // this lane's pixel and channels of a transposed read
+    const uint32_t g = lane >> 4, r = lane & 15u;
+    const uint32_t col = 4u * (g & 1u) + (r >> 2), row = g >> 1;
+    const uint16_t* const gbase = gt + (row * kWgX + col) * GP + 4u * (r & 3u);
+    const uint16_t* const xbase = xt + ((row + wave) * XW + col) * XP + 4u * (r & 3u);
+    const bool do_bias = wave == 1u && blockIdx.y == 0u;
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+    f32x4 acc[3][NCI][NCO], bacc[NCO];
+#pragma unroll
+    for (int j = 0; j < NCO; ++j) {
+        bacc[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < 3 * NCI; ++k) acc[k / NCI][k % NCI][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
+    uint32_t t = blockIdx.x * a.tiles_chunk;
+    if (t < t1) fetch(t);
+    for (; t < t1; ++t) {
+        __syncthreads();   // the previous tile is no longer read
+#pragma unroll
+        for (uint32_t b = 0; b < GB; ++b) {
+            const uint32_t i = tid + kWgThreads * b;
+            if (i < GCH) *reinterpret_cast<u32x4*>(gt + i / (2u * NCO) * GP + 8u * (i % (2u * NCO))) = gpre[b];
+        }
+#pragma unroll
+        for (uint32_t b = 0; b < XB; ++b) {
+            const uint32_t i = tid + kWgThreads * b;
+            if (i < XCH) *reinterpret_cast<u32x4*>(xt + i / (2u * NCI) * XP + 8u * (i % (2u * NCI))) = xpre[b];
+        }
+        __syncthreads();
+        if (t + 1u < t1) fetch(t + 1u);
+#pragma unroll
+        for (uint32_t ks = 0; ks < kWgY / 2u; ++ks) {
+            bf16x8 A[NCO];
+#pragma unroll
+            for (int j = 0; j < NCO; ++j) A[j] = ld_tr(gbase + 2u * ks * kWgX * GP + 16u * j, GP);
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                for (int c = 0; c < NCI; ++c) {
+                    const bf16x8 B = ld_tr(xbase + (2u * ks * XW + dx) * XP + 16u * c, XP);
+#pragma unroll
+                    for (int j = 0; j < NCO; ++j)
+                        acc[dx][c][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[j], B, acc[dx][c][j], 0, 0, 0);
+                }
+            if (do_bias)
+#pragma unroll
+                for (int j = 0; j < NCO; ++j)
+                    bacc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[j], ones, bacc[j], 0, 0, 0);
+        }
+    }
+    // D layout: lane holds output channels 16 j + 4 g + i (rows) at input channel r (column)
+    const uint32_t K = 9u * a.Cin;
+    float* const part = a.part + (size_t)blockIdx.x * (a.Cout * K + a.Cout);
+#pragma unroll
+    for (int j = 0; j < NCO; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t co = 16u * j + 4u * g + (uint32_t)i;
+            if (co >= a.Cout) continue;
+#pragma unroll
+            for (int c = 0; c < NCI; ++c) {
+                const uint32_t ci = ci0 + 16u * c + r;
+                if (ci >= a.Cin) continue;
+#pragma unroll
+                for (uint32_t dx = 0; dx < 3; ++dx) part[(size_t)co * K + (3u * wave + dx) * a.Cin + ci] = acc[dx][c][j][i];
+            }
+            if (do_bias && r == 0u) part[a.Cout * K + co] = bacc[j][i];
+        }
+}
+
+// The chunks' partial sums of every layer, added up in chunk order (deterministic): parameter i of
+// layer l is part[off + c * n + i - first] over its chunks c.  One launch for the whole network at
+// the end of the backward pass: a layer alone is too few threads to fill the GPU.
+struct PartTable {
+    struct {
+        uint64_t off;
+        uint32_t chunks, n, first;   // n: the layer's weights and biases, from parameter `first`
+    } l[kLayers];
+};
+__global__ __launch_bounds__(256) void k_wgrad_reduce(const float* __restrict__ part, PartTable T, uint32_t nparam,
+                                                      float* __restrict__ grads) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= nparam) return;
+    uint32_t l = 0;
+    while (l + 1u < (uint32_t)kLayers && i >= T.l[l + 1].first) ++l;
+    const uint32_t n = T.l[l].n, chunks = T.l[l].chunks;
+    const float* p = part + T.l[l].off + (i - T.l[l].first);
+    float s = 0.0f;
+#pragma unroll 8
+    for (uint32_t c = 0; c < chunks; ++c) s += p[(size_t)c * n];
+    grads[i] = s;
 }
 
 // ---- element-wise kernels (8 channels per thread) ----------------------------------------
@@ -1051,6 +1116,7 @@ struct Net {
     float* lpart = nullptr;
     float* part = nullptr;
     size_t part_cap = 0;
+    PartTable parts{};         // where each layer's partial sums lie (ensure_part)
     float* losses = nullptr;   // device, one per training iteration
     size_t losses_cap = 0;
     // training frames
@@ -1356,37 +1422,81 @@ int conv_bwd_data(int li, const Tensor& g, const Tensor& dx, const Tensor* mask,
     return mask ? launch_conv_nt<false, false, true>(nt, a, s) : launch_conv_nt<false, false, false>(nt, a, s);
 }
 
+template <int NCO>
+void launch_wgrad(uint32_t nci, const WGradArgs& a, dim3 grid, hipStream_t s) {
+    if (nci == 1) hipLaunchKernelGGL((k_conv3x3_wgrad<NCO, 1>), grid, dim3(kWgThreads), 0, s, a);
+    else hipLaunchKernelGGL((k_conv3x3_wgrad<NCO, 2>), grid, dim3(kWgThreads), 0, s, a);
+}
+
+// How a layer's weight gradient is split: about two workgroups per CU (fewer leave CUs idle, more
+// write and read more partial sums).
+struct WGradPlan {
+    uint32_t nco, nci, cib, ntx, nty, tiles, tiles_chunk, chunks;
+};
+WGradPlan wgrad_plan(const Layer& L, uint32_t N, uint32_t H, uint32_t W) {
+    WGradPlan p;
+    p.nco = (L.cout + 15u) / 16u;
+    p.nci = L.cin <= 16u ? 1u : 2u;
+    p.cib = (L.cin + 16u * p.nci - 1u) / (16u * p.nci);
+    p.ntx = (W + kWgX - 1u) / kWgX;
+    p.nty = (H + kWgY - 1u) / kWgY;
+    p.tiles = N * p.ntx * p.nty;
+    const uint32_t want = std::max(1u, 2u * device_cus() / p.cib);
+    p.tiles_chunk = (p.tiles + want - 1u) / want;
+    p.chunks = (p.tiles + p.tiles_chunk - 1u) / p.tiles_chunk;
+    return p;
+}
+// level of a layer's pixels: 0 at full size, each next one half the width and height
+uint32_t layer_level(int li) { return li < 10 ? (uint32_t)li / 2u : li < 18 ? 3u - (uint32_t)(li - 10) / 2u : 0u; }
+
+// plans and partial sums of every layer for a batch of N x H x W
+int ensure_part(uint32_t N, uint32_t H, uint32_t W) {
+    uint64_t off = 0;
+    for (int i = 0; i < kLayers; ++i) {
+        const Layer& L = net.L[i];
+        const uint32_t lvl = layer_level(i);
+        const WGradPlan p = wgrad_plan(L, N, H >> lvl, W >> lvl);
+        net.parts.l[i].off = off;
+        net.parts.l[i].chunks = p.chunks;
+        net.parts.l[i].n = L.d.nw + L.cout;
+        net.parts.l[i].first = L.d.w_off;
+        off += (uint64_t)p.chunks * (L.d.nw + L.cout);
+    }
+    if (off <= net.part_cap && net.part) return 0;
+    hipFree(net.part);
+    net.part = nullptr;
+    net.part_cap = 0;
+    if (hipMalloc(&net.part, off * 4) != hipSuccess) {
+        net.part = nullptr;
+        return -1;
+    }
+    net.part_cap = off;
+    return 0;
+}
+
 int conv_wgrad(int li, const Tensor& x, const Tensor& g, uint32_t N, uint32_t H, uint32_t W, hipStream_t s) {
     const Layer& L = net.L[li];
-    const size_t P = (size_t)N * H * W;
-    uint32_t chunk_px = 1024;
-    while (chunk_px > 32 && ((P + chunk_px - 1) / chunk_px) * 9u * ((L.cin + 31u) / 32u) < 1024u) chunk_px >>= 1;
-    const uint32_t chunks = (uint32_t)((P + chunk_px - 1) / chunk_px);
-    const size_t nw = (size_t)L.cout * 9u * L.cin;
-    const size_t need = (size_t)chunks * (nw + L.cout);
-    if (need > net.part_cap) {
-        hipFree(net.part);
-        if (hipMalloc(&net.part, need * 4) != hipSuccess) {
-            net.part = nullptr;
-            net.part_cap = 0;
-            return -1;
-        }
-        net.part_cap = need;
-    }
+    const WGradPlan p = wgrad_plan(L, N, H, W);
     WGradArgs a{};
     a.in = x.p;
     a.in_stride = x.C;
     a.g = g.p;
     a.g_stride = g.C;
-    a.part = net.part;
-    a.bpart = net.part + (size_t)chunks * nw;
+    a.part = net.part + net.parts.l[li].off;
     a.N = N; a.H = H; a.W = W;
     a.Cin = L.cin;
     a.Cout = L.cout;
-    a.chunk_px = chunk_px;
-    hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(chunks, 9, (L.cin + 31u) / 32u), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(blocks(nw + L.cout)), dim3(256), 0, s, net.part, a.bpart, chunks,
-                       (uint32_t)nw, L.cout, net.grads + L.d.w_off, net.grads + L.d.b_off);
+    a.ntx = p.ntx; a.nty = p.nty; a.tiles = p.tiles; a.tiles_chunk = p.tiles_chunk;
+    const dim3 grid(p.chunks, p.cib);
+    switch (p.nco) {
+        case 1: launch_wgrad<1>(p.nci, a, grid, s); break;
+        case 2: launch_wgrad<2>(p.nci, a, grid, s); break;
+        case 3: launch_wgrad<3>(p.nci, a, grid, s); break;
+        case 4: launch_wgrad<4>(p.nci, a, grid, s); break;
+        case 5: launch_wgrad<5>(p.nci, a, grid, s); break;
+        case 6: launch_wgrad<6>(p.nci, a, grid, s); break;
+        default: return -1;
+    }
     return 0;
 }
 
@@ -1443,6 +1553,7 @@ int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, hipStream_t s)
     const size_t P0 = (size_t)N * H * W;
     const float scale = 1.0f / (float)(3 * P0);
     const uint32_t lb = blocks(P0);
+    if (ensure_part(N, H, W) != 0) return -1;
     hipLaunchKernelGGL(k_loss, dim3(lb), dim3(256), 0, s, net.y, net.target, net.x0.p, (uint32_t)P0, scale,
                        net.gy.p, net.lpart);
     hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(256), 0, s, net.lpart, lb, scale, loss_dev);
@@ -1485,6 +1596,8 @@ int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, hipStream_t s)
         rc |= conv_wgrad(2 * l, in, net.ga[l], N, h, w, s);
         if (l > 0) rc |= conv_bwd_data(2 * l, net.ga[l], net.gpool[l - 1], nullptr, N, h, w, s);
     }
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3(blocks(net.nparam)), dim3(256), 0, s, net.part, net.parts,
+                       (uint32_t)net.nparam, net.grads);
     return rc == 0 && hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

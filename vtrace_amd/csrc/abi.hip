@@ -32,6 +32,7 @@ static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 namespace {
 
 constexpr uint32_t kMaxTextures = 65536;  // lib/common.h:35
+constexpr uint32_t kFlatInstances = 16;    // trees of so few leaves fit the traversal stack in LDS
 constexpr uint32_t kMaxChunks = 4;         // chunks (streams) per frame
 constexpr uint64_t kSplitMinSamples = 1ull << 21;   // smaller frames: one stream by default
 
@@ -46,8 +47,7 @@ struct State {
     user_input input{};
     double cursor[2] = {0.0, 0.0};    // headless cursor position (vt_set_cursor)
     // instances (lib/memory.c:221-267)
-    float* inst_host = nullptr;    // pinned staging
-    float* inst_dev = nullptr;
+    float* inst_host = nullptr;    // pinned; the tree build reads it in place
     uint32_t inst_capacity = 0;
     uint32_t inst_count = 0;
     uint32_t bvh_depth = 0;
@@ -269,12 +269,9 @@ int grow_instances(uint32_t n) {
     while (cap < n + 1) cap *= 2;  // round_up_p2(n + 1), lib/memory.c:191
     if (g.inst_copied) hipEventSynchronize(g.inst_copied);
     hipHostFree(g.inst_host);
-    hipFree(g.inst_dev);
     g.inst_host = nullptr;
-    g.inst_dev = nullptr;
     hipError_t e;
-    if ((e = hipHostMalloc(&g.inst_host, (size_t)cap * 64, hipHostMallocDefault)) != hipSuccess ||
-        (e = hipMalloc(&g.inst_dev, (size_t)cap * 64)) != hipSuccess) {
+    if ((e = hipHostMalloc(&g.inst_host, (size_t)cap * 64, hipHostMallocDefault)) != hipSuccess) {
         set_err("instance buffer allocation", e);
         g.inst_capacity = 0;
         return -1;
@@ -734,7 +731,7 @@ void cleanup(void) {
     g.vols.clear();
     vt_lbvh_free(g.bvh);
     hipHostFree(g.inst_host);
-    hipFree(g.inst_dev); hipFree(g.vol_table); hipFree(g.staging); hipFree(g.remap);
+    hipFree(g.vol_table); hipFree(g.staging); hipFree(g.remap);
     hipFree(g.hits); hipFree(g.rad); hipFree(g.bgra); hipFree(g.gbuf); hipFree(g.gsamp); hipFree(g.stats); hipFree(g.srgb_dec); hipFree(g.srgb_thr);
     hipFree(g.wave_mem);
     for (uint32_t k = 0; k < kMaxChunks; ++k) {
@@ -795,25 +792,27 @@ int32_t end_update_instances(uint32_t instance_count) {
         std::memcmp(g.inst_prev.data(), g.inst_host, nrec * 4) == 0)
         return 0;
     g.inst_prev.clear();
-    hipError_t e = hipMemcpyAsync(g.inst_dev, g.inst_host, (size_t)instance_count * 64, hipMemcpyHostToDevice, g.stream);
-    if (e != hipSuccess) {
-        set_err("instance copy", e);
-        return -1;
-    }
-    hipEventRecord(g.inst_copied, g.stream);
-    if (vt_lbvh_build(g.bvh, g.inst_dev, instance_count, g.vol_table, (uint32_t)g.vols.size(), g.stream) != 0) {
+    if (vt_lbvh_build(g.bvh, g.inst_host, instance_count, g.vol_table, (uint32_t)g.vols.size(), g.stream) != 0) {
         set_err("lbvh build", hipGetLastError());
         return -1;
     }
+    hipEventRecord(g.inst_copied, g.stream);
     // the tree depth selects the traversal-stack variant (LDS stack or a deep private stack);
-    // it is read by the next frame (scene_gpu), so the update does not wait for the build
-    e = hipMemcpyAsync(g.depth_host, g.bvh.depth, 4, hipMemcpyDeviceToHost, g.stream);
-    if (e == hipSuccess) e = hipEventRecord(g.depth_ready, g.stream);
-    if (e != hipSuccess) {
-        set_err("lbvh depth", e);
-        return -1;
+    // it is read by the next frame (scene_gpu), so the update does not wait for the build.  A tree of
+    // n leaves is at most n - 1 deep: up to kFlatInstances that bound fits the LDS stack, and the
+    // frame does not wait for the build either (about 15 us between the build and the frame's launch).
+    if (instance_count <= kFlatInstances) {
+        g.bvh_depth = instance_count - 1;
+        g.depth_pending = false;
+    } else {
+        hipError_t e = hipMemcpyAsync(g.depth_host, g.bvh.depth, 4, hipMemcpyDeviceToHost, g.stream);
+        if (e == hipSuccess) e = hipEventRecord(g.depth_ready, g.stream);
+        if (e != hipSuccess) {
+            set_err("lbvh depth", e);
+            return -1;
+        }
+        g.depth_pending = true;
     }
-    g.depth_pending = true;
     g.inst_count = instance_count;
     g.inst_prev.assign(g.inst_host, g.inst_host + nrec);
     g.inst_prev_vols = g.vols.size();
@@ -829,16 +828,11 @@ int32_t vt_refit_instances(uint32_t instance_count) {
         set_err("vt_refit_instances: the instance count differs from the last build");
         return -1;
     }
-    hipError_t e = hipMemcpyAsync(g.inst_dev, g.inst_host, (size_t)instance_count * 64, hipMemcpyHostToDevice, g.stream);
-    if (e != hipSuccess) {
-        set_err("instance copy", e);
-        return -1;
-    }
-    hipEventRecord(g.inst_copied, g.stream);
-    if (vt_lbvh_refit(g.bvh, g.inst_dev, instance_count, g.vol_table, (uint32_t)g.vols.size(), g.stream) != 0) {
+    if (vt_lbvh_refit(g.bvh, g.inst_host, instance_count, g.vol_table, (uint32_t)g.vols.size(), g.stream) != 0) {
         set_err("lbvh refit", hipGetLastError());
         return -1;
     }
+    hipEventRecord(g.inst_copied, g.stream);
     g.inst_prev.assign(g.inst_host, g.inst_host + (size_t)instance_count * 16);
     g.inst_prev_vols = g.vols.size();
     return 0;

@@ -42,7 +42,7 @@ struct LbvhWork {
     uint32_t* vals[2] = {nullptr, nullptr};
     int32_t* parent = nullptr;  // 2*cap - 1
     uint32_t* counters = nullptr;  // cap
-    float* bounds = nullptr;    // 6
+    float* bounds = nullptr;    // 6 per workgroup of k_instance_prep
     uint32_t* depth = nullptr;  // tree depth (edges on the longest root-leaf path)
     uint32_t* sort_hist = nullptr;  // 256 digit counts per 1024-key chunk (multi-workgroup sort)
 };

@@ -324,7 +324,7 @@ int upload_volume(const void* data, size_t bytes, uint32_t fmt, const uint32_t d
         }
         g.staging_size = sz;
     }
-    if ((e = hipMemcpyAsync(g.staging, data, total, hipMemcpyHostToDevice, g.stream)) != hipSuccess) {
+    if ((e = vt_copy_in(g.staging, data, total, g.stream)) != hipSuccess) {
         set_err("volume copy", e);
         return -1;
     }
@@ -746,6 +746,7 @@ void cleanup(void) {
     hipStreamDestroy(g.stream);
     vt_trace_set_tables(nullptr, nullptr);
     vt_trace_release();
+    vt_copy_release();
     g = State{};
 }
 
@@ -877,7 +878,7 @@ static int32_t read_frame(const void* src, void* dst, uint64_t bytes, size_t ele
         set_err("read-back buffer too small");
         return -1;
     }
-    hipError_t e = hipMemcpyAsync(dst, src, need, hipMemcpyDeviceToHost, g.stream);
+    hipError_t e = vt_copy_out(dst, src, need, g.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
     if (e != hipSuccess) {
         set_err("read-back", e);
@@ -1065,7 +1066,7 @@ int32_t vt_read_volume(int32_t id, void* dst, uint64_t bytes) {
     d.palette = v.palette;
     d.blocks = v.blocks;
     int rc = vt_debrick(d, tmp, g.stream);
-    if (rc == 0) hipMemcpyAsync(dst, tmp, need, hipMemcpyDeviceToHost, g.stream);
+    if (rc == 0 && vt_copy_out(dst, tmp, need, g.stream) != hipSuccess) rc = -1;
     if (hipStreamSynchronize(g.stream) != hipSuccess) rc = -1;
     hipFree(tmp);
     return rc;

@@ -1755,12 +1755,12 @@ int32_t vt_dn_set_params(const float* params, uint64_t n) {
     if (!net.on || !params || n != net.nparam) return -1;
     hipSetDevice(vt_rt_device());
     hipStream_t s = vt_rt_stream();
-    hipMemcpyAsync(net.params, params, n * 4, hipMemcpyHostToDevice, s);
+    const hipError_t e = vt_copy_in(net.params, params, n * 4, s);
     hipMemsetAsync(net.adam_m, 0, n * 4, s);
     hipMemsetAsync(net.adam_v, 0, n * 4, s);
     net.adam_t = 0;
     net.weights_dirty = true;
-    return hipStreamSynchronize(s) == hipSuccess ? 0 : -1;
+    return hipStreamSynchronize(s) == hipSuccess && e == hipSuccess ? 0 : -1;
 }
 
 int32_t vt_dn_get_params(float* params, uint64_t n) {
@@ -1768,8 +1768,8 @@ int32_t vt_dn_get_params(float* params, uint64_t n) {
     if (!net.on || !params || n != net.nparam) return -1;
     hipSetDevice(vt_rt_device());
     hipStream_t s = vt_rt_stream();
-    hipMemcpyAsync(params, net.params, n * 4, hipMemcpyDeviceToHost, s);
-    return hipStreamSynchronize(s) == hipSuccess ? 0 : -1;
+    const hipError_t e = vt_copy_out(params, net.params, n * 4, s);
+    return hipStreamSynchronize(s) == hipSuccess && e == hipSuccess ? 0 : -1;
 }
 
 int32_t vt_dn_grad(const float* x, const float* target, uint32_t n, uint32_t h, uint32_t w, float* y, float* grad,
@@ -1846,14 +1846,14 @@ int32_t vt_dn_add_frame(const float* rad_rgba, const float* gbuf8, const float* 
     fd.target = reinterpret_cast<const float*>(static_cast<char*>(mem) + fbytes);
     fd.h = h;
     fd.w = w;
-    hipMemcpyAsync(rad, rad_rgba, npx * 16, hipMemcpyHostToDevice, s);
-    hipMemcpyAsync(gb, gbuf8, npx * 32, hipMemcpyHostToDevice, s);
+    hipError_t e = vt_copy_in(rad, rad_rgba, npx * 16, s);
+    if (e == hipSuccess) e = vt_copy_in(gb, gbuf8, npx * 32, s);
     hipLaunchKernelGGL(k_features, dim3(blocks(npx)), dim3(256), 0, s, rad, gb, h, w, h, w, spp_feature(spp),
                        static_cast<uint16_t*>(mem));
-    hipMemcpyAsync(rad, target_rgba, npx * 16, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = vt_copy_in(rad, target_rgba, npx * 16, s);
     hipLaunchKernelGGL(k_rgba_to_rgb, dim3(blocks(npx)), dim3(256), 0, s, rad, const_cast<float*>(fd.target),
                        (uint32_t)npx);
-    if (hipStreamSynchronize(s) != hipSuccess) {
+    if (hipStreamSynchronize(s) != hipSuccess || e != hipSuccess) {
         hipFree(mem);
         return -1;
     }
@@ -1957,14 +1957,13 @@ int32_t vt_dn_denoise(const float* rad_rgba, const float* gbuf8, uint32_t h, uin
     float4* rad = reinterpret_cast<float4*>(io);
     float4* gb = reinterpret_cast<float4*>(io + npx * 16);
     float4* out = reinterpret_cast<float4*>(io + npx * 48);
-    hipMemcpyAsync(rad, rad_rgba, npx * 16, hipMemcpyHostToDevice, s);
-    hipMemcpyAsync(gb, gbuf8, npx * 32, hipMemcpyHostToDevice, s);
-    if (denoise_device(rad, gb, h, w, spp, out, gpu_ms, s) != 0) {
+    if (vt_copy_in(rad, rad_rgba, npx * 16, s) != hipSuccess || vt_copy_in(gb, gbuf8, npx * 32, s) != hipSuccess ||
+        denoise_device(rad, gb, h, w, spp, out, gpu_ms, s) != 0) {
         vt_rt_set_error("vt_dn_denoise: failed");
         return -1;
     }
-    hipMemcpyAsync(out_rgba, out, npx * 16, hipMemcpyDeviceToHost, s);
-    return hipStreamSynchronize(s) == hipSuccess ? 0 : -1;
+    const hipError_t e = vt_copy_out(out_rgba, out, npx * 16, s);
+    return hipStreamSynchronize(s) == hipSuccess && e == hipSuccess ? 0 : -1;
 }
 
 int32_t vt_dn_denoise_frame(float* out_rgba, float* gpu_ms) {
@@ -1984,8 +1983,8 @@ int32_t vt_dn_denoise_frame(float* out_rgba, float* gpu_ms) {
         vt_rt_set_error("vt_dn_denoise_frame: failed");
         return -1;
     }
-    hipMemcpyAsync(out_rgba, out, npx * 16, hipMemcpyDeviceToHost, s);
-    return hipStreamSynchronize(s) == hipSuccess ? 0 : -1;
+    const hipError_t e = vt_copy_out(out_rgba, out, npx * 16, s);
+    return hipStreamSynchronize(s) == hipSuccess && e == hipSuccess ? 0 : -1;
 }
 
 int32_t vt_dn_set_blend(const float* alpha, uint32_t n) {

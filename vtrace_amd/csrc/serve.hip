@@ -530,9 +530,10 @@ int32_t vt_serve_read(int64_t id, float* rgba, uint64_t bytes, void* hits, uint6
     // the request's last iteration has completed (its event was waited for), so the copy may
     // run beside the iteration now in flight
     const char* base = sv.arena_mem + r.off;
-    if (rgba) hipMemcpyAsync(rgba, base + npx * 32, npx * 16, hipMemcpyDeviceToHost, sv.copy);
-    if (hits) hipMemcpyAsync(hits, base, npx * 16, hipMemcpyDeviceToHost, sv.copy);
-    if (hipStreamSynchronize(sv.copy) != hipSuccess) return -1;
+    hipError_t e = hipSuccess;
+    if (rgba) e = vt_copy_out(rgba, base + npx * 32, npx * 16, sv.copy);
+    if (hits && e == hipSuccess) e = vt_copy_out(hits, base, npx * 16, sv.copy);
+    if (hipStreamSynchronize(sv.copy) != hipSuccess || e != hipSuccess) return -1;
     sv.arena.release(r.off, r.bytes);
     sv.reqs.erase(it);
     return 0;

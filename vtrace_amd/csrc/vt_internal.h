@@ -33,6 +33,11 @@ int vt_brick_volume(const uint8_t* dense_dev, uint32_t fmt, const uint32_t* pale
 int vt_debrick(const VolumeDesc& v, uint8_t* dense_dev, hipStream_t s);
 
 // lbvh.hip: builds InstanceGPU records and the LBVH from n ABI records on the device.
+// Copies to and from the caller's host memory (hostcopy.hip).
+hipError_t vt_copy_in(void* dev, const void* host, size_t bytes, hipStream_t s);
+hipError_t vt_copy_out(void* host, const void* dev, size_t bytes, hipStream_t s);
+void vt_copy_release();
+
 struct LbvhWork {
     uint32_t cap = 0;           // instances the buffers hold
     InstanceGPU* inst = nullptr;

@@ -66,9 +66,7 @@ struct State {
     VolumeDesc* vol_table = nullptr;  // kMaxTextures descriptors
     uint8_t* staging = nullptr;
     size_t staging_size = 0;
-    uint32_t* palette_rgba_identity = nullptr;
-    uint16_t* remap = nullptr;        // 3 tables
-    size_t remap_cap = 0;
+    BrickWork brick;
     // frame
     vt_render_params params{};
     HitRecord* hits = nullptr;
@@ -281,18 +279,6 @@ int grow_instances(uint32_t n) {
     return 0;
 }
 
-// Nearest-texel remap per axis: the texel NEAREST + CLAMP_TO_EDGE sampling of voxel/size
-// selects (shaders/trace.frag:77, lib/descriptor.c:100-105), FP32.
-uint16_t nearest_texel(int v, uint32_t dim) {
-    float size = (float)dim;
-    float u = (float)v / size;
-    float x = u * size;
-    int t = (int)std::floor(x);
-    if (t < 0) t = 0;
-    if (t > (int)dim - 1) t = (int)dim - 1;
-    return (uint16_t)t;
-}
-
 // count volumes of one size, packed one after another (bytes each), bricked in one pass;
 // ids are consecutive from the returned first id.
 int upload_volume(const void* data, size_t bytes, uint32_t fmt, const uint32_t dim[3], const uint32_t* palette,
@@ -328,54 +314,10 @@ int upload_volume(const void* data, size_t bytes, uint32_t fmt, const uint32_t d
         set_err("volume copy", e);
         return -1;
     }
-    size_t rc = (size_t)dim[0] + dim[1] + dim[2];
-    if (rc > g.remap_cap) {
-        hipFree(g.remap);
-        if ((e = hipMalloc(&g.remap, rc * 2)) != hipSuccess) {
-            set_err("remap allocation", e);
-            g.remap_cap = 0;
-            return -1;
-        }
-        g.remap_cap = rc;
-    }
-    std::vector<uint16_t> rm(rc);
-    size_t off = 0;
-    for (int a = 0; a < 3; ++a)
-        for (uint32_t i = 0; i < dim[a]; ++i) rm[off++] = nearest_texel((int)i, dim[a]);
-    hipMemcpyAsync(g.remap, rm.data(), rc * 2, hipMemcpyHostToDevice, g.stream);
-    VolumeStore vs;
-    if (fmt == 0) {
-        if ((e = hipMalloc(&vs.palette, 1024)) != hipSuccess) {
-            set_err("palette allocation", e);
-            return -1;
-        }
-        hipMemcpyAsync(vs.palette, palette, 1024, hipMemcpyHostToDevice, g.stream);
-    }
-    const uint16_t* remaps[3] = {g.remap, g.remap + dim[0], g.remap + dim[0] + dim[1]};
-    std::vector<VolumeStore> out(count);
-    if (vt_brick_volume(g.staging, fmt, vs.palette, remaps, dim, count, out.data(), g.stream) != 0) {
-        hipFree(vs.palette);
-        set_err("bricking failed");
-        return -1;
-    }
-    std::vector<VolumeDesc> descs(count);
-    for (uint32_t k = 0; k < count; ++k) {
-        const VolumeStore& v = out[k];
-        VolumeDesc& d = descs[k];
-        d = VolumeDesc{};
-        for (int a = 0; a < 3; ++a) { d.dim[a] = v.dim[a]; d.bdim[a] = v.bdim[a]; }
-        d.fmt = v.fmt;
-        d.nbricks = v.nbricks;
-        d.brick_map = v.brick_map;
-        d.masks = v.masks;
-        d.payload = v.payload;
-        d.palette = v.palette;
-        d.blocks = v.blocks;
-    }
     const int32_t id = (int32_t)g.vols.size();
-    hipMemcpyAsync(&g.vol_table[id], descs.data(), sizeof(VolumeDesc) * count, hipMemcpyHostToDevice, g.stream);
-    if ((e = hipStreamSynchronize(g.stream)) != hipSuccess) {
-        set_err("upload", e);
+    std::vector<VolumeStore> out(count);
+    if (vt_brick_volume(g.brick, g.staging, fmt, palette, dim, count, out.data(), &g.vol_table[id], g.stream) != 0) {
+        set_err("bricking failed");
         return -1;
     }
     g.vols.insert(g.vols.end(), out.begin(), out.end());
@@ -726,12 +668,13 @@ void cleanup(void) {
     vt_dn_release();
     for (auto& v : g.vols) {
         if (!v.owner) continue;  // shares the pools of the first volume of its batch
-        hipFree(v.brick_map); hipFree(v.masks); hipFree(v.payload); hipFree(v.palette); hipFree(v.blocks);
+        hipFree(v.pool);
     }
     g.vols.clear();
+    vt_brick_free(g.brick);
     vt_lbvh_free(g.bvh);
     hipHostFree(g.inst_host);
-    hipFree(g.vol_table); hipFree(g.staging); hipFree(g.remap);
+    hipFree(g.vol_table); hipFree(g.staging);
     hipFree(g.hits); hipFree(g.rad); hipFree(g.bgra); hipFree(g.gbuf); hipFree(g.gsamp); hipFree(g.stats); hipFree(g.srgb_dec); hipFree(g.srgb_thr);
     hipFree(g.wave_mem);
     for (uint32_t k = 0; k < kMaxChunks; ++k) {

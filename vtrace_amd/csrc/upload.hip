@@ -12,58 +12,93 @@
 // the pools, so every volume is laid out exactly as if it had been uploaded alone.
 //
 // Kernels:
-//   k_brick_classify  one 512-thread block per brick: occupancy bit per voxel
-//                     (alpha > 0, trace.frag:78), one ballot per z-slice -> 8 x u64 mask,
-//                     and the 2^3-block mask (one bit per 2x2x2 block holding a voxel);
-//   k_scan_*          exclusive scan of the non-empty flags -> brick ids in brick order;
-//   k_radius_*        empty-space radius of every empty brick: breadth-first layers of
-//                     26-neighbour dilation from the non-empty bricks (in place, layer k marks
-//                     the still-unreached bricks next to layer k-1);
-//   k_cube_*          per empty brick and octant, the side of the largest empty cube with the
-//                     brick as its corner: layer k grows the side from k to k + 1 where the
-//                     7 neighbours towards the octant all have sides >= k (in place: sides only
-//                     grow, so a neighbour updated during the layer decides the same way);
-//   k_brick_scatter   brick map (id, or VT_EMPTY_BRICK with radius and cube sides), masks,
-//                     block masks and payload of non-empty bricks into the pools.
+//   k_brick_classify  a workgroup per row of 8 bricks (64 x 8 x 8 voxels), lanes along x: one ballot per
+//                     row of voxels gives 8 bricks' bits (alpha > 0, trace.frag:78) -> 8 x u64 mask per
+//                     brick and the 2^3-block mask (one bit per 2x2x2 block holding a voxel; zero
+//                     for an empty brick);
+//   k_scan_*          exclusive scan of the non-empty bricks -> brick ids in brick order;
+//   k_dist_x, _y, _z  per empty brick the distance (largest of the axes') to the nearest non-empty brick
+//                     of the volume, over all directions (its empty-space radius + 1) and over each
+//                     octant alone (the side of the largest empty cube with the brick as its
+//                     corner), one axis after another -> its brick map entry;
+//   k_brick_scatter   brick map (id, or that entry), masks, block masks and payload of non-empty
+//                     bricks into the pools, through LDS so that a brick is written in whole lines;
+//                     palette and volume descriptors.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <vector>
 
 #include "vt_internal.h"
 
 namespace {
 
-__device__ inline uint32_t texel_rgba(const uint8_t* dense, uint32_t fmt, const uint32_t* palette, size_t ti,
-                                      uint32_t* raw) {
-    if (fmt == 0) {
-        uint32_t i = dense[ti];
-        *raw = i;
-        return palette[i];
-    }
-    uint32_t c = reinterpret_cast<const uint32_t*>(dense)[ti];
-    *raw = c;
-    return c;
-}
+constexpr uint32_t kRowBricks = 8;      // bricks of a workgroup: 64 voxels along x
+constexpr uint32_t kRowThreads = 256;   // wave w: z-slices 2 w and 2 w + 1
 
 struct BrickArgs {
     const uint8_t* dense;      // nvol volumes, one after another
     const uint32_t* palette;
-    const uint16_t* remap[3];
     uint32_t dim[3];
     uint32_t bdim[3];
     uint32_t fmt;
     uint32_t nbv;              // bricks per volume
+    uint32_t nb;               // bricks of the batch
+    uint32_t rows_x;           // rows of kRowBricks bricks along x
     size_t vol_texels;         // texels per volume
 };
 
-// brick b of the batch -> (texel offset of its volume, brick coordinates inside the volume)
-__device__ inline size_t brick_coords(const BrickArgs& a, uint32_t b, uint32_t* bx, uint32_t* by, uint32_t* bz) {
-    const uint32_t k = b / a.nbv, lb = b - k * a.nbv;
-    *bx = lb % a.bdim[0];
-    *by = (lb / a.bdim[0]) % a.bdim[1];
-    *bz = lb / (a.bdim[0] * a.bdim[1]);
-    return (size_t)k * a.vol_texels;
+// Nearest-texel remap of an axis: the texel NEAREST + CLAMP_TO_EDGE sampling of voxel / size selects
+// (shaders/trace.frag:77, lib/descriptor.c:100-105), FP32.
+__device__ __forceinline__ uint32_t nearest_texel(uint32_t v, uint32_t dim) {
+    const float size = (float)dim;
+    const float u = (float)v / size;
+    const float x = u * size;
+    const int t = (int)floorf(x);
+    return (uint32_t)(t < 0 ? 0 : (t > (int)dim - 1 ? (int)dim - 1 : t));
+}
+
+// The row of bricks of workgroup `row`: its first brick's number in the batch, its bricks, and this
+// lane's column of texels (wave w holds the z-slices 2 w and 2 w + 1 of the row).
+struct Row {
+    uint32_t b0, n, by, bz;
+    bool x_in;
+    size_t col;   // texel index of this lane's x at y = z = 0
+    __device__ __forceinline__ Row(const BrickArgs& a, uint32_t row) {
+        const uint32_t rx = row % a.rows_x, rest = row / a.rows_x;
+        by = rest % a.bdim[1];
+        const uint32_t kz = rest / a.bdim[1], k = kz / a.bdim[2];
+        bz = kz % a.bdim[2];
+        b0 = k * a.nbv + rx * kRowBricks + a.bdim[0] * (by + a.bdim[1] * bz);
+        n = min(kRowBricks, a.bdim[0] - rx * kRowBricks);
+        const uint32_t x = rx * kRowBricks * 8u + (threadIdx.x & 63u);
+        x_in = x < a.dim[0];
+        col = (size_t)k * a.vol_texels + nearest_texel(x_in ? x : 0u, a.dim[0]);
+    }
+};
+// f(z, y, raw) for the 16 voxels of this lane, z in {2 w, 2 w + 1} and y in 0..7 of the row: the texel as
+// stored, 0 outside the volume.  (All 16 loads are issued before the first is used.)
+template <typename F>
+__device__ __forceinline__ void for_voxels(const BrickArgs& a, const Row& R, F&& f) {
+    const uint32_t z0 = 2u * (threadIdx.x >> 6);
+    uint32_t ty[8], tz[2], raw[2][8];
+    bool in[2][8];
+#pragma unroll
+    for (uint32_t y = 0; y < 8; ++y) ty[y] = nearest_texel(min(R.by * 8 + y, a.dim[1] - 1), a.dim[1]);
+#pragma unroll
+    for (uint32_t z = 0; z < 2; ++z) tz[z] = nearest_texel(min(R.bz * 8 + z0 + z, a.dim[2] - 1), a.dim[2]);
+#pragma unroll
+    for (uint32_t z = 0; z < 2; ++z)
+#pragma unroll
+        for (uint32_t y = 0; y < 8; ++y) {
+            in[z][y] = R.x_in && R.by * 8 + y < a.dim[1] && R.bz * 8 + z0 + z < a.dim[2];
+            const size_t ti = R.col + (size_t)a.dim[0] * ((size_t)ty[y] + (size_t)a.dim[1] * tz[z]);
+            raw[z][y] = 0u;
+            if (in[z][y]) raw[z][y] = a.fmt == 0 ? (uint32_t)a.dense[ti] : reinterpret_cast<const uint32_t*>(a.dense)[ti];
+        }
+#pragma unroll
+    for (uint32_t z = 0; z < 2; ++z)
+#pragma unroll
+        for (uint32_t y = 0; y < 8; ++y) f(z, y, raw[z][y], in[z][y]);
 }
 
 // 2x2 footprints of a z-slice's occupancy (bit x + 8y) -> 16 bits, bit bx + 4by for the
@@ -77,132 +112,177 @@ __device__ inline uint32_t slice_blocks(uint64_t m) {
     return r;
 }
 
-__global__ __launch_bounds__(512) void k_brick_classify(BrickArgs a, uint64_t* masks_all, uint64_t* blocks_all,
-                                                        uint32_t* flags) {
-    const uint32_t b = blockIdx.x;
-    uint32_t bx, by, bz;
-    const size_t vbase = brick_coords(a, b, &bx, &by, &bz);
-    const uint32_t t = threadIdx.x;  // x + 8y + 64z inside the brick
-    const uint32_t gx = bx * 8 + (t & 7), gy = by * 8 + ((t >> 3) & 7), gz = bz * 8 + (t >> 6);
-    bool occ = false;
-    if (gx < a.dim[0] && gy < a.dim[1] && gz < a.dim[2]) {
-        size_t ti = vbase + (size_t)a.remap[0][gx] +
-                    (size_t)a.dim[0] * ((size_t)a.remap[1][gy] + (size_t)a.dim[1] * a.remap[2][gz]);
-        uint32_t raw;
-        occ = (texel_rgba(a.dense, a.fmt, a.palette, ti, &raw) >> 24) != 0u;
+// Bound by reading the volume once.  (One workgroup per brick with 8-byte segments of a row per load,
+// remap tables and a palette load per voxel took 70 us for 256^3 indices; this takes 20 us.)
+__global__ __launch_bounds__(kRowThreads) void k_brick_classify(BrickArgs a, uint64_t* masks_all, uint64_t* blocks_all) {
+    __shared__ uint64_t alpha[4];   // palette entries with alpha > 0
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    if (a.fmt == 0) {
+        const uint64_t bits = __ballot((a.palette[tid] >> 24) != 0u);
+        if (lane == 0) alpha[wave] = bits;
+        __syncthreads();
     }
-    uint64_t m = __ballot(occ);  // wave t>>6 holds z-slice t>>6
+    const Row R(a, blockIdx.x);
+    uint64_t m[2] = {0, 0};   // lane b < 8: brick b's slices
+    for_voxels(a, R, [&](uint32_t z, uint32_t y, uint32_t raw, bool in) {
+        const bool occ = in && (a.fmt == 0 ? ((alpha[raw >> 6] >> (raw & 63u)) & 1ull) != 0ull : (raw >> 24) != 0u);
+        const uint64_t bits = __ballot(occ);
+        m[z] |= ((bits >> (8u * (lane & 7u))) & 0xFFull) << (8u * y);
+    });
+    if (lane < R.n) {
+        const size_t b = R.b0 + lane;
+        masks_all[b * 8 + 2 * wave] = m[0];
+        masks_all[b * 8 + 2 * wave + 1] = m[1];
+        reinterpret_cast<uint16_t*>(blocks_all)[b * 4 + wave] = (uint16_t)slice_blocks(m[0] | m[1]);
+    }
+}
+
+// ---- distances ------------------------------------------------------------------------------
+// The largest-axis distance to the nearest non-empty brick q is min over q of max(|dx|, |dy|, |dz|), so
+// it can be taken one axis after another: along x the nearest in the row, then along y the minimum of
+// max(|dy|, that), then along z; the same for the bricks q of one octant alone.  A search along an
+// axis ends where its distance reaches what it has found.  Bricks outside the volume are empty.
+// (Growing the radii layer by layer took 31 launches and the cubes 7: 160 us and 38 launches for
+// 32^3 bricks; these three take 19 us.)
+constexpr uint32_t kFar = VT_BRICK_RADIUS_CAP + 1u;   // no non-empty brick nearer: radius VT_BRICK_RADIUS_CAP
+// packed: all directions in bits 0..7, octant c in bits 8 + 4 c (at most VT_BRICK_CUBE_CAP)
+__device__ __forceinline__ uint32_t oct_dist(uint32_t v, uint32_t c) { return (v >> (8u + 4u * c)) & 15u; }
+
+__global__ __launch_bounds__(256) void k_dist_x(const uint64_t* blocks_all, uint32_t nb, uint32_t bx, uint32_t* out) {
+    const uint32_t b = blockIdx.x * 256u + threadIdx.x;
+    if (b >= nb) return;
+    uint32_t f = 0, g = 0;   // the next non-empty brick up and down the row
+    if (blocks_all[b] == 0ull) {
+        const uint32_t x = b % bx;
+        f = g = kFar;
+        for (uint32_t d = 1; d < kFar; ++d) {
+            if (f == kFar && x + d < bx && blocks_all[b + d] != 0ull) f = d;
+            if (g == kFar && x >= d && blocks_all[b - d] != 0ull) g = d;
+            if (min(f, g) <= d && (max(f, g) <= d || d >= VT_BRICK_CUBE_CAP)) break;
+        }
+    }
+    out[b] = min(f, g) | (min(f, VT_BRICK_CUBE_CAP) << 8) | (min(g, VT_BRICK_CUBE_CAP) << 12);
+}
+
+// Along an axis of n bricks, `stride` apart: NC octants in, 2 NC out (octant c + NC towards lower indices).
+template <uint32_t NC>
+__device__ __forceinline__ void dist_axis(const uint32_t* in, uint32_t b, uint32_t at, uint32_t n, uint32_t stride,
+                                          uint32_t* r_out, uint32_t (&oct)[2 * NC]) {
+    const uint32_t v = in[b];
+    uint32_t r = v & 255u, far = 0;
+    for (uint32_t c = 0; c < NC; ++c) {
+        oct[c] = oct[c + NC] = oct_dist(v, c);
+        far = max(far, oct[c]);
+    }
+    far = max(far, r);
+    for (uint32_t d = 1; d < far; ++d) {
+        far = 0;
+        const uint32_t up = at + d < n ? in[b + (size_t)d * stride] : ~0u;
+        const uint32_t down = at >= d ? in[b - (size_t)d * stride] : ~0u;
+        if (up != ~0u) r = min(r, max(d, up & 255u));
+        if (down != ~0u) r = min(r, max(d, down & 255u));
+        for (uint32_t c = 0; c < NC; ++c) {
+            if (up != ~0u) oct[c] = min(oct[c], max(d, oct_dist(up, c)));
+            if (down != ~0u) oct[c + NC] = min(oct[c + NC], max(d, oct_dist(down, c)));
+            far = max(far, max(oct[c], oct[c + NC]));
+        }
+        far = max(far, r);
+    }
+    *r_out = r;
+}
+
+__global__ __launch_bounds__(256) void k_dist_y(const uint32_t* in, uint32_t nb, uint32_t bx, uint32_t by, uint32_t* out) {
+    const uint32_t b = blockIdx.x * 256u + threadIdx.x;
+    if (b >= nb) return;
+    uint32_t r, oct[4];
+    dist_axis<2>(in, b, b / bx % by, by, bx, &r, oct);
+    for (uint32_t c = 0; c < 4; ++c) r |= oct[c] << (8u + 4u * c);
+    out[b] = r;
+}
+
+// -> the brick map's entry of an empty brick (anything for a non-empty one)
+__global__ __launch_bounds__(256) void k_dist_z(const uint32_t* in, uint32_t nb, uint32_t bxy, uint32_t bz, uint32_t* entry) {
+    const uint32_t b = blockIdx.x * 256u + threadIdx.x;
+    if (b >= nb) return;
+    uint32_t r, oct[8];
+    dist_axis<4>(in, b, b / bxy % bz, bz, bxy, &r, oct);
+    uint32_t e = VT_EMPTY_BRICK | ((r - 1u) & 31u) << 24;
+    for (uint32_t o = 0; o < 8; ++o) e |= ((oct[o] - 1u) & 7u) << (3u * o);
+    entry[b] = e;
+}
+
+// ---- pools ----------------------------------------------------------------------------------
+struct PoolArgs {
+    const uint64_t *masks_all, *blocks_all;
+    const uint32_t *ids, *entry;   // ids[nb]: the total
+    uint32_t* map;
+    uint64_t *masks, *blocks;
+    uint8_t* payload;
+    uint32_t* palette;             // fmt 0
+    VolumeDesc* descs;             // of the batch's volumes
+};
+
+// A workgroup per row of bricks, as k_brick_classify; bricks meet in LDS (padded by 16 B, so that the 8
+// bricks of a row of voxels lie in different banks) and leave as 16-byte stores: 48 -> 17 us for 256^3.
+template <uint32_t BPV>
+__global__ __launch_bounds__(kRowThreads) void k_brick_scatter(BrickArgs a, PoolArgs p) {
+    constexpr uint32_t kBytes = 512u * BPV, kPitch = kBytes + 16u;
+    __shared__ __align__(16) uint8_t tile[kRowBricks * kPitch];
     __shared__ uint32_t any;
-    __shared__ uint32_t blk[2];   // 2^3-block mask: slices 2bz, 2bz+1 -> bits 16bz.. (bz = 0, 1 | 2, 3)
-    if (t == 0) { any = 0; blk[0] = 0; blk[1] = 0; }
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    if (BPV == 1 && blockIdx.x == 0) p.palette[tid] = a.palette[tid];
+    const Row R(a, blockIdx.x);
+    if (tid == 0) any = 0u;
     __syncthreads();
-    if ((t & 63) == 0) {
-        masks_all[(size_t)b * 8 + (t >> 6)] = m;
-        if (m) {
-            atomicOr(&any, 1u);
-            const uint32_t bz = (t >> 6) >> 1;
-            atomicOr(&blk[bz >> 1], slice_blocks(m) << (16u * (bz & 1u)));
+    const uint32_t first = p.ids[R.b0 / a.nbv * a.nbv];   // pool slot of the volume's first brick
+    if (tid < R.n) {
+        const uint32_t b = R.b0 + tid;
+        const bool full = p.blocks_all[b] != 0ull;
+        p.map[b] = full ? p.ids[b] - first : p.entry[b];
+        if (full) {
+            p.blocks[p.ids[b]] = p.blocks_all[b];
+            atomicOr(&any, 1u << tid);
         }
+    }
+    if (tid == 0 && R.b0 % a.nbv == 0u) {
+        const uint32_t k = R.b0 / a.nbv, next = (k + 1u) * a.nbv;
+        VolumeDesc d;
+        for (int c = 0; c < 3; ++c) { d.dim[c] = a.dim[c]; d.bdim[c] = a.bdim[c]; }
+        d.fmt = a.fmt;
+        d.nbricks = p.ids[next] - first;
+        d.brick_map = p.map + (size_t)k * a.nbv;
+        d.masks = reinterpret_cast<const uint32_t*>(p.masks + (size_t)first * 8);
+        d.payload = p.payload + (size_t)first * kBytes;
+        d.palette = p.palette;
+        d.blocks = p.blocks + first;
+        p.descs[k] = d;
     }
     __syncthreads();
-    if (t == 0) {
-        flags[b] = any;
-        blocks_all[b] = (uint64_t)blk[0] | ((uint64_t)blk[1] << 32);
+    const uint32_t full = any;
+    if (full == 0u) return;
+    if (tid < 64u && ((full >> (tid >> 3)) & 1u)) {
+        const uint32_t b = R.b0 + (tid >> 3);
+        p.masks[(size_t)p.ids[b] * 8 + (tid & 7u)] = p.masks_all[(size_t)b * 8 + (tid & 7u)];
+    }
+    for_voxels(a, R, [&](uint32_t z, uint32_t y, uint32_t raw, bool) {
+        uint8_t* at = tile + (lane >> 3) * kPitch + ((lane & 7u) + 8u * y + 64u * (2u * wave + z)) * BPV;
+        if (BPV == 1) *at = (uint8_t)raw;   // the payload keeps the texel as stored
+        else *reinterpret_cast<uint32_t*>(at) = raw;
+    });
+    __syncthreads();
+    for (uint32_t c = tid; c < kRowBricks * kBytes / 16u; c += kRowThreads) {
+        const uint32_t k = c / (kBytes / 16u), o = c % (kBytes / 16u) * 16u;
+        if ((full >> k) & 1u)
+            *reinterpret_cast<uint4*>(p.payload + (size_t)p.ids[R.b0 + k] * kBytes + o) =
+                *reinterpret_cast<const uint4*>(tile + k * kPitch + o);
     }
 }
 
-// cube sides of all 8 octants packed 4 bits each (0 for a non-empty brick, 1 for an empty one)
-__global__ void k_cube_init(const uint32_t* flags, uint32_t* cube, uint32_t nb) {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < nb) cube[b] = flags[b] ? 0u : 0x11111111u;
-}
-
-// layer k over nvol volumes of bx*by*bz bricks each (neighbours within the same volume; outside
-// the volume counts as a side of VT_BRICK_CUBE_CAP)
-__global__ void k_cube_step(uint32_t* cube, uint32_t bx, uint32_t by, uint32_t bz, uint32_t nvol, uint32_t k) {
-    const uint32_t gb = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t nbv = bx * by * bz;
-    if (gb >= nbv * nvol) return;
-    const uint32_t cur = cube[gb];
-    if (cur == 0u) return;
-    const uint32_t base = (gb / nbv) * nbv, b = gb - base;
-    const int x = (int)(b % bx), y = (int)((b / bx) % by), z = (int)(b / (bx * by));
-    uint32_t out = cur;
-    for (uint32_t o = 0; o < 8; ++o) {
-        if (((cur >> (4u * o)) & 15u) != k) continue;
-        const int dx = (o & 1u) ? -1 : 1, dy = (o & 2u) ? -1 : 1, dz = (o & 4u) ? -1 : 1;
-        bool grow = true;
-        for (int n = 1; n < 8 && grow; ++n) {
-            const int X = x + ((n & 1) ? dx : 0), Y = y + ((n & 2) ? dy : 0), Z = z + ((n & 4) ? dz : 0);
-            if (X < 0 || Y < 0 || Z < 0 || X >= (int)bx || Y >= (int)by || Z >= (int)bz) continue;
-            const uint32_t nk = (cube[base + (uint32_t)X + bx * ((uint32_t)Y + by * (uint32_t)Z)] >> (4u * o)) & 15u;
-            grow = nk >= k;
-        }
-        if (grow) out += 1u << (4u * o);
-    }
-    if (out != cur) cube[gb] = out;
-}
-
-__global__ void k_radius_init(const uint32_t* flags, uint32_t* dist, uint32_t nb) {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < nb) dist[b] = flags[b] ? 0u : 255u;
-}
-
-// layer k over nvol volumes of bx*by*bz bricks each (neighbours within the same volume)
-__global__ void k_radius_step(uint32_t* dist, uint32_t bx, uint32_t by, uint32_t bz, uint32_t nvol, uint32_t k) {
-    const uint32_t gb = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t nbv = bx * by * bz;
-    if (gb >= nbv * nvol || dist[gb] != 255u) return;
-    const uint32_t base = (gb / nbv) * nbv, b = gb - base;
-    const int x = (int)(b % bx), y = (int)((b / bx) % by), z = (int)(b / (bx * by));
-    for (int dz = -1; dz <= 1; ++dz)
-        for (int dy = -1; dy <= 1; ++dy)
-            for (int dx = -1; dx <= 1; ++dx) {
-                const int X = x + dx, Y = y + dy, Z = z + dz;
-                if (X < 0 || Y < 0 || Z < 0 || X >= (int)bx || Y >= (int)by || Z >= (int)bz) continue;
-                if (dist[base + (uint32_t)X + bx * ((uint32_t)Y + by * (uint32_t)Z)] == k - 1u) {
-                    dist[gb] = k;
-                    return;
-                }
-            }
-}
-
-__global__ __launch_bounds__(512) void k_brick_scatter(BrickArgs a, const uint64_t* masks_all,
-                                                       const uint64_t* blocks_all, const uint32_t* ids,
-                                                       const uint32_t* flags, const uint32_t* dist, const uint32_t* cube,
-                                                       uint32_t* brick_map, uint64_t* masks, uint64_t* blocks,
-                                                       uint8_t* payload) {
-    const uint32_t b = blockIdx.x;
-    const uint32_t t = threadIdx.x;
-    const bool nonempty = flags[b] != 0;
-    const uint32_t id = ids[b];                            // pool slot
-    const uint32_t first = ids[(b / a.nbv) * a.nbv];        // pool slot of the volume's first brick
-    if (t == 0) {
-        uint32_t e = id - first;
-        if (!nonempty) {
-            e = VT_EMPTY_BRICK | ((min(dist[b], VT_BRICK_RADIUS_CAP + 1u) - 1u) << 24);
-            for (uint32_t o = 0; o < 8; ++o) e |= (((cube[b] >> (4u * o)) & 15u) - 1u) << (3u * o);
-        }
-        brick_map[b] = e;
-    }
-    if (!nonempty) return;
-    if (t < 8) masks[(size_t)id * 8 + t] = masks_all[(size_t)b * 8 + t];
-    if (t == 8) blocks[id] = blocks_all[b];
-    uint32_t bx, by, bz;
-    const size_t vbase = brick_coords(a, b, &bx, &by, &bz);
-    const uint32_t gx = bx * 8 + (t & 7), gy = by * 8 + ((t >> 3) & 7), gz = bz * 8 + (t >> 6);
-    uint32_t raw = 0;
-    if (gx < a.dim[0] && gy < a.dim[1] && gz < a.dim[2]) {
-        size_t ti = vbase + (size_t)a.remap[0][gx] +
-                    (size_t)a.dim[0] * ((size_t)a.remap[1][gy] + (size_t)a.dim[1] * a.remap[2][gz]);
-        (void)texel_rgba(a.dense, a.fmt, a.palette, ti, &raw);  // payload keeps the texel as stored
-    }
-    if (a.fmt == 0) payload[(size_t)id * 512 + t] = (uint8_t)raw;
-    else reinterpret_cast<uint32_t*>(payload)[(size_t)id * 512 + t] = raw;
-}
-
-// ---- exclusive scan of u32 flags (3 phases, 1024 elements per block) ----------------
+// ---- exclusive scan of the non-empty bricks ---------------------------------------------
 constexpr int kScanBlock = 1024;
+// Bricks that one workgroup numbers by itself (4 per thread and step, 19 us for 32768); more: 3
+// launches, 1024 per block (14 us for 32768, gaps not counted)
+constexpr uint32_t kScanOneMax = 16384;
 
 __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* total) {
     __shared__ uint32_t wsum[kScanBlock / 64];
@@ -229,9 +309,32 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* total) {
     return incl - v;
 }
 
-__global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const uint32_t* in, uint32_t n, uint32_t* block_sums) {
+// ids[0, nb) and the total in ids[nb]; counts (page-locked host memory): ids[k * nbv], k = 0..nvol
+__global__ __launch_bounds__(kScanBlock) void k_scan_one(const uint64_t* blocks_all, uint32_t nb, uint32_t* ids,
+                                                         uint32_t nbv, uint32_t nvol, uint32_t* counts) {
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < nb; base += 4u * kScanBlock) {
+        const uint32_t i = base + 4u * threadIdx.x;
+        uint32_t f[4], sum = 0, total;
+        for (uint32_t q = 0; q < 4; ++q) {
+            f[q] = i + q < nb && blocks_all[i + q] != 0ull ? 1u : 0u;
+            sum += f[q];
+        }
+        uint32_t at = carry + block_exclusive_scan(sum, &total);
+        for (uint32_t q = 0; q < 4; ++q) {
+            if (i + q < nb) ids[i + q] = at;
+            at += f[q];
+        }
+        carry += total;
+    }
+    if (threadIdx.x == 0) ids[nb] = carry;
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k <= nvol; k += kScanBlock) counts[k] = ids[k * nbv];
+}
+
+__global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const uint64_t* in, uint32_t n, uint32_t* block_sums) {
     uint32_t i = blockIdx.x * kScanBlock + threadIdx.x;
-    uint32_t v = i < n ? (in[i] != 0u ? 1u : 0u) : 0u;
+    uint32_t v = i < n && in[i] != 0ull ? 1u : 0u;
     uint32_t total;
     block_exclusive_scan(v, &total);
     if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
@@ -255,118 +358,154 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_blocks(uint32_t* block_sums
     if (threadIdx.x == 0) *grand_total = carry;
 }
 
-__global__ __launch_bounds__(kScanBlock) void k_scan_apply(const uint32_t* in, uint32_t n, const uint32_t* block_sums,
+__global__ __launch_bounds__(kScanBlock) void k_scan_apply(const uint64_t* in, uint32_t n, const uint32_t* block_sums,
                                                             uint32_t* out) {
     uint32_t i = blockIdx.x * kScanBlock + threadIdx.x;
-    uint32_t v = i < n ? (in[i] != 0u ? 1u : 0u) : 0u;
+    uint32_t v = i < n && in[i] != 0ull ? 1u : 0u;
     uint32_t total;
     uint32_t ex = block_exclusive_scan(v, &total);
     if (i < n) out[i] = ex + block_sums[blockIdx.x];
 }
 
-}  // namespace
-
-// Exclusive scan of (flag != 0) over n entries; *total_dev receives the count.
-hipError_t vt_scan_flags(const uint32_t* flags, uint32_t n, uint32_t* out, uint32_t* scratch_blocks, uint32_t* total_dev,
-                         hipStream_t s) {
-    uint32_t nb = (n + kScanBlock - 1) / kScanBlock;
-    if (nb == 0) nb = 1;
-    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kScanBlock), 0, s, flags, n, scratch_blocks);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(kScanBlock), 0, s, scratch_blocks, nb, total_dev);
-    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kScanBlock), 0, s, flags, n, scratch_blocks, out);
-    return hipGetLastError();
+__global__ void k_scan_counts(const uint32_t* ids, uint32_t nbv, uint32_t nvol, uint32_t* counts) {
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k <= nvol; k += gridDim.x * blockDim.x) counts[k] = ids[k * nbv];
 }
 
-// Brick nvol dense device volumes of one size (packed one after another).  Allocates one set
-// of pools for all of them (after one sync to learn the count); out[0] owns the allocations.
-int vt_brick_volume(const uint8_t* dense_dev, uint32_t fmt, const uint32_t* palette_dev, const uint16_t* remap_dev[3],
-                    const uint32_t dim[3], uint32_t nvol, VolumeStore* out, hipStream_t s) {
+constexpr size_t kKeepWorkspace = (size_t)64 << 20;   // a larger workspace is given back after its upload
+
+}  // namespace
+
+void vt_brick_free(BrickWork& w) {
+    hipFree(w.mem);
+    hipHostFree(w.counts);
+    if (w.counted) hipEventDestroy(w.counted);
+    w = BrickWork{};
+}
+
+// Brick nvol dense device volumes of one size (packed one after another; fmt 0: palette_host, 256
+// entries) and write their descriptors.  One pool for all of them, allocated once the non-empty bricks are
+// counted (the GPU works on the distances meanwhile); out[0] owns it.
+int vt_brick_volume(BrickWork& w, const uint8_t* dense_dev, uint32_t fmt, const uint32_t* palette_host,
+                    const uint32_t dim[3], uint32_t nvol, VolumeStore* out, VolumeDesc* descs, hipStream_t s) {
     if (nvol == 0) return -1;
     BrickArgs a{};
     a.dense = dense_dev;
-    a.palette = palette_dev;
     for (int k = 0; k < 3; ++k) {
-        a.remap[k] = remap_dev[k];
         a.dim[k] = dim[k];
         a.bdim[k] = (dim[k] + 7) / 8;
     }
     a.fmt = fmt;
-    a.nbv = a.bdim[0] * a.bdim[1] * a.bdim[2];
-    a.vol_texels = (size_t)dim[0] * dim[1] * dim[2];
-    const uint64_t nb64 = (uint64_t)a.nbv * nvol;
+    const uint64_t nb64 = (uint64_t)a.bdim[0] * a.bdim[1] * a.bdim[2] * nvol;
     if (nb64 >= 0x7FFFFFFFull) return -1;
-    const uint32_t nb = (uint32_t)nb64;
-    uint64_t *masks_all = nullptr, *blocks_all = nullptr;
-    uint32_t *flags = nullptr, *ids = nullptr, *blocks = nullptr, *total = nullptr, *dist = nullptr, *cube = nullptr;
-    const uint32_t nblk = (nb + kScanBlock - 1) / kScanBlock + 1;
-    auto free_temps = [&]() {
-        hipFree(masks_all); hipFree(blocks_all); hipFree(flags); hipFree(ids); hipFree(blocks); hipFree(total);
-        hipFree(dist); hipFree(cube);
-    };
-    if (hipMalloc(&masks_all, (size_t)nb * 64) != hipSuccess || hipMalloc(&blocks_all, (size_t)nb * 8) != hipSuccess ||
-        hipMalloc(&flags, (size_t)nb * 4) != hipSuccess || hipMalloc(&ids, (size_t)nb * 4) != hipSuccess ||
-        hipMalloc(&blocks, (size_t)nblk * 4) != hipSuccess || hipMalloc(&total, 4) != hipSuccess ||
-        hipMalloc(&dist, (size_t)nb * 4) != hipSuccess || hipMalloc(&cube, (size_t)nb * 4) != hipSuccess) {
-        free_temps();
+    a.nbv = a.bdim[0] * a.bdim[1] * a.bdim[2];
+    a.nb = (uint32_t)nb64;
+    a.rows_x = (a.bdim[0] + kRowBricks - 1) / kRowBricks;
+    a.vol_texels = (size_t)dim[0] * dim[1] * dim[2];
+    const uint32_t rows = a.rows_x * a.bdim[1] * a.bdim[2] * nvol, tb = (a.nb + 255) / 256;
+    const uint32_t nblk = (a.nb + kScanBlock - 1) / kScanBlock;
+    // workspace: masks, block masks, ids and total, two distance arrays, scan sums, palette
+    const size_t n = a.nb;
+    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t at_blocks = up(n * 64), at_ids = at_blocks + up(n * 8), at_d0 = at_ids + up(n * 4 + 4),
+                 at_d1 = at_d0 + up(n * 4), at_sums = at_d1 + up(n * 4), at_pal = at_sums + up((size_t)nblk * 4),
+                 need = at_pal + 1024;
+    if (need > w.cap) {
+        hipFree(w.mem);
+        w.mem = nullptr;
+        w.cap = 0;
+        if (hipMalloc(&w.mem, need) != hipSuccess) return -1;
+        w.cap = need;
+    }
+    if (nvol + 1 > w.counts_cap) {
+        hipHostFree(w.counts);
+        w.counts = nullptr;
+        w.counts_cap = 0;
+        const uint32_t cap = std::max(1024u, nvol + 1);
+        if (hipHostMalloc(reinterpret_cast<void**>(&w.counts), (size_t)cap * 4, hipHostMallocDefault) != hipSuccess) return -1;
+        w.counts_cap = cap;
+    }
+    if (!w.counted && hipEventCreateWithFlags(&w.counted, hipEventDisableTiming) != hipSuccess) return -1;
+    char* const mem = static_cast<char*>(w.mem);
+    uint64_t* const masks_all = reinterpret_cast<uint64_t*>(mem);
+    uint64_t* const blocks_all = reinterpret_cast<uint64_t*>(mem + at_blocks);
+    uint32_t* const ids = reinterpret_cast<uint32_t*>(mem + at_ids);
+    uint32_t* const d0 = reinterpret_cast<uint32_t*>(mem + at_d0);
+    uint32_t* const d1 = reinterpret_cast<uint32_t*>(mem + at_d1);
+    uint32_t* const sums = reinterpret_cast<uint32_t*>(mem + at_sums);
+    uint32_t* const pal = reinterpret_cast<uint32_t*>(mem + at_pal);
+    if (fmt == 0) {
+        if (hipMemcpyAsync(pal, palette_host, 1024, hipMemcpyHostToDevice, s) != hipSuccess) return -1;
+        a.palette = pal;
+    }
+    hipLaunchKernelGGL(k_brick_classify, dim3(rows), dim3(kRowThreads), 0, s, a, masks_all, blocks_all);
+    if (a.nb <= kScanOneMax) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kScanBlock), 0, s, blocks_all, a.nb, ids, a.nbv, nvol, w.counts);
+    } else {
+        hipLaunchKernelGGL(k_scan_reduce, dim3(nblk), dim3(kScanBlock), 0, s, blocks_all, a.nb, sums);
+        hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(kScanBlock), 0, s, sums, nblk, ids + a.nb);
+        hipLaunchKernelGGL(k_scan_apply, dim3(nblk), dim3(kScanBlock), 0, s, blocks_all, a.nb, sums, ids);
+        hipLaunchKernelGGL(k_scan_counts, dim3(std::min(256u, nvol / 256u + 1u)), dim3(256), 0, s, ids, a.nbv, nvol,
+                           w.counts);
+    }
+    hipError_t e = hipEventRecord(w.counted, s);
+    hipLaunchKernelGGL(k_dist_x, dim3(tb), dim3(256), 0, s, blocks_all, a.nb, a.bdim[0], d0);
+    hipLaunchKernelGGL(k_dist_y, dim3(tb), dim3(256), 0, s, d0, a.nb, a.bdim[0], a.bdim[1], d1);
+    hipLaunchKernelGGL(k_dist_z, dim3(tb), dim3(256), 0, s, d1, a.nb, a.bdim[0] * a.bdim[1], a.bdim[2], d0);
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e == hipSuccess) e = hipEventSynchronize(w.counted);
+    const size_t bpv = fmt == 0 ? 1 : 4;
+    char* pool = nullptr;
+    size_t cnt = 0, at_masks = 0, at_pblocks = 0, at_payload = 0, at_ppal = 0;
+    if (e == hipSuccess) {
+        cnt = w.counts[nvol];
+        at_masks = up(n * 4);
+        at_pblocks = at_masks + up(cnt * 64);
+        at_payload = at_pblocks + up(cnt * 8);
+        at_ppal = at_payload + up(cnt * 512 * bpv);
+        e = hipMalloc(reinterpret_cast<void**>(&pool), at_ppal + 1024);
+    }
+    PoolArgs p{};
+    if (e == hipSuccess) {
+        p.masks_all = masks_all;
+        p.blocks_all = blocks_all;
+        p.ids = ids;
+        p.entry = d0;
+        p.map = reinterpret_cast<uint32_t*>(pool);
+        p.masks = reinterpret_cast<uint64_t*>(pool + at_masks);
+        p.blocks = reinterpret_cast<uint64_t*>(pool + at_pblocks);
+        p.payload = reinterpret_cast<uint8_t*>(pool + at_payload);
+        p.palette = fmt == 0 ? reinterpret_cast<uint32_t*>(pool + at_ppal) : nullptr;
+        p.descs = descs;
+        if (fmt == 0) hipLaunchKernelGGL(k_brick_scatter<1>, dim3(rows), dim3(kRowThreads), 0, s, a, p);
+        else hipLaunchKernelGGL(k_brick_scatter<4>, dim3(rows), dim3(kRowThreads), 0, s, a, p);
+        e = hipGetLastError();
+    }
+    const hipError_t done = hipStreamSynchronize(s);   // (also before the workspace may go)
+    if (w.cap > kKeepWorkspace) {
+        hipFree(w.mem);
+        w.mem = nullptr;
+        w.cap = 0;
+    }
+    if (e != hipSuccess || done != hipSuccess) {
+        hipFree(pool);
         return -1;
     }
-    hipLaunchKernelGGL(k_brick_classify, dim3(nb), dim3(512), 0, s, a, masks_all, blocks_all, flags);
-    vt_scan_flags(flags, nb, ids, blocks, total, s);
-    hipLaunchKernelGGL(k_radius_init, dim3((nb + 255) / 256), dim3(256), 0, s, flags, dist, nb);
-    const uint32_t layers = std::min<uint32_t>(VT_BRICK_RADIUS_CAP + 1u,
-                                               std::max(a.bdim[0], std::max(a.bdim[1], a.bdim[2])));
-    for (uint32_t k = 1; k <= layers; ++k)
-        hipLaunchKernelGGL(k_radius_step, dim3((nb + 255) / 256), dim3(256), 0, s, dist, a.bdim[0], a.bdim[1],
-                           a.bdim[2], nvol, k);
-    hipLaunchKernelGGL(k_cube_init, dim3((nb + 255) / 256), dim3(256), 0, s, flags, cube, nb);
-    for (uint32_t k = 1; k < VT_BRICK_CUBE_CAP; ++k)
-        hipLaunchKernelGGL(k_cube_step, dim3((nb + 255) / 256), dim3(256), 0, s, cube, a.bdim[0], a.bdim[1],
-                           a.bdim[2], nvol, k);
-    // pool slot of each volume's first brick (ids[k * nbv]) and the total
-    std::vector<uint32_t> first(nvol + 1, 0);
-    hipMemcpy2DAsync(first.data(), 4, ids, (size_t)a.nbv * 4, 4, nvol, hipMemcpyDeviceToHost, s);
-    hipMemcpyAsync(&first[nvol], total, 4, hipMemcpyDeviceToHost, s);
-    hipError_t e = hipStreamSynchronize(s);
-    int rc = 0;
-    if (e != hipSuccess) rc = -1;
-    const uint32_t count = first[nvol];
-    const size_t bpv = fmt == 0 ? 1 : 4;
-    uint32_t* pool_map = nullptr;
-    uint32_t* pool_masks = nullptr;
-    uint64_t* pool_blocks = nullptr;
-    uint8_t* pool_payload = nullptr;
-    if (rc == 0) {
-        const size_t cnt = count ? count : 1;
-        if (hipMalloc(&pool_map, (size_t)nb * 4) != hipSuccess || hipMalloc(&pool_masks, cnt * 64) != hipSuccess ||
-            hipMalloc(&pool_blocks, cnt * 8) != hipSuccess || hipMalloc(&pool_payload, cnt * 512 * bpv) != hipSuccess) {
-            hipFree(pool_map); hipFree(pool_masks); hipFree(pool_blocks); hipFree(pool_payload);
-            rc = -1;
-        }
+    for (uint32_t k = 0; k < nvol; ++k) {
+        VolumeStore& o = out[k];
+        const size_t first = w.counts[k];
+        o.owner = k == 0;
+        o.pool = pool;
+        o.nbricks = w.counts[k + 1] - w.counts[k];
+        o.fmt = fmt;
+        for (int c = 0; c < 3; ++c) { o.dim[c] = dim[c]; o.bdim[c] = a.bdim[c]; }
+        o.brick_map = p.map + (size_t)k * a.nbv;
+        o.masks = reinterpret_cast<uint32_t*>(p.masks + first * 8);
+        o.payload = p.payload + first * 512 * bpv;
+        o.blocks = p.blocks + first;
+        o.palette = p.palette;
+        o.bytes = (size_t)a.nbv * 4 + (size_t)o.nbricks * (64 + 8 + 512 * bpv);
     }
-    if (rc == 0) {
-        hipLaunchKernelGGL(k_brick_scatter, dim3(nb), dim3(512), 0, s, a, masks_all, blocks_all, ids, flags, dist, cube,
-                           pool_map, reinterpret_cast<uint64_t*>(pool_masks), pool_blocks, pool_payload);
-        if (hipGetLastError() != hipSuccess) rc = -1;
-        if (hipStreamSynchronize(s) != hipSuccess) rc = -1;
-        if (rc != 0) { hipFree(pool_map); hipFree(pool_masks); hipFree(pool_blocks); hipFree(pool_payload); }
-    }
-    if (rc == 0) {
-        for (uint32_t k = 0; k < nvol; ++k) {
-            VolumeStore& o = out[k];
-            o.owner = k == 0;
-            o.nbricks = first[k + 1] - first[k];
-            o.fmt = fmt;
-            for (int c = 0; c < 3; ++c) { o.dim[c] = dim[c]; o.bdim[c] = a.bdim[c]; }
-            o.brick_map = pool_map + (size_t)k * a.nbv;
-            o.masks = pool_masks + (size_t)first[k] * 16;
-            o.payload = pool_payload + (size_t)first[k] * 512 * bpv;
-            o.blocks = pool_blocks + first[k];
-            o.palette = const_cast<uint32_t*>(palette_dev);
-            o.bytes = (size_t)a.nbv * 4 + (size_t)o.nbricks * (64 + 8 + 512 * bpv);
-        }
-    }
-    free_temps();
-    return rc;
+    return 0;
 }
 
 namespace {

@@ -22,14 +22,22 @@ struct VolumeStore {
     uint32_t* palette = nullptr;
     uint64_t* blocks = nullptr;
     size_t bytes = 0;
-    bool owner = true;          // frees brick_map/masks/payload/palette (volumes bricked together share them)
+    void* pool = nullptr;       // the allocation that holds them all
+    bool owner = true;          // frees the pool (volumes bricked together share it)
 };
 
 // upload.hip
-hipError_t vt_scan_flags(const uint32_t* flags, uint32_t n, uint32_t* out, uint32_t* scratch_blocks, uint32_t* total_dev,
-                         hipStream_t s);
-int vt_brick_volume(const uint8_t* dense_dev, uint32_t fmt, const uint32_t* palette_dev, const uint16_t* remap_dev[3],
-                    const uint32_t dim[3], uint32_t nvol, VolumeStore* out, hipStream_t s);
+// Workspace of uploads, kept from one to the next (bounded, see upload.hip).
+struct BrickWork {
+    void* mem = nullptr;
+    size_t cap = 0;
+    uint32_t* counts = nullptr;      // page-locked: non-empty bricks before each volume
+    uint32_t counts_cap = 0;
+    hipEvent_t counted = nullptr;
+};
+int vt_brick_volume(BrickWork& w, const uint8_t* dense_dev, uint32_t fmt, const uint32_t* palette_host,
+                    const uint32_t dim[3], uint32_t nvol, VolumeStore* out, VolumeDesc* descs, hipStream_t s);
+void vt_brick_free(BrickWork& w);
 int vt_debrick(const VolumeDesc& v, uint8_t* dense_dev, hipStream_t s);
 
 // lbvh.hip: builds InstanceGPU records and the LBVH from n ABI records on the device.

@@ -13,22 +13,20 @@
 // are deterministic) and Adam state are FP32.
 //
 // Kernels:
-//   k_conv3x3        forward conv (+bias, ReLU) and backward-data conv: dX = conv(dY, W')
-//                    with W'[ci][8-tap][co] = W[co][tap][ci]; its epilogue multiplies by the
-//                    ReLU mask of the layer that produced X (X > 0).  Each wave computes 32
-//                    pixels x all output channels; A fragments (8 channels of one pixel at
-//                    one tap) are 16-byte loads from NHWC tensors, B fragments from the
-//                    [co][tap][ci] weight rows.  Weights are the first MFMA operand, so a
-//                    lane's outputs are 4 consecutive channels of one pixel.  For inputs of
-//                    up to 160 channels the same computation runs from LDS:
-//                    k_conv3x3_res (persistent workgroups of 8 waves with the layer's weights
-//                    resident in LDS, 16 x 16 pixel tiles with their halo, the next tile
-//                    fetched into registers during the current one, a software-pipelined K
-//                    loop with no barrier) for up to 96 channels where weights and a tile
-//                    fit in 160 KiB, else k_conv3x3_tile (16 x 8 tiles, weights streamed
-//                    through LDS in 32-wide K slices).  Both can pool their output (2x2
-//                    mean) in the epilogue and read the decoder's upsampled channels from
-//                    the lower level in their staging.
+//   forward conv (+bias, ReLU) and backward-data conv: dX = conv(dY, W') with W'[ci][8-tap][co] =
+//                    W[co][tap][ci]; its epilogue multiplies by the ReLU mask of the layer that
+//                    produced X (X > 0).  A fragments are 8 channels of one pixel at one tap, read
+//                    from an LDS tile of the NHWC input with its halo, B fragments 8 channels of a
+//                    [co][tap][ci] weight row.  Weights are the first MFMA operand, so a lane's
+//                    outputs are 4 consecutive channels of one pixel.
+//   k_conv3x3_res    persistent workgroups of 8 waves with the layer's weights resident in LDS, 16 x 16
+//                    pixel tiles, the next tile fetched into registers during the current one, a
+//                    software-pipelined K loop with no barrier: inputs of up to 96 channels
+//                    where weights and a tile fit in 160 KiB and there are tiles enough.
+//   k_conv3x3_split  16 x 8 pixel tiles with the output channels split over workgroups, weights from L2
+//                    into registers several K steps ahead: everything else.
+//                    Both can pool their output (2x2 mean) in the epilogue and read the decoder's
+//                    upsampled channels from the lower level in their staging.
 //   k_conv3x3_wgrad  dW[co][tap][ci] = sum_p dY[p][co] X[p+tap][ci] over a chunk of pixel tiles,
 //                    all nine taps of a block of input channels in registers, the operands
 //                    transposed on the way out of LDS; dbias in the same pass.
@@ -52,7 +50,6 @@ constexpr int kInCh = 16;       // input feature channels (10 used)
 constexpr int kOutCh = 3;
 constexpr int kLayers = 19;
 constexpr int kMaxWidth = 96;   // widest layer (accumulators of the weight-gradient kernel)
-constexpr uint32_t kConvPix = 128;
 constexpr float kAlbedoEps = 0.01f;  // demodulation: irradiance = radiance / (albedo + eps)
 constexpr float kLogMax = 16.0f;     // clamp of the predicted log irradiance
 
@@ -83,30 +80,30 @@ struct ConvArgs {
     void* out;               // N x H x W x out_stride, channels [out_off, out_off + Cout)
     const uint16_t* mask;    // MASK: N x H x W x mask_stride; out = 0 where mask <= 0
     uint16_t* pool;          // optional: 2x2 mean pool of the BF16 output, N x H/2 x W/2 x Cout
-    const uint16_t* up;      // optional: input channels [0, up_C) read from this N x H/2 x W/2 x up_C
-                             // tensor at (y/2, x/2) (nearest upsampling), the rest from `in`
+    const uint16_t* up;      // input channels [0, up_C) read from this N x H/2 x W/2 x up_C tensor at
+                             // (y/2, x/2) (nearest upsampling), the rest from `in`; up_C = 0: `in`
     uint32_t up_C;
     uint32_t in_stride, out_stride, out_off, mask_stride;
     uint32_t N, H, W, Cin, Cout;
 };
 
 // Epilogue of the LDS-tiled kernels (waves of two 16-pixel rows, weights as the first MFMA
-// operand: a lane holds channels 16j + 4g .. 16j + 4g + 3 of pixel r of rows m = 0, 1) for a
+// operand: a lane holds channels cobase + 16j + 4g .. + 3 of pixel r of rows m = 0, 1) for a
 // layer whose BF16 output is also pooled (a.pool; H and W even, 4-aligned strides and
 // offset).  Rows m = 0, 1 are an even/odd row pair (tile origins are multiples of 8) and lanes
 // r, r ^ 1 an even/odd column pair, so the pooled value comes from this lane and its
-// neighbour with k_pool_fwd's operations: the four BF16 outputs summed in row-major order,
+// neighbour: the four BF16 outputs summed in row-major order,
 // times 0.25, rounded to BF16.  Every lane reaches the shuffles; only stores are guarded.
 template <int NT, bool RELU>
 __device__ __forceinline__ void epilogue_pool(const ConvArgs& a, const f32x4 (&acc)[2][NT], const float (&bias)[NT][4],
-                                              uint32_t n, int x, int y0, uint32_t g, uint32_t r) {
+                                              uint32_t cobase, uint32_t n, int x, int y0, uint32_t g, uint32_t r) {
     const bool xin = x < (int)a.W, yin = y0 < (int)a.H;
     const size_t img = (size_t)n * a.H * a.W;
     const uint32_t hw = a.W / 2u;
     const size_t q = ((size_t)n * (a.H / 2u) + (size_t)(y0 >> 1)) * hw + (size_t)(x >> 1);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const uint32_t co0 = (uint32_t)j * 16u + 4u * g;
+        const uint32_t co0 = cobase + (uint32_t)j * 16u + 4u * g;
         const bool cin = co0 < a.Cout;
         uint32_t pk[2][2];
 #pragma unroll
@@ -144,239 +141,156 @@ __device__ __forceinline__ void epilogue_pool(const ConvArgs& a, const f32x4 (&a
     }
 }
 
-template <int NT, bool RELU, bool OUTF, bool MASK>
-__global__ __launch_bounds__(256) void k_conv3x3(ConvArgs a) {
+// 16 bytes of a tile's halo: channels c .. c + 7 of pixel (y, x) of image n, zeros outside the image.  The
+// load is unconditional (a clamped address): conditional ones make a branch each, and a wait
+// for every outstanding load where the branches join.  in: whether to keep the value (the
+// caller selects, where it stores).
+__device__ __forceinline__ u32x4 halo_chunk(const ConvArgs& a, uint32_t n, int y, int x, uint32_t c, bool& in) {
+    in = in && y >= 0 && y < (int)a.H && x >= 0 && x < (int)a.W;
+    const uint32_t yc = (uint32_t)min(max(y, 0), (int)a.H - 1), xc = (uint32_t)min(max(x, 0), (int)a.W - 1);
+    const uint16_t* const p = a.in + ((size_t)(n * a.H + yc) * a.W + xc) * a.in_stride + c;
+    const uint16_t* const q = a.up + ((size_t)(n * (a.H >> 1) + (yc >> 1)) * (a.W >> 1) + (xc >> 1)) * a.up_C + c;
+    return *reinterpret_cast<const u32x4*>(c < a.up_C ? q : p);
+}
+
+// Convolution over kTileX x kTileY pixel tiles with the output channels split over workgroups (4
+// waves, grid: tiles x groups of 16 channels), for the layers that do not fill the GPU otherwise: the
+// lower levels of the network, training batches, small frames.  The input tile with a one-pixel
+// halo is staged in LDS once (zeros outside the image), so the nine taps of each pixel read LDS.  Each wave
+// owns two rows of 16 pixels.  Weight fragments come straight from the [co][tap][ci] rows in L2, kDepth
+// K steps ahead in registers, the first ones before the tile is staged: the K loop has no barrier
+// and waits for no load it has just issued.
+// Bound by latency: a launch of 8 images of 8 x 8 to 64 x 64 pixels is a few microseconds of dependent
+// steps (the tile, 9 Cin / 32 K steps) on workgroups that used to be too few (8 for the lowest level, each
+// with all output channels and a barrier per K step): 27 such launches of a fine-tuning step 431 -> 224
+// us, the lower levels of a 720p inference 170 -> 122 us.  Two groups of channels per wave were no
+// faster anywhere (218 and 126 us).
+constexpr int kTileX = 16, kTileY = 8;
+constexpr uint32_t kResMaxCin = 96;
+constexpr uint32_t kDepth = 9;
+
+inline size_t conv_split_lds(uint32_t cin) { return (size_t)(kTileY + 2) * (kTileX + 2) * (cin + 8u) * 2u; }
+
+template <bool RELU, bool OUTF, bool MASK>
+__global__ __launch_bounds__(256) void k_conv3x3_split(ConvArgs a, uint32_t ntx, uint32_t nty) {
+    constexpr int MT = 2, NG = 1;   // rows of pixels, 16-channel groups of a wave
+    extern __shared__ __align__(16) uint16_t tile[];  // (kTileY + 2) x (kTileX + 2) pixels x cs
+    const uint32_t cs = a.Cin + 8u;                   // LDS pixel stride (16 B of padding)
+    const uint32_t tx = blockIdx.x % ntx, rest = blockIdx.x / ntx, n = rest / nty;
+    const int tx0 = (int)tx * kTileX, ty0 = (int)(rest % nty) * kTileY;
+    const uint32_t cobase = blockIdx.y * 16u * NG;
+    const size_t img = (size_t)n * a.H * a.W;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t g = lane >> 4, r = lane & 15u;
-    const uint32_t HW = a.H * a.W, P = a.N * HW;
-    const uint32_t pbase = blockIdx.x * kConvPix + wave * 32u;
-    int py[2], px[2];
-    uint32_t img[2];
-    bool pv[2];
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const uint32_t p = pbase + m * 16u + r;
-        pv[m] = p < P;
-        const uint32_t q = pv[m] ? p : 0u;
-        const uint32_t n = q / HW, rem = q - n * HW;
-        py[m] = (int)(rem / a.W);
-        px[m] = (int)(rem - (uint32_t)py[m] * a.W);
-        img[m] = n * HW;
-    }
-    f32x4 acc[2][NT];
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[m][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t K = 9u * a.Cin;
-    for (uint32_t k0 = 0; k0 < K; k0 += 32u) {
-        const uint32_t k = k0 + 8u * g;
-        const bool kv = k < K;
-        uint32_t tap = 0, ci = 0;
-        if (kv) {
-            tap = k / a.Cin;
-            ci = k - tap * a.Cin;
-        }
-        const int dy = (int)(tap / 3u) - 1, dx = (int)(tap % 3u) - 1;
-        bf16x8 A[2];
+    const uint32_t S = (K + 32u * kDepth - 1u) / (32u * kDepth) * kDepth;   // K steps, whole rings
+    // this lane's weight rows (those past Cout repeat the last: outputs nobody stores)
+    const uint16_t* wrow[NG];
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            const int yy = py[m] + dy, xx = px[m] + dx;
-            const bool ok = kv && pv[m] && yy >= 0 && yy < (int)a.H && xx >= 0 && xx < (int)a.W;
-            A[m] = ok ? ld8(a.in + (size_t)(img[m] + (uint32_t)yy * a.W + (uint32_t)xx) * a.in_stride + ci) : zero8();
-        }
+    for (int j = 0; j < NG; ++j) wrow[j] = a.w + (size_t)min(cobase + 16u * j + r, a.Cout - 1u) * K;
+    u32x4 B[kDepth][NG];
+    // (past 9 Cin a clamped address; the zeros are selected where the fragment is used)
+    auto fetch = [&](uint32_t ks, u32x4 (&dst)[NG]) {
+        const uint32_t k = min(32u * ks + 8u * g, K - 8u);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const uint32_t co = (uint32_t)j * 16u + r;
-            const bf16x8 B = (kv && co < a.Cout) ? ld8(a.w + (size_t)co * K + k) : zero8();
-            // weights as the first operand: D rows are output channels, columns pixels
-            acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B, A[0], acc[0][j], 0, 0, 0);
-            acc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B, A[1], acc[1][j], 0, 0, 0);
-        }
-    }
-    // D layout: lane holds output channels 16j + 4g .. 16j + 4g + 3 of pixel r of tile m
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const uint32_t p = pbase + (uint32_t)m * 16u + r;
-        if (p >= P) continue;
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t co = (uint32_t)j * 16u + 4u * g + (uint32_t)i;
-                if (co >= a.Cout) continue;
-                float v = acc[m][j][i] + (a.bias ? a.bias[co] : 0.0f);
-                if (RELU) v = v > 0.0f ? v : 0.0f;
-                if (MASK && !(bf2f(a.mask[(size_t)p * a.mask_stride + co]) > 0.0f)) v = 0.0f;
-                if (OUTF) reinterpret_cast<float*>(a.out)[(size_t)p * a.out_stride + a.out_off + co] = v;
-                else reinterpret_cast<uint16_t*>(a.out)[(size_t)p * a.out_stride + a.out_off + co] = f2bf(v);
-            }
-    }
-}
-
-// Tiled form of k_conv3x3 for inputs of at most kTileMaxCin channels: a workgroup (4 waves)
-// computes a kTileX x (4 MT) pixel tile of one image.  The input tile with a one-pixel halo is
-// staged in LDS once (zeros outside the image), so the nine taps of each pixel read LDS
-// instead of fetching the same 16-byte chunks again from L1/L2.  Each wave owns MT rows of 16
-// pixels (MT 16-row MFMA tiles) x all output channels, so every weight fragment it reads feeds
-// MT MFMAs.  The weights pass through LDS in 32-wide K slices, double-buffered: each slice is
-// fetched from global memory into registers while the previous one feeds the MFMAs.  K chunks,
-// operands and their order are those of k_conv3x3 (steps past 9 Cin add zero products), so
-// every output is the same sum in the same order.
-constexpr int kTileX = 16;
-constexpr uint32_t kTileMaxCin = 160;   // the sliced kernel (the resident one: kResMaxCin)
-constexpr uint32_t kResMaxCin = 96;
-
-// LDS row pitch (elements) of a staged 32-wide K slice of the weights: 80 B rows, so the 16
-// rows one MFMA operand reads start in different banks
-constexpr uint32_t kBPitch = 40;
-
-template <int NT>
-inline size_t conv_tile_lds(int mt, uint32_t cin) {
-    return ((size_t)(4 * mt + 2) * (kTileX + 2) * (cin + 8u) + 2u * NT * 16u * kBPitch) * 2u;
-}
-
-template <int MT, int NT, bool RELU, bool OUTF, bool MASK>
-__global__ __launch_bounds__(256) void k_conv3x3_tile(ConvArgs a) {
-    constexpr int TY = 4 * MT;
-    extern __shared__ __align__(16) uint16_t tile[];  // (TY + 2) x (kTileX + 2) pixels x cs, then
-                                                      // 2 x NT*16 rows x kBPitch weight slices
-    const uint32_t cs = a.Cin + 8u;                   // LDS pixel stride (16 B of padding)
-    uint16_t* const bsl = tile + (size_t)((TY + 2) * (kTileX + 2)) * cs;
-    const uint32_t n = blockIdx.z;
-    const int tx0 = (int)blockIdx.x * kTileX, ty0 = (int)blockIdx.y * TY;
-    const size_t img = (size_t)n * a.H * a.W;
+        for (int j = 0; j < NG; ++j) dst[j] = *reinterpret_cast<const u32x4*>(wrow[j] + k);
+    };
     // cpp + 1 chunks of 16 B per pixel: its channels, then its padding, set to zeros (K past
     // the end reads the padding, so no select is needed)
     const uint32_t cpp = a.Cin / 8u + 1u;
-    const uint32_t total = (uint32_t)((TY + 2) * (kTileX + 2)) * cpp;
-    // i / cpp as (i * inv) >> 20: exact while i < 2^20 / cpp (cpp <= 21, i < 6000); i * inv
+    const uint32_t total = (uint32_t)((kTileY + 2) * (kTileX + 2)) * cpp;
+    // i / cpp as (i * inv) >> 20: exact while i < 2^20 / cpp (cpp <= 25, i < 6600); i * inv
     // stays below 2^32 since cpp >= 2
     const uint32_t inv = ((1u << 20) + cpp - 1u) / cpp;
     // staging in batches: all loads of a batch are issued before its LDS stores, so a thread
     // waits for one round trip per batch instead of one per 16-byte chunk
     constexpr uint32_t kBatch = 8;
-    for (uint32_t i0 = 0; i0 < total; i0 += 256u * kBatch) {
+    auto stage = [&](uint32_t i0, bool first) {
         u32x4 v[kBatch];
+        bool ok[kBatch];
 #pragma unroll
         for (uint32_t b = 0; b < kBatch; ++b) {
-            const uint32_t i = i0 + threadIdx.x + 256u * b;
+            const uint32_t i = min(i0 + threadIdx.x + 256u * b, total - 1u);
             const uint32_t pix = (i * inv) >> 20, c8 = i - pix * cpp;
-            const int ly = (int)(pix / (uint32_t)(kTileX + 2)), lx = (int)(pix % (uint32_t)(kTileX + 2));
-            const int y = ty0 + ly - 1, x = tx0 + lx - 1;
-            v[b] = u32x4{0u, 0u, 0u, 0u};
-            if (i < total && c8 + 1u < cpp && y >= 0 && y < (int)a.H && x >= 0 && x < (int)a.W)
-                v[b] = *reinterpret_cast<const u32x4*>(
-                    (a.up && 8u * c8 < a.up_C)
-                        ? a.up + (((size_t)n * (a.H >> 1) + (size_t)(y >> 1)) * (a.W >> 1) + (size_t)(x >> 1)) * a.up_C +
-                              8u * c8
-                        : a.in + (img + (size_t)y * a.W + (size_t)x) * a.in_stride + 8u * c8);
+            ok[b] = c8 + 1u < cpp;
+            v[b] = halo_chunk(a, n, ty0 + (int)(pix / (uint32_t)(kTileX + 2)) - 1, tx0 + (int)(pix % (uint32_t)(kTileX + 2)) - 1,
+                              8u * min(c8, cpp - 2u), ok[b]);
+        }
+        if (first) {   // after the tile's loads, which complete first
+#pragma unroll
+            for (uint32_t d = 0; d < kDepth; ++d) fetch(d, B[d]);
         }
 #pragma unroll
         for (uint32_t b = 0; b < kBatch; ++b) {
             const uint32_t i = i0 + threadIdx.x + 256u * b;
             const uint32_t pix = (i * inv) >> 20, c8 = i - pix * cpp;
-            if (i < total) *reinterpret_cast<u32x4*>(tile + (size_t)pix * cs + 8u * c8) = v[b];
+            if (i < total) *reinterpret_cast<u32x4*>(tile + (size_t)pix * cs + 8u * c8) = ok[b] ? v[b] : u32x4{0u, 0u, 0u, 0u};
         }
-    }
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t g = lane >> 4, r = lane & 15u;
-    f32x4 acc[MT][NT];
+    };
+    stage(0u, true);
+    for (uint32_t i0 = 256u * kBatch; i0 < total; i0 += 256u * kBatch) stage(i0, false);
+    __syncthreads();
+    f32x4 acc[MT][NG];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[m][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const uint32_t K = 9u * a.Cin;
-    const uint32_t S = (K + 31u) / 32u;
-    // weight slices: slice s holds rows co < NT*16, k = 32s .. 32s+31 (zeros past Cout or K);
-    // piece q of a slice is 16 B: row q / 4, k offset 8 (q % 4)
-    constexpr uint32_t kPieces = (uint32_t)NT * 64u;
-    constexpr uint32_t kPer = (kPieces + 255u) / 256u;
-    // loads are unconditional (a clamped address, zeros selected afterwards): conditional
-    // loads make the compiler wait for every outstanding load at the join
-    // every thread fetches and stores kPer pieces: past kPieces it repeats a piece (the same
-    // value to the same place), so nothing is conditional and the compiler keeps the fetch
-    // where it is issued instead of sinking it next to the store
-    auto piece = [&](uint32_t t) -> uint32_t {
-        const uint32_t q = threadIdx.x + 256u * t;
-        return q < kPieces ? q : q - kPieces * ((q - kPieces) / kPieces + 1u);
-    };
-    // (pieces outside the weights are fetched from a clamped address and zeroed at the store,
-    // so the wait for the fetch comes at the store)
-    auto fetch = [&](uint32_t sl, u32x4 (&dst)[kPer], bool (&ok)[kPer]) {
-#pragma unroll
-        for (uint32_t t = 0; t < kPer; ++t) {
-            const uint32_t q = piece(t);
-            const uint32_t co = q >> 2, kk = 32u * sl + 8u * (q & 3u);
-            ok[t] = co < a.Cout && kk < K;
-            dst[t] = *reinterpret_cast<const u32x4*>(a.w + (ok[t] ? (size_t)co * K + kk : 0u));
-        }
-    };
-    auto store = [&](uint32_t buf, const u32x4 (&src)[kPer], const bool (&ok)[kPer]) {
-#pragma unroll
-        for (uint32_t t = 0; t < kPer; ++t) {
-            const uint32_t q = piece(t);
-            *reinterpret_cast<u32x4*>(bsl + (size_t)buf * (NT * 16u * kBPitch) + (q >> 2) * kBPitch + 8u * (q & 3u)) =
-                ok[t] ? src[t] : u32x4{0u, 0u, 0u, 0u};
-        }
-    };
-    u32x4 nx[kPer];
-    bool nok[kPer];
-    fetch(0, nx, nok);
-    store(0, nx, nok);
-    __syncthreads();
+        for (int j = 0; j < NG; ++j) acc[m][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     // k = 32 s + 8 g as (tap, channel): tap = (k * invc) >> 20, exact while k < 2^20 / Cin
-    // (k < 9 Cin + 32 <= 1472)
+    // (k < 9 Cin + 32 kDepth <= 2016)
     const uint32_t invc = ((1u << 20) + a.Cin - 1u) / a.Cin;
     const uint32_t rowbase = (uint32_t)MT * wave;
-    for (uint32_t sl = 0; sl < S; ++sl) {
-        const uint32_t cur = sl & 1u;
-        // the next slice (the last one again past the end: a buffer nobody reads)
-        fetch(min(sl + 1u, S - 1u), nx, nok);
-        __builtin_amdgcn_sched_barrier(0);
-        const uint32_t k = 32u * sl + 8u * g;
+    const uint16_t* const abase = tile + (size_t)((rowbase + 1u) * (kTileX + 2) + r + 1u) * cs;
+    const uint32_t rstep = (uint32_t)(kTileX + 2) * cs;
+    auto load_a = [&](uint32_t ks, bf16x8 (&A)[MT]) {
+        const uint32_t k = 32u * ks + 8u * g;
         const uint32_t tap = (k * invc) >> 20;
         const bool kv = tap < 9u;
-        const uint32_t tp = kv ? tap : 4u, cc = kv ? k - tap * a.Cin : a.Cin;   // past K: the zero padding
-        const uint32_t ty = (tp >= 3u ? 1u : 0u) + (tp >= 6u ? 1u : 0u);
-        const int dy = (int)ty - 1, dx = (int)(tp - 3u * ty) - 1;
-        bf16x8 A[MT];
+        const int tp = kv ? (int)tap : 4, cc = kv ? (int)(k - tap * a.Cin) : (int)a.Cin;   // past K: the zero padding
+        const int ty = (tp >= 3 ? 1 : 0) + (tp >= 6 ? 1 : 0);
+        const uint16_t* const p = abase + ((ty - 1) * (kTileX + 2) + tp - 3 * ty - 1) * (int)cs + cc;
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const int ly = (int)rowbase + m + 1 + dy, lx = (int)r + 1 + dx;
-            A[m] = __builtin_bit_cast(
-                bf16x8, *reinterpret_cast<const u32x4*>(tile + (size_t)(ly * (kTileX + 2) + lx) * cs + cc));
+        for (int m = 0; m < MT; ++m) A[m] = ld8(p + (size_t)m * rstep);
+    };
+    bf16x8 A[2][MT];
+    load_a(0u, A[0]);
+    // two rings per iteration, so that ring and operand buffers have fixed indexes
+    auto ring = [&](uint32_t s0, uint32_t par) {
+#pragma unroll
+        for (uint32_t d = 0; d < kDepth; ++d) {
+            const uint32_t ks = s0 + d, cur = (par + d) & 1u;
+            load_a(ks + 1u, A[cur ^ 1u]);
+            const bool kv = 32u * ks + 8u * g < K;
+#pragma unroll
+            for (int j = 0; j < NG; ++j) {
+                const bf16x8 w = __builtin_bit_cast(bf16x8, kv ? B[d][j] : u32x4{0u, 0u, 0u, 0u});
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+                    acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, A[cur][m], acc[m][j], 0, 0, 0);
+            }
+            fetch(ks + kDepth, B[d]);
         }
-        const uint16_t* bs = bsl + (size_t)cur * (NT * 16u * kBPitch);
-        bf16x8 B[NT];
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-            B[j] = __builtin_bit_cast(
-                bf16x8, *reinterpret_cast<const u32x4*>(bs + ((uint32_t)j * 16u + r) * kBPitch + 8u * g));
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-                acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[j], A[m], acc[m][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        store(cur ^ 1u, nx, nok);
-        __syncthreads();
+    };
+    for (uint32_t s0 = 0;;) {
+        ring(s0, 0u);
+        if ((s0 += kDepth) >= S) break;
+        ring(s0, kDepth & 1u);
+        if ((s0 += kDepth) >= S) break;
     }
     // D layout: lane holds output channels 16j + 4g .. 16j + 4g + 3 of pixel r of its row m.
     // BF16 outputs at 4-channel aligned strides and offsets go out as one 8-byte store per
     // four channels (mask read the same way); otherwise one store per channel
     const int x = tx0 + (int)r;
-    if constexpr (MT == 2 && !OUTF && !MASK) {
+    if constexpr (!OUTF && !MASK) {
         if (a.pool) {
-            float bias[NT][4];
+            float bias[NG][4];
 #pragma unroll
-            for (int j = 0; j < NT; ++j)
+            for (int j = 0; j < NG; ++j)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const uint32_t co = (uint32_t)j * 16u + 4u * g + (uint32_t)i;
+                    const uint32_t co = cobase + (uint32_t)j * 16u + 4u * g + (uint32_t)i;
                     bias[j][i] = (a.bias && co < a.Cout) ? a.bias[co] : 0.0f;
                 }
-            epilogue_pool<NT, RELU>(a, acc, bias, n, x, ty0 + (int)rowbase, g, r);
+            epilogue_pool<NG, RELU>(a, acc, bias, cobase, n, x, ty0 + (int)rowbase, g, r);
             return;
         }
     }
@@ -389,8 +303,8 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(ConvArgs a) {
         if (y >= (int)a.H) continue;
         const size_t p = img + (size_t)y * a.W + (size_t)x;
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const uint32_t co0 = (uint32_t)j * 16u + 4u * g;
+        for (int j = 0; j < NG; ++j) {
+            const uint32_t co0 = cobase + (uint32_t)j * 16u + 4u * g;
             if (co0 >= a.Cout) continue;
             if (vec) {
                 float v[4];
@@ -430,7 +344,7 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(ConvArgs a) {
 // operand reads then start in different banks), and walk the kTileX x (NW MT) pixel tiles of
 // the grid.  The next tile's input is fetched into registers while the current tile is
 // computed, so the K loop reads only LDS and has no barrier; each K step's tap offset comes
-// from a small LDS table.  K chunks, operands and their order are those of k_conv3x3 (steps
+// from a small LDS table.  K chunks, operands and their order are those of k_conv3x3_split (steps
 // past 9 Cin add zero products), so every output is the same sum in the same order.
 template <int MT, int NW>
 constexpr uint32_t res_chunks() {   // 16-B chunks of a halo tile per thread, Cin <= 96 (12 + 1 pad)
@@ -512,7 +426,7 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3_res(ConvArgs a, uint32_t nt
             pre[b] = u32x4{0u, 0u, 0u, 0u};
             if (i < total && c8 + 1u < cpp && y >= 0 && y < (int)a.H && x >= 0 && x < (int)a.W)
                 pre[b] = *reinterpret_cast<const u32x4*>(
-                    (a.up && 8u * c8 < a.up_C)
+                    8u * c8 < a.up_C
                         ? a.up + (((size_t)n * (a.H >> 1) + (size_t)(y >> 1)) * (a.W >> 1) + (size_t)(x >> 1)) * a.up_C +
                               8u * c8
                         : a.in + (img + (size_t)y * a.W + (size_t)x) * a.in_stride + 8u * c8);
@@ -597,7 +511,7 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3_res(ConvArgs a, uint32_t nt
         const int x = tx0 + (int)r;
         if constexpr (MT == 2 && !OUTF && !MASK) {
             if (a.pool) {
-                epilogue_pool<NT, RELU>(a, acc, bias, n, x, ty0 + (int)rowbase, g, r);
+                epilogue_pool<NT, RELU>(a, acc, bias, 0u, n, x, ty0 + (int)rowbase, g, r);
                 continue;
             }
         }
@@ -811,27 +725,6 @@ __global__ __launch_bounds__(256) void k_wgrad_reduce(const float* __restrict__ 
 }
 
 // ---- element-wise kernels (8 channels per thread) ----------------------------------------
-// out (N x h x w x C) = 2x2 mean of in (N x 2h x 2w, stride, off)
-__global__ void k_pool_fwd(const uint16_t* __restrict__ in, uint32_t in_stride, uint32_t in_off,
-                           uint16_t* __restrict__ out, uint32_t N, uint32_t h, uint32_t w, uint32_t C) {
-    const uint32_t c8n = C / 8u;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N * h * w * c8n) return;
-    const uint32_t c8 = i % c8n, q = i / c8n;
-    const uint32_t x = q % w, y = (q / w) % h, n = q / (w * h);
-    const uint32_t W = 2u * w, H = 2u * h;
-    float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (uint32_t d = 0; d < 4; ++d) {
-        const uint32_t p = (n * H + 2u * y + (d >> 1)) * W + 2u * x + (d & 1u);
-        const u32x4 v = *reinterpret_cast<const u32x4*>(in + (size_t)p * in_stride + in_off + c8 * 8u);
-        for (int t = 0; t < 8; ++t) s[t] += bf2f(half16(v, t));
-    }
-    u32x4 o;
-    for (int t = 0; t < 4; ++t)
-        o[t] = (uint32_t)f2bf(0.25f * s[2 * t]) | ((uint32_t)f2bf(0.25f * s[2 * t + 1]) << 16);
-    *reinterpret_cast<u32x4*>(out + (size_t)q * C + c8 * 8u) = o;
-}
-
 // g (N x H x W x C) = (gpool[parent] / 4 + gcat[p, off..]) * (act[p, off..] > 0)
 __global__ void k_pool_bwd(const uint16_t* __restrict__ gpool, const uint16_t* __restrict__ gcat,
                            const uint16_t* __restrict__ act, uint32_t stride, uint32_t off, uint16_t* __restrict__ g,
@@ -1266,22 +1159,6 @@ int ensure_grad(size_t P0) {
 }
 
 // ---- launches ----------------------------------------------------------------------------
-// launches one tiled instantiation; workgroups above 64 KiB of LDS are allowed first (once
-// per instantiation and size)
-template <int MT, int NT, bool RELU, bool OUTF, bool MASK>
-int launch_tile(const ConvArgs& a, dim3 tg, hipStream_t s) {
-    const size_t lds = conv_tile_lds<NT>(MT, a.Cin);
-    static size_t allowed = 65536;
-    if (lds > allowed) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conv3x3_tile<MT, NT, RELU, OUTF, MASK>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-            return -1;
-        allowed = lds;
-    }
-    hipLaunchKernelGGL((k_conv3x3_tile<MT, NT, RELU, OUTF, MASK>), tg, dim3(256), lds, s, a);
-    return 0;
-}
-
 // compute units of the current device (queried once)
 uint32_t device_cus() {
     static int n = 0;
@@ -1315,57 +1192,46 @@ int launch_res(const ConvArgs& a, hipStream_t s) {
     return 0;
 }
 
+// LDS above 64 KiB is allowed first (once per instantiation and size)
 template <bool RELU, bool OUTF, bool MASK>
-int launch_conv_nt(uint32_t nt, const ConvArgs& a, hipStream_t s) {
-    if (a.Cin <= kTileMaxCin && a.Cin % 8u == 0 && a.in_stride % 8u == 0 && nt <= 6) {
-        // resident weights where they fit and the grid has enough tiles, else weight slices
-        int rc = 1;
-        switch (nt) {
-            case 1: rc = launch_res<2, 8, 1, RELU, OUTF, MASK>(a, s); break;
-            case 2: rc = launch_res<2, 8, 2, RELU, OUTF, MASK>(a, s); break;
-            case 3: rc = launch_res<2, 8, 3, RELU, OUTF, MASK>(a, s); break;
-            case 4: rc = launch_res<2, 8, 4, RELU, OUTF, MASK>(a, s); break;
-            case 5: rc = launch_res<2, 8, 5, RELU, OUTF, MASK>(a, s); break;
-            case 6: rc = launch_res<2, 8, 6, RELU, OUTF, MASK>(a, s); break;
-            default: break;
-        }
-        if (rc <= 0) return rc;
-        const dim3 tg((a.W + kTileX - 1) / kTileX, (a.H + 7u) / 8u, a.N);
-        switch (nt) {
-            case 1: return launch_tile<2, 1, RELU, OUTF, MASK>(a, tg, s);
-            case 2: return launch_tile<2, 2, RELU, OUTF, MASK>(a, tg, s);
-            case 3: return launch_tile<2, 3, RELU, OUTF, MASK>(a, tg, s);
-            case 4: return launch_tile<2, 4, RELU, OUTF, MASK>(a, tg, s);
-            case 5: return launch_tile<2, 5, RELU, OUTF, MASK>(a, tg, s);
-            case 6: return launch_tile<2, 6, RELU, OUTF, MASK>(a, tg, s);
-            default: break;
-        }
+int launch_split(const ConvArgs& a, uint32_t groups, hipStream_t s) {
+    const uint32_t ntx = (a.W + kTileX - 1u) / kTileX, nty = (a.H + kTileY - 1u) / kTileY;
+    const size_t lds = conv_split_lds(a.Cin);
+    static size_t allowed = 65536;
+    if (lds > allowed) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conv3x3_split<RELU, OUTF, MASK>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return -1;
+        allowed = lds;
     }
-    const dim3 grid(blocks((size_t)a.N * a.H * a.W, kConvPix)), blk(256);
-    switch (nt) {
-        case 1: hipLaunchKernelGGL((k_conv3x3<1, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((k_conv3x3<2, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 3: hipLaunchKernelGGL((k_conv3x3<3, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 4: hipLaunchKernelGGL((k_conv3x3<4, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 5: hipLaunchKernelGGL((k_conv3x3<5, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 6: hipLaunchKernelGGL((k_conv3x3<6, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 7: hipLaunchKernelGGL((k_conv3x3<7, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 8: hipLaunchKernelGGL((k_conv3x3<8, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 9: hipLaunchKernelGGL((k_conv3x3<9, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 10: hipLaunchKernelGGL((k_conv3x3<10, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 11: hipLaunchKernelGGL((k_conv3x3<11, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        case 12: hipLaunchKernelGGL((k_conv3x3<12, RELU, OUTF, MASK>), grid, blk, 0, s, a); break;
-        default: return -1;
-    }
+    hipLaunchKernelGGL((k_conv3x3_split<RELU, OUTF, MASK>), dim3(ntx * nty * a.N, groups), dim3(256), lds, s, a, ntx,
+                       nty);
     return 0;
 }
 
+// nt: 16-channel groups of the output
+template <bool RELU, bool OUTF, bool MASK>
+int launch_conv_nt(uint32_t nt, const ConvArgs& a, hipStream_t s) {
+    // resident weights where they fit and the grid has enough tiles, else split output channels
+    int rc = 1;
+    switch (nt) {
+        case 1: rc = launch_res<2, 8, 1, RELU, OUTF, MASK>(a, s); break;
+        case 2: rc = launch_res<2, 8, 2, RELU, OUTF, MASK>(a, s); break;
+        case 3: rc = launch_res<2, 8, 3, RELU, OUTF, MASK>(a, s); break;
+        case 4: rc = launch_res<2, 8, 4, RELU, OUTF, MASK>(a, s); break;
+        case 5: rc = launch_res<2, 8, 5, RELU, OUTF, MASK>(a, s); break;
+        case 6: rc = launch_res<2, 8, 6, RELU, OUTF, MASK>(a, s); break;
+        default: break;
+    }
+    if (rc <= 0) return rc;
+    return launch_split<RELU, OUTF, MASK>(a, nt, s);
+}
+
 // forward conv of layer li: in (Cin channels, stride in.C) -> out (stride out_stride, offset out_off)
-// pool (optional, BF16 outputs only): also writes the 2x2 mean pool of the output (N x H/2 x W/2
-// x Cout), fused into the epilogue of the LDS-tiled kernels, else by k_pool_fwd afterwards
-// up (optional): input channels [0, up.C) are the nearest 2x upsampling of `up` (N x H/2 x W/2),
-// read by the LDS-tiled kernels' staging; returns 1 (nothing launched) when the layer does
-// not run on those kernels, so the caller materialises the upsampling instead
+// pool (optional, BF16 outputs only, H and W even): also writes the 2x2 mean pool of the output
+// (N x H/2 x W/2 x Cout), fused into the epilogue
+// up (optional, H and W even): input channels [0, up.C) are the nearest 2x upsampling of `up`
+// (N x H/2 x W/2), read by the kernels' staging
 int conv_fwd(int li, const Tensor& in, void* out, uint32_t out_stride, uint32_t out_off, uint32_t N, uint32_t H,
              uint32_t W, bool outf, hipStream_t s, uint16_t* pool = nullptr, const Tensor* up = nullptr) {
     const Layer& L = net.L[li];
@@ -1380,24 +1246,12 @@ int conv_fwd(int li, const Tensor& in, void* out, uint32_t out_stride, uint32_t 
     a.N = N; a.H = H; a.W = W;
     a.Cin = L.cin;
     a.Cout = L.cout;
+    a.pool = pool;
+    a.up = up ? up->p : in.p;
+    a.up_C = up ? up->C : 0u;
     const uint32_t nt = (L.cout + 15u) / 16u;
-    const bool tiled = a.Cin <= kTileMaxCin && a.Cin % 8u == 0 && a.in_stride % 8u == 0 && nt <= 6;
-    if (up) {
-        if (!tiled || up->C % 8u != 0 || H % 2u != 0 || W % 2u != 0) return 1;
-        a.up = up->p;
-        a.up_C = up->C;
-    }
     if (outf) return launch_conv_nt<false, true, false>(nt, a, s);
-    const bool fuse = pool && a.Cin <= kTileMaxCin && a.Cin % 8u == 0 && a.in_stride % 8u == 0 && nt <= 6 &&
-                      a.Cout % 4u == 0 && a.out_stride % 4u == 0 && a.out_off % 4u == 0 && H % 2u == 0 && W % 2u == 0;
-    a.pool = fuse ? pool : nullptr;
-    const int rc = L.relu ? launch_conv_nt<true, false, false>(nt, a, s) : launch_conv_nt<false, false, false>(nt, a, s);
-    if (rc == 0 && pool && !fuse) {
-        const size_t n8 = (size_t)N * (H / 2) * (W / 2) * (L.cout / 8);
-        hipLaunchKernelGGL(k_pool_fwd, dim3(blocks(n8)), dim3(256), 0, s, static_cast<const uint16_t*>(out), out_stride,
-                           out_off, pool, N, H / 2, W / 2, L.cout);
-    }
-    return rc;
+    return L.relu ? launch_conv_nt<true, false, false>(nt, a, s) : launch_conv_nt<false, false, false>(nt, a, s);
 }
 
 // backward-data of layer li: g (Cout channels, stride g.C, g.C % 8 == 0) -> dX (Cin channels),
@@ -1406,7 +1260,7 @@ int conv_bwd_data(int li, const Tensor& g, const Tensor& dx, const Tensor* mask,
                   hipStream_t s) {
     const Layer& L = net.L[li];
     ConvArgs a{};
-    a.in = g.p;
+    a.in = a.up = g.p;
     a.in_stride = g.C;
     a.w = net.wt + L.d.wt_off;
     a.bias = nullptr;
@@ -1530,12 +1384,9 @@ int forward(uint32_t N, uint32_t H, uint32_t W, hipStream_t s, bool fuse_up = fa
     for (int l = 3; l >= 0 && rc == 0; --l) {
         const uint32_t h = H >> l, w = W >> l;
         const int li = 10 + 2 * (3 - l);
-        int fused = 1;
         if (fuse_up) {
-            fused = conv_fwd(li, net.cat[l], net.d1[l].p, net.d1[l].C, 0, N, h, w, false, s, nullptr, &prev);
-            rc |= fused < 0 ? fused : 0;
-        }
-        if (fused == 1) {
+            rc |= conv_fwd(li, net.cat[l], net.d1[l].p, net.d1[l].C, 0, N, h, w, false, s, nullptr, &prev);
+        } else {
             const size_t n8 = (size_t)N * h * w * (net.U[l] / 8);
             hipLaunchKernelGGL(k_up_fwd, dim3(blocks(n8)), dim3(256), 0, s, prev.p, net.cat[l].p, net.cat[l].C, 0u, N,
                                h, w, net.U[l]);

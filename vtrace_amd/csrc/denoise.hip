@@ -568,11 +568,17 @@ struct WGradArgs {
     uint32_t N, H, W, Cin, Cout;
     uint32_t ntx, nty, tiles;   // kWgX x kWgY pixel tiles: per row, per column, of the batch
     uint32_t tiles_chunk;       // consecutive tiles of one workgroup
+    uint32_t nco, nci;          // 16-channel groups of a workgroup's outputs and inputs
+    uint32_t cob, cib;          // workgroups that share a chunk: per outputs and per inputs
+    uint32_t first;             // its first workgroup in the launch
+};
+struct WGradTable {
+    WGradArgs l[kLayers];
 };
 
 // dW[co][tap][ci] = sum_p dY[p][co] X[p + tap][ci] as a GEMM over pixels: rows co, columns ci, one
-// accumulator tile per tap.  A workgroup takes a chunk of kWgX x kWgY pixel tiles and 16 NCI of the
-// input channels and holds all nine taps' sums of all 16 NCO output channels in registers: wave w
+// accumulator tile per tap.  A workgroup takes a chunk of kWgX x kWgY pixel tiles, 16 NCI of the
+// input channels and 16 NCO of the outputs and holds all nine taps' sums in registers: wave w
 // the taps of row dy = w - 1 (three shifts in x share every dY fragment).  A tile of dY and of X with
 // a one-pixel halo is staged in LDS as it lies in memory (pixel by pixel); ds_read_b64_tr_b16
 // transposes on the way to the registers (16 lanes read 4 pixels x 16 channels, lane i gets channel i
@@ -581,9 +587,7 @@ struct WGradArgs {
 // A K step is 2 rows of 16 pixels: k = 8 g + 4 h + j is the pixel 4 (g & 1) + 8 h + j of row g >> 1,
 // the same for both operands.  LDS pixels lie an odd multiple of 32 B apart, so the 8 pixels that
 // half a wave reads are in different banks.
-// Bound by the matrix pipe and the staging together.  The form before (one tap and 32 input channels
-// per workgroup, the transpose by 2-byte LDS stores, dY read 9 Cin / 32 times) took 4.9 ms of a
-// 14.1 ms fine-tuning call (8 steps of 8 crops of 128 x 128); this one 1.2 ms.
+// Bound by the matrix pipe and the staging together.
 constexpr uint32_t kWgX = 16, kWgY = 4, kWgThreads = 192;
 constexpr uint32_t wg_pitch(uint32_t n16) { return 16u * (n16 | 1u); }
 
@@ -596,19 +600,21 @@ __device__ __forceinline__ bf16x8 ld_tr(const uint16_t* p, uint32_t pitch) {
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// grid (chunks, ceil(Cin / (16 NCI)))
+constexpr uint32_t kWgMaxCo = 3, kWgMaxCi = 2;   // more accumulators leave two waves per SIMD
+constexpr uint32_t kWgLds = kWgX * kWgY * wg_pitch(kWgMaxCo) + (kWgX + 2u) * (kWgY + 2u) * wg_pitch(kWgMaxCi);
+
 template <int NCO, int NCI>
-__global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_conv3x3_wgrad(WGradArgs a) {
+__device__ __forceinline__ void wgrad_block(const WGradArgs& a, uint32_t chunk, uint32_t cib, uint32_t cob, uint16_t* lds) {
     constexpr uint32_t GP = wg_pitch(NCO), XP = wg_pitch(NCI), XW = kWgX + 2u, XH = kWgY + 2u;
     constexpr uint32_t GCH = kWgX * kWgY * 2u * NCO, XCH = XW * XH * 2u * NCI;   // 16-byte chunks of a tile
     constexpr uint32_t GB = (GCH + kWgThreads - 1u) / kWgThreads, XB = (XCH + kWgThreads - 1u) / kWgThreads;
-    __shared__ __align__(16) uint16_t gt[kWgX * kWgY * GP];
-    __shared__ __align__(16) uint16_t xt[XW * XH * XP];
+    uint16_t* const gt = lds;
+    uint16_t* const xt = lds + kWgX * kWgY * GP;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // tap row: dy = wave - 1
-    const uint32_t ci0 = blockIdx.y * 16u * NCI;
+    const uint32_t ci0 = cib * 16u * NCI, co0 = cob * 16u * NCO;
     const uint32_t cout8 = (a.Cout + 7u) & ~7u;
-    const uint32_t t1 = min(a.tiles, (blockIdx.x + 1u) * a.tiles_chunk);
+    const uint32_t t1 = min(a.tiles, (chunk + 1u) * a.tiles_chunk);
     u32x4 gpre[GB], xpre[XB];
     auto fetch = [&](uint32_t t) {
         const uint32_t tx = t % a.ntx, rest = t / a.ntx, ty = rest % a.nty, n = rest / a.nty;
@@ -616,7 +622,7 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2)))
         const size_t img = (size_t)n * a.H * a.W;
 #pragma unroll
         for (uint32_t b = 0; b < GB; ++b) {
-            const uint32_t i = tid + kWgThreads * b, pix = i / (2u * NCO), c = 8u * (i % (2u * NCO));
+            const uint32_t i = tid + kWgThreads * b, pix = i / (2u * NCO), c = co0 + 8u * (i % (2u * NCO));
             const uint32_t x = (uint32_t)x0 + pix % kWgX, y = (uint32_t)y0 + pix / kWgX;
             gpre[b] = u32x4{0u, 0u, 0u, 0u};
             if (i < GCH && c < cout8 && x < a.W && y < a.H)
@@ -636,7 +642,7 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2)))
     const uint32_t col = 4u * (g & 1u) + (r >> 2), row = g >> 1;
     const uint16_t* const gbase = gt + (row * kWgX + col) * GP + 4u * (r & 3u);
     const uint16_t* const xbase = xt + ((row + wave) * XW + col) * XP + 4u * (r & 3u);
-    const bool do_bias = wave == 1u && blockIdx.y == 0u;
+    const bool do_bias = wave == 1u && cib == 0u;
     const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
     f32x4 acc[3][NCI][NCO], bacc[NCO];
 #pragma unroll
@@ -645,7 +651,7 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
         for (int k = 0; k < 3 * NCI; ++k) acc[k / NCI][k % NCI][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    uint32_t t = blockIdx.x * a.tiles_chunk;
+    uint32_t t = chunk * a.tiles_chunk;
     if (t < t1) fetch(t);
     for (; t < t1; ++t) {
         __syncthreads();   // the previous tile is no longer read
@@ -681,14 +687,14 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2)))
                     bacc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[j], ones, bacc[j], 0, 0, 0);
         }
     }
-    // D layout: lane holds output channels 16 j + 4 g + i (rows) at input channel r (column)
+    // D layout: lane holds output channels co0 + 16 j + 4 g + i (rows) at input channel r (column)
     const uint32_t K = 9u * a.Cin;
-    float* const part = a.part + (size_t)blockIdx.x * (a.Cout * K + a.Cout);
+    float* const part = a.part + (size_t)chunk * (a.Cout * K + a.Cout);
 #pragma unroll
     for (int j = 0; j < NCO; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint32_t co = 16u * j + 4u * g + (uint32_t)i;
+            const uint32_t co = co0 + 16u * j + 4u * g + (uint32_t)i;
             if (co >= a.Cout) continue;
 #pragma unroll
             for (int c = 0; c < NCI; ++c) {
@@ -701,27 +707,81 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2)))
         }
 }
 
+// Every layer's weight gradient in one launch at the end of the backward pass: a layer alone has
+// too little work to fill the GPU and to hide its start (19 launches: 175 us a step of 8 crops of 128 x
+// 128, this one 106).  The workgroups that share a chunk are consecutive.
+__global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_conv3x3_wgrad(WGradTable T) {
+    __shared__ __align__(16) uint16_t lds[kWgLds];
+    uint32_t l = 0;
+    while (l + 1u < (uint32_t)kLayers && blockIdx.x >= T.l[l + 1].first) ++l;
+    const WGradArgs& a = T.l[l];
+    const uint32_t b = blockIdx.x - a.first, per = a.cib * a.cob, sub = b % per;
+    const uint32_t chunk = b / per, cib = sub % a.cib, cob = sub / a.cib;
+    switch (a.nco * 4u + a.nci) {
+        case 5: wgrad_block<1, 1>(a, chunk, cib, cob, lds); break;
+        case 6: wgrad_block<1, 2>(a, chunk, cib, cob, lds); break;
+        case 9: wgrad_block<2, 1>(a, chunk, cib, cob, lds); break;
+        case 10: wgrad_block<2, 2>(a, chunk, cib, cob, lds); break;
+        case 13: wgrad_block<3, 1>(a, chunk, cib, cob, lds); break;
+        default: wgrad_block<3, 2>(a, chunk, cib, cob, lds); break;
+    }
+}
+
+struct LayerDev {
+    uint32_t cin, cout, cout8;
+    uint32_t w_off, b_off;     // in the FP32 parameter vector
+    uint32_t wb_off, wt_off;   // BF16 forward weights [co][tap][ci], transposed [ci][8-tap][cout8]
+    uint32_t nw;               // cout * 9 * cin
+};
+// weight i of a layer into its BF16 forward and transposed (tap-flipped) copies
+__device__ __forceinline__ void put_weight(const LayerDev& d, uint32_t i, float w, uint16_t* __restrict__ wb,
+                                           uint16_t* __restrict__ wt) {
+    const uint32_t co = i / (9u * d.cin), rem = i - co * 9u * d.cin;
+    const uint32_t tap = rem / d.cin, ci = rem - tap * d.cin;
+    const uint16_t b = f2bf(w);
+    wb[d.wb_off + i] = b;
+    wt[d.wt_off + (ci * 9u + (8u - tap)) * d.cout8 + co] = b;
+}
+
 // The chunks' partial sums of every layer, added up in chunk order (deterministic): parameter i of
-// layer l is part[off + c * n + i - first] over its chunks c.  One launch for the whole network at
-// the end of the backward pass: a layer alone is too few threads to fill the GPU.
+// layer l is part[off + c * n + i - first] over its chunks c.  One launch for the whole network:
+// a layer alone is too few threads to fill the GPU.  ADAM: the step (Kingma & Ba 2015) on the
+// FP32 master parameters and their BF16 copies in the same pass, else the gradient into `grads`.
 struct PartTable {
     struct {
         uint64_t off;
         uint32_t chunks, n, first;   // n: the layer's weights and biases, from parameter `first`
     } l[kLayers];
 };
+struct AdamArgs {
+    float *w, *m, *v;
+    const LayerDev* layers;
+    uint16_t *wb, *wt;
+    float lr, b1, b2, eps, bc1, bc2;
+};
+template <bool ADAM>
 __global__ __launch_bounds__(256) void k_wgrad_reduce(const float* __restrict__ part, PartTable T, uint32_t nparam,
-                                                      float* __restrict__ grads) {
+                                                      float* __restrict__ grads, AdamArgs o) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= nparam) return;
     uint32_t l = 0;
     while (l + 1u < (uint32_t)kLayers && i >= T.l[l + 1].first) ++l;
-    const uint32_t n = T.l[l].n, chunks = T.l[l].chunks;
-    const float* p = part + T.l[l].off + (i - T.l[l].first);
+    const uint32_t n = T.l[l].n, chunks = T.l[l].chunks, k = i - T.l[l].first;
+    const float* p = part + T.l[l].off + k;
     float s = 0.0f;
 #pragma unroll 8
     for (uint32_t c = 0; c < chunks; ++c) s += p[(size_t)c * n];
-    grads[i] = s;
+    if (!ADAM) {
+        grads[i] = s;
+        return;
+    }
+    const float mi = o.b1 * o.m[i] + (1.0f - o.b1) * s;
+    const float vi = o.b2 * o.v[i] + (1.0f - o.b2) * s * s;
+    o.m[i] = mi;
+    o.v[i] = vi;
+    const float w = o.w[i] - o.lr * (mi / o.bc1) / (sqrtf(vi / o.bc2) + o.eps);
+    o.w[i] = w;
+    if (k < o.layers[l].nw) put_weight(o.layers[l], k, w, o.wb, o.wt);
 }
 
 // ---- element-wise kernels (8 channels per thread) ----------------------------------------
@@ -906,27 +966,6 @@ __global__ __launch_bounds__(256) void k_loss_sum(const float* __restrict__ part
     if (threadIdx.x == 0) *out = red[0] * scale;
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 master parameters
-__global__ void k_adam(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
-                       const float* __restrict__ g, size_t n, float lr, float b1, float b2, float eps, float bc1,
-                       float bc2) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    w[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
-}
-
-struct LayerDev {
-    uint32_t cin, cout, cout8;
-    uint32_t w_off, b_off;     // in the FP32 parameter vector
-    uint32_t wb_off, wt_off;   // BF16 forward weights [co][tap][ci], transposed [ci][8-tap][cout8]
-    uint32_t nw;               // cout * 9 * cin
-};
-
 // FP32 master -> BF16 forward and transposed (tap-flipped) weights of every layer
 __global__ void k_prep_weights(const float* __restrict__ params, const LayerDev* __restrict__ L, uint32_t nl,
                                uint16_t* __restrict__ wb, uint16_t* __restrict__ wt, uint32_t total) {
@@ -937,12 +976,7 @@ __global__ void k_prep_weights(const float* __restrict__ params, const LayerDev*
         i -= L[l].nw;
         ++l;
     }
-    const LayerDev d = L[l];
-    const uint32_t co = i / (9u * d.cin), rem = i - co * 9u * d.cin;
-    const uint32_t tap = rem / d.cin, ci = rem - tap * d.cin;
-    const uint16_t b = f2bf(params[d.w_off + i]);
-    wb[d.wb_off + i] = b;
-    wt[d.wt_off + (ci * 9u + (8u - tap)) * d.cout8 + co] = b;
+    put_weight(L[l], i, params[L[l].w_off + i], wb, wt);
 }
 
 // network output (hp x wp x 3 log-irradiance corrections, FP32) -> h x w RGBA32F radiance
@@ -1009,7 +1043,9 @@ struct Net {
     float* lpart = nullptr;
     float* part = nullptr;
     size_t part_cap = 0;
-    PartTable parts{};         // where each layer's partial sums lie (ensure_part)
+    WGradTable wg{};           // the weight gradients' launch and where its partial sums lie
+    PartTable parts{};         // (plan_wgrad)
+    uint32_t wg_blocks = 0;
     float* losses = nullptr;   // device, one per training iteration
     size_t losses_cap = 0;
     // training frames
@@ -1276,82 +1312,71 @@ int conv_bwd_data(int li, const Tensor& g, const Tensor& dx, const Tensor* mask,
     return mask ? launch_conv_nt<false, false, true>(nt, a, s) : launch_conv_nt<false, false, false>(nt, a, s);
 }
 
-template <int NCO>
-void launch_wgrad(uint32_t nci, const WGradArgs& a, dim3 grid, hipStream_t s) {
-    if (nci == 1) hipLaunchKernelGGL((k_conv3x3_wgrad<NCO, 1>), grid, dim3(kWgThreads), 0, s, a);
-    else hipLaunchKernelGGL((k_conv3x3_wgrad<NCO, 2>), grid, dim3(kWgThreads), 0, s, a);
-}
-
-// How a layer's weight gradient is split: about two workgroups per CU (fewer leave CUs idle, more
-// write and read more partial sums).
-struct WGradPlan {
-    uint32_t nco, nci, cib, ntx, nty, tiles, tiles_chunk, chunks;
-};
-WGradPlan wgrad_plan(const Layer& L, uint32_t N, uint32_t H, uint32_t W) {
-    WGradPlan p;
-    p.nco = (L.cout + 15u) / 16u;
-    p.nci = L.cin <= 16u ? 1u : 2u;
-    p.cib = (L.cin + 16u * p.nci - 1u) / (16u * p.nci);
-    p.ntx = (W + kWgX - 1u) / kWgX;
-    p.nty = (H + kWgY - 1u) / kWgY;
-    p.tiles = N * p.ntx * p.nty;
-    const uint32_t want = std::max(1u, 2u * device_cus() / p.cib);
-    p.tiles_chunk = (p.tiles + want - 1u) / want;
-    p.chunks = (p.tiles + p.tiles_chunk - 1u) / p.tiles_chunk;
-    return p;
-}
 // level of a layer's pixels: 0 at full size, each next one half the width and height
 uint32_t layer_level(int li) { return li < 10 ? (uint32_t)li / 2u : li < 18 ? 3u - (uint32_t)(li - 10) / 2u : 0u; }
 
-// plans and partial sums of every layer for a batch of N x H x W
-int ensure_part(uint32_t N, uint32_t H, uint32_t W) {
-    uint64_t off = 0;
+// How the weight gradients of a batch of N x H x W are split over one launch's workgroups, and where
+// their partial sums lie: about kWgPerCu workgroups per CU in all (as many as are resident: fewer
+// leave CUs idle, more write and read more partial sums), each of about the same work (a tile
+// costs its staging, about as much as 4 blocks of 16 x 16 channels, and its blocks).
+constexpr uint32_t kWgPerCu = 4;
+int plan_wgrad(uint32_t N, uint32_t H, uint32_t W) {
+    uint64_t work = 0;
+    auto cost = [](const WGradArgs& a) { return 4u + a.nco * a.nci; };
     for (int i = 0; i < kLayers; ++i) {
         const Layer& L = net.L[i];
-        const uint32_t lvl = layer_level(i);
-        const WGradPlan p = wgrad_plan(L, N, H >> lvl, W >> lvl);
+        WGradArgs& a = net.wg.l[i];
+        const uint32_t lvl = layer_level(i), co = (L.cout + 15u) / 16u, ci = (L.cin + 15u) / 16u;
+        a.N = N; a.H = H >> lvl; a.W = W >> lvl;
+        a.Cin = L.cin;
+        a.Cout = L.cout;
+        a.cob = (co + kWgMaxCo - 1u) / kWgMaxCo;
+        a.nco = (co + a.cob - 1u) / a.cob;
+        a.nci = std::min(ci, kWgMaxCi);
+        a.cib = (ci + a.nci - 1u) / a.nci;
+        a.ntx = (a.W + kWgX - 1u) / kWgX;
+        a.nty = (a.H + kWgY - 1u) / kWgY;
+        a.tiles = N * a.ntx * a.nty;
+        work += (uint64_t)a.tiles * a.cob * a.cib * cost(a);
+    }
+    const uint64_t share = work / (kWgPerCu * device_cus()) + 1u;   // of one workgroup
+    uint64_t off = 0;
+    uint32_t first = 0;
+    for (int i = 0; i < kLayers; ++i) {
+        const Layer& L = net.L[i];
+        WGradArgs& a = net.wg.l[i];
+        a.tiles_chunk = (uint32_t)std::max<uint64_t>(1u, std::min<uint64_t>(a.tiles, (share + cost(a) - 1u) / cost(a)));
+        const uint32_t chunks = (a.tiles + a.tiles_chunk - 1u) / a.tiles_chunk;
+        a.first = first;
+        first += chunks * a.cob * a.cib;
         net.parts.l[i].off = off;
-        net.parts.l[i].chunks = p.chunks;
+        net.parts.l[i].chunks = chunks;
         net.parts.l[i].n = L.d.nw + L.cout;
         net.parts.l[i].first = L.d.w_off;
-        off += (uint64_t)p.chunks * (L.d.nw + L.cout);
+        off += (uint64_t)chunks * (L.d.nw + L.cout);
     }
-    if (off <= net.part_cap && net.part) return 0;
-    hipFree(net.part);
-    net.part = nullptr;
-    net.part_cap = 0;
-    if (hipMalloc(&net.part, off * 4) != hipSuccess) {
+    net.wg_blocks = first;
+    if (off > net.part_cap || !net.part) {
+        hipFree(net.part);
         net.part = nullptr;
-        return -1;
+        net.part_cap = 0;
+        if (hipMalloc(&net.part, off * 4) != hipSuccess) {
+            net.part = nullptr;
+            return -1;
+        }
+        net.part_cap = off;
     }
-    net.part_cap = off;
+    for (int i = 0; i < kLayers; ++i) net.wg.l[i].part = net.part + net.parts.l[i].off;
     return 0;
 }
 
-int conv_wgrad(int li, const Tensor& x, const Tensor& g, uint32_t N, uint32_t H, uint32_t W, hipStream_t s) {
-    const Layer& L = net.L[li];
-    const WGradPlan p = wgrad_plan(L, N, H, W);
-    WGradArgs a{};
+// the operands of layer li's weight gradient: its input x and its output's gradient g
+void wgrad_of(int li, const Tensor& x, const Tensor& g) {
+    WGradArgs& a = net.wg.l[li];
     a.in = x.p;
     a.in_stride = x.C;
     a.g = g.p;
     a.g_stride = g.C;
-    a.part = net.part + net.parts.l[li].off;
-    a.N = N; a.H = H; a.W = W;
-    a.Cin = L.cin;
-    a.Cout = L.cout;
-    a.ntx = p.ntx; a.nty = p.nty; a.tiles = p.tiles; a.tiles_chunk = p.tiles_chunk;
-    const dim3 grid(p.chunks, p.cib);
-    switch (p.nco) {
-        case 1: launch_wgrad<1>(p.nci, a, grid, s); break;
-        case 2: launch_wgrad<2>(p.nci, a, grid, s); break;
-        case 3: launch_wgrad<3>(p.nci, a, grid, s); break;
-        case 4: launch_wgrad<4>(p.nci, a, grid, s); break;
-        case 5: launch_wgrad<5>(p.nci, a, grid, s); break;
-        case 6: launch_wgrad<6>(p.nci, a, grid, s); break;
-        default: return -1;
-    }
-    return 0;
 }
 
 void prep_weights(hipStream_t s) {
@@ -1399,26 +1424,27 @@ int forward(uint32_t N, uint32_t H, uint32_t W, hipStream_t s, bool fuse_up = fa
     return rc == 0 && hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// loss of net.y against net.target and the backward pass -> net.grads; loss into *loss_dev
-int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, hipStream_t s) {
+// loss of net.y against net.target and the backward pass; loss into *loss_dev.  lr null: gradient
+// -> net.grads, else an Adam step at that rate (parameters and their BF16 copies)
+int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, const float* lr, hipStream_t s) {
     const size_t P0 = (size_t)N * H * W;
     const float scale = 1.0f / (float)(3 * P0);
     const uint32_t lb = blocks(P0);
-    if (ensure_part(N, H, W) != 0) return -1;
+    if (plan_wgrad(N, H, W) != 0) return -1;
     hipLaunchKernelGGL(k_loss, dim3(lb), dim3(256), 0, s, net.y, net.target, net.x0.p, (uint32_t)P0, scale,
                        net.gy.p, net.lpart);
     hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(256), 0, s, net.lpart, lb, scale, loss_dev);
     int rc = 0;
     // output layer
-    rc |= conv_wgrad(18, net.d2[0], net.gy, N, H, W, s);
+    wgrad_of(18, net.d2[0], net.gy);
     rc |= conv_bwd_data(18, net.gy, net.gd2[0], &net.d2[0], N, H, W, s);
     // decoder, level 0 up to 3
     for (int l = 0; l < 4 && rc == 0; ++l) {
         const uint32_t h = H >> l, w = W >> l;
         const int li = 10 + 2 * (3 - l);
-        rc |= conv_wgrad(li + 1, net.d1[l], net.gd2[l], N, h, w, s);
+        wgrad_of(li + 1, net.d1[l], net.gd2[l]);
         rc |= conv_bwd_data(li + 1, net.gd2[l], net.gd1[l], &net.d1[l], N, h, w, s);
-        rc |= conv_wgrad(li, net.cat[l], net.gd1[l], N, h, w, s);
+        wgrad_of(li, net.cat[l], net.gd1[l]);
         rc |= conv_bwd_data(li, net.gd1[l], net.gcat[l], &net.cat[l], N, h, w, s);
         // up part of the concatenation -> gradient of the coarser level's output
         const Tensor& gprev = l < 3 ? net.gd2[l + 1] : net.gb2;
@@ -1428,9 +1454,9 @@ int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, hipStream_t s)
     }
     // bottleneck
     const uint32_t h4 = H >> 4, w4 = W >> 4;
-    rc |= conv_wgrad(9, net.b1, net.gb2, N, h4, w4, s);
+    wgrad_of(9, net.b1, net.gb2);
     rc |= conv_bwd_data(9, net.gb2, net.gb1, &net.b1, N, h4, w4, s);
-    rc |= conv_wgrad(8, net.pool[3], net.gb1, N, h4, w4, s);
+    wgrad_of(8, net.pool[3], net.gb1);
     rc |= conv_bwd_data(8, net.gb1, net.gpool[3], nullptr, N, h4, w4, s);
     // encoder, level 3 down to 0
     for (int l = 3; l >= 0 && rc == 0; --l) {
@@ -1440,25 +1466,27 @@ int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, hipStream_t s)
                            net.cat[l].p, net.cat[l].C, net.U[l], net.gskip[l].p, N, h, w, net.E[l]);
         // enc conv 2: input a[l], output (skip) in cat[l]
         Tensor skip_in = net.a[l];
-        rc |= conv_wgrad(2 * l + 1, skip_in, net.gskip[l], N, h, w, s);
+        wgrad_of(2 * l + 1, skip_in, net.gskip[l]);
         rc |= conv_bwd_data(2 * l + 1, net.gskip[l], net.ga[l], &net.a[l], N, h, w, s);
         // enc conv 1: input pool[l-1] (or x0)
         const Tensor& in = l > 0 ? net.pool[l - 1] : net.x0;
-        rc |= conv_wgrad(2 * l, in, net.ga[l], N, h, w, s);
+        wgrad_of(2 * l, in, net.ga[l]);
         if (l > 0) rc |= conv_bwd_data(2 * l, net.ga[l], net.gpool[l - 1], nullptr, N, h, w, s);
     }
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(blocks(net.nparam)), dim3(256), 0, s, net.part, net.parts,
-                       (uint32_t)net.nparam, net.grads);
+    hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(net.wg_blocks), dim3(kWgThreads), 0, s, net.wg);
+    AdamArgs o{};
+    if (lr) {
+        net.adam_t += 1;
+        const float b1 = 0.9f, b2 = 0.999f;
+        o = AdamArgs{net.params, net.adam_m, net.adam_v, net.ldev, net.wb, net.wt, *lr, b1, b2, 1e-8f,
+                     1.0f - powf(b1, (float)net.adam_t), 1.0f - powf(b2, (float)net.adam_t)};
+        hipLaunchKernelGGL(k_wgrad_reduce<true>, dim3(blocks(net.nparam)), dim3(256), 0, s, net.part, net.parts,
+                           (uint32_t)net.nparam, net.grads, o);
+    } else {
+        hipLaunchKernelGGL(k_wgrad_reduce<false>, dim3(blocks(net.nparam)), dim3(256), 0, s, net.part, net.parts,
+                           (uint32_t)net.nparam, net.grads, o);
+    }
     return rc == 0 && hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-void adam_step(float lr, hipStream_t s) {
-    net.adam_t += 1;
-    const float b1 = 0.9f, b2 = 0.999f;
-    const float bc1 = 1.0f - powf(b1, (float)net.adam_t), bc2 = 1.0f - powf(b2, (float)net.adam_t);
-    hipLaunchKernelGGL(k_adam, dim3(blocks(net.nparam)), dim3(256), 0, s, net.params, net.adam_m, net.adam_v,
-                       net.grads, net.nparam, lr, b1, b2, 1e-8f, bc1, bc2);
-    net.weights_dirty = true;
 }
 
 int ensure_io(size_t bytes) {
@@ -1641,7 +1669,7 @@ int32_t vt_dn_grad(const float* x, const float* target, uint32_t n, uint32_t h, 
     hipLaunchKernelGGL(k_f32_to_bf16, dim3(blocks(P0 * kInCh)), dim3(256), 0, s, static_cast<const float*>(net.io),
                        net.x0.p, P0 * kInCh);
     hipMemcpyAsync(net.target, target, P0 * 3 * 4, hipMemcpyHostToDevice, s);
-    if (forward(n, h, w, s) != 0 || backward(n, h, w, net.losses, s) != 0) {
+    if (forward(n, h, w, s) != 0 || backward(n, h, w, net.losses, nullptr, s) != 0) {
         vt_rt_set_error("vt_dn_grad: launch failed");
         return -1;
     }
@@ -1782,15 +1810,14 @@ int32_t vt_dn_train(uint32_t iters, uint32_t batch, uint32_t crop, float lr, uin
     for (uint32_t it = 0; it < iters; ++it) {
         hipLaunchKernelGGL(k_gather_crops, dim3(blocks(P0)), dim3(256), 0, s, net.frames_dev,
                            net.crops_dev + (size_t)it * batch, batch, crop, net.x0.p, net.target);
-        if (forward(batch, crop, crop, s) != 0 || backward(batch, crop, crop, net.losses + it, s) != 0) {
-            vt_rt_set_error("vt_dn_train: launch failed");
-            return -1;
-        }
         // linear warm-up, then cosine decay to 5% of lr
         const float t = (float)it / (float)iters;
         float lr_t = lr * (0.05f + 0.95f * 0.5f * (1.0f + cosf(3.14159265f * t)));
         if (it < warm) lr_t *= (float)(it + 1) / (float)warm;
-        adam_step(lr_t, s);
+        if (forward(batch, crop, crop, s) != 0 || backward(batch, crop, crop, net.losses + it, &lr_t, s) != 0) {
+            vt_rt_set_error("vt_dn_train: launch failed");
+            return -1;
+        }
     }
     if (losses) hipMemcpyAsync(losses, net.losses, (size_t)iters * 4, hipMemcpyDeviceToHost, s);
     return hipStreamSynchronize(s) == hipSuccess ? 0 : -1;

@@ -87,56 +87,70 @@ struct ConvArgs {
     uint32_t N, H, W, Cin, Cout;
 };
 
-// Epilogue of the LDS-tiled kernels (waves of two 16-pixel rows, weights as the first MFMA
-// operand: a lane holds channels cobase + 16j + 4g .. + 3 of pixel r of rows m = 0, 1) for a
-// layer whose BF16 output is also pooled (a.pool; H and W even, 4-aligned strides and
-// offset).  Rows m = 0, 1 are an even/odd row pair (tile origins are multiples of 8) and lanes
-// r, r ^ 1 an even/odd column pair, so the pooled value comes from this lane and its
-// neighbour: the four BF16 outputs summed in row-major order,
-// times 0.25, rounded to BF16.  Every lane reaches the shuffles; only stores are guarded.
-template <int NT, bool RELU>
-__device__ __forceinline__ void epilogue_pool(const ConvArgs& a, const f32x4 (&acc)[2][NT], const float (&bias)[NT][4],
-                                              uint32_t cobase, uint32_t n, int x, int y0, uint32_t g, uint32_t r) {
-    const bool xin = x < (int)a.W, yin = y0 < (int)a.H;
-    const size_t img = (size_t)n * a.H * a.W;
-    const uint32_t hw = a.W / 2u;
-    const size_t q = ((size_t)n * (a.H / 2u) + (size_t)(y0 >> 1)) * hw + (size_t)(x >> 1);
+// The 2x2 mean pool of a layer whose output is also pooled (a.pool; H and W even): o0, o1 are the
+// BF16 outputs of this lane's pixels (x, y0) and (x, y0 + 1), y0 even, and lanes r, r ^ 1 an even/odd
+// column pair, so the pooled value comes from this lane and its neighbour: the four outputs
+// summed in row-major order, times 0.25, rounded to BF16.  Every lane reaches the shuffles.
+__device__ __forceinline__ void put_pool(const ConvArgs& a, const uint2& o0, const uint2& o1, uint32_t co0, uint32_t n,
+                                         int x, int y0, uint32_t r, bool in) {
+    const uint32_t own[2][2] = {{o0.x, o0.y}, {o1.x, o1.y}};
+    uint32_t nb[2][2];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const uint32_t co0 = cobase + (uint32_t)j * 16u + 4u * g;
-        const bool cin = co0 < a.Cout;
-        uint32_t pk[2][2];
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            float v[4];
+        for (int t = 0; t < 2; ++t) nb[m][t] = (uint32_t)__shfl_xor((int)own[m][t], 1, 64);
+    if ((r & 1u) != 0u || !in) return;
+    float o[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                v[i] = acc[m][j][i] + bias[j][i];
-                if (RELU) v[i] = v[i] > 0.0f ? v[i] : 0.0f;
-            }
-            pk[m][0] = pk2bf(v[0], v[1]);
-            pk[m][1] = pk2bf(v[2], v[3]);
-            if (xin && yin && cin) {
-                const size_t p = img + (size_t)(y0 + m) * a.W + (size_t)x;
-                *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + p * a.out_stride + a.out_off + co0) =
-                    make_uint2(pk[m][0], pk[m][1]);
-            }
+    for (int i = 0; i < 4; ++i) {
+        const int t = i >> 1, sh = 16 * (i & 1);
+        const float s = ((bf2f(own[0][t] >> sh) + bf2f(nb[0][t] >> sh)) + bf2f(own[1][t] >> sh)) + bf2f(nb[1][t] >> sh);
+        o[i] = 0.25f * s;
+    }
+    const size_t q = ((size_t)n * (a.H / 2u) + (size_t)(y0 >> 1)) * (a.W / 2u) + (size_t)(x >> 1);
+    *reinterpret_cast<uint2*>(a.pool + q * a.Cout + co0) = make_uint2(pk2bf(o[0], o[1]), pk2bf(o[2], o[3]));
+}
+
+// Epilogue of the convolutions for a wave's ROWS rows of 16 pixels from (tx0, y0), y0 even: a lane holds
+// output channels co0 .. co0 + 3 of pixel r of each row (weights are the first MFMA operand).  BF16
+// outputs (widths and strides are multiples of 8) go out as one 8-byte store, the mask read the
+// same way; FP32 ones channel by channel.  A row's address is wave-uniform and a lane's place in it
+// the same for every tile, so no vector instruction goes into addresses.
+template <int ROWS, bool RELU, bool OUTF, bool MASK>
+__device__ __forceinline__ void put_rows(const ConvArgs& a, const f32x4 (&acc)[ROWS], const float (&bias)[4], uint32_t co0,
+                                         uint32_t n, int tx0, int y0, uint32_t r) {
+    const bool in_x = tx0 + (int)r < (int)a.W && co0 < a.Cout;
+    const uint32_t at = r * a.out_stride + co0, at_mask = r * a.mask_stride + co0;
+    uint2 o[2] = {make_uint2(0u, 0u), make_uint2(0u, 0u)};
+#pragma unroll
+    for (int m = 0; m < ROWS; ++m) {
+        const int y = y0 + m;
+        if (y >= (int)a.H) break;   // (uniform)
+        const size_t p = ((size_t)n * a.H + (size_t)y) * a.W + (size_t)tx0;
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = acc[m][i] + bias[i];
+            if (RELU) v[i] = v[i] > 0.0f ? v[i] : 0.0f;
         }
-        uint32_t nb[2][2];
+        if constexpr (OUTF) {
+            float* const row = reinterpret_cast<float*>(a.out) + p * a.out_stride + a.out_off;
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) nb[m][t] = (uint32_t)__shfl_xor((int)pk[m][t], 1, 64);
-        if ((r & 1u) == 0u && xin && yin && cin) {
-            float o[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = i >> 1, sh = 16 * (i & 1);
-                const float s = ((bf2f(pk[0][t] >> sh) + bf2f(nb[0][t] >> sh)) + bf2f(pk[1][t] >> sh)) +
-                                bf2f(nb[1][t] >> sh);
-                o[i] = 0.25f * s;
+            for (uint32_t i = 0; i < 4u; ++i)
+                if (in_x && co0 + i < a.Cout) row[at + i] = v[i];
+        } else {
+            if (MASK && in_x) {
+                const uint2 mk = *reinterpret_cast<const uint2*>(a.mask + p * a.mask_stride + at_mask);
+                if (!(bf2f(mk.x) > 0.0f)) v[0] = 0.0f;
+                if (!(bf2f(mk.x >> 16) > 0.0f)) v[1] = 0.0f;
+                if (!(bf2f(mk.y) > 0.0f)) v[2] = 0.0f;
+                if (!(bf2f(mk.y >> 16) > 0.0f)) v[3] = 0.0f;
             }
-            *reinterpret_cast<uint2*>(a.pool + q * a.Cout + co0) = make_uint2(pk2bf(o[0], o[1]), pk2bf(o[2], o[3]));
+            o[m & 1] = make_uint2(pk2bf(v[0], v[1]), pk2bf(v[2], v[3]));
+            if (in_x) *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + p * a.out_stride + a.out_off + at) = o[m & 1];
+            if constexpr (!MASK) {
+                if ((m & 1) && a.pool) put_pool(a, o[0], o[1], co0, n, tx0 + (int)r, y - 1, r, in_x);
+            }
         }
     }
 }
@@ -166,34 +180,28 @@ __device__ __forceinline__ u32x4 halo_chunk(const ConvArgs& a, uint32_t n, int y
 // us, the lower levels of a 720p inference 170 -> 122 us.  Two groups of channels per wave were no
 // faster anywhere (218 and 126 us).
 constexpr int kTileX = 16, kTileY = 8;
-constexpr uint32_t kResMaxCin = 96;
 constexpr uint32_t kDepth = 9;
 
 inline size_t conv_split_lds(uint32_t cin) { return (size_t)(kTileY + 2) * (kTileX + 2) * (cin + 8u) * 2u; }
 
 template <bool RELU, bool OUTF, bool MASK>
 __global__ __launch_bounds__(256) void k_conv3x3_split(ConvArgs a, uint32_t ntx, uint32_t nty) {
-    constexpr int MT = 2, NG = 1;   // rows of pixels, 16-channel groups of a wave
+    constexpr int MT = 2;   // rows of pixels of a wave
     extern __shared__ __align__(16) uint16_t tile[];  // (kTileY + 2) x (kTileX + 2) pixels x cs
     const uint32_t cs = a.Cin + 8u;                   // LDS pixel stride (16 B of padding)
     const uint32_t tx = blockIdx.x % ntx, rest = blockIdx.x / ntx, n = rest / nty;
     const int tx0 = (int)tx * kTileX, ty0 = (int)(rest % nty) * kTileY;
-    const uint32_t cobase = blockIdx.y * 16u * NG;
-    const size_t img = (size_t)n * a.H * a.W;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t cobase = blockIdx.y * 16u;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t g = lane >> 4, r = lane & 15u;
     const uint32_t K = 9u * a.Cin;
     const uint32_t S = (K + 32u * kDepth - 1u) / (32u * kDepth) * kDepth;   // K steps, whole rings
-    // this lane's weight rows (those past Cout repeat the last: outputs nobody stores)
-    const uint16_t* wrow[NG];
-#pragma unroll
-    for (int j = 0; j < NG; ++j) wrow[j] = a.w + (size_t)min(cobase + 16u * j + r, a.Cout - 1u) * K;
-    u32x4 B[kDepth][NG];
+    // this lane's weight row (past Cout the last again: outputs nobody stores)
+    const uint16_t* const wrow = a.w + (size_t)min(cobase + r, a.Cout - 1u) * K;
+    u32x4 B[kDepth];
     // (past 9 Cin a clamped address; the zeros are selected where the fragment is used)
-    auto fetch = [&](uint32_t ks, u32x4 (&dst)[NG]) {
-        const uint32_t k = min(32u * ks + 8u * g, K - 8u);
-#pragma unroll
-        for (int j = 0; j < NG; ++j) dst[j] = *reinterpret_cast<const u32x4*>(wrow[j] + k);
+    auto fetch = [&](uint32_t ks, u32x4& dst) {
+        dst = *reinterpret_cast<const u32x4*>(wrow + min(32u * ks + 8u * g, K - 8u));
     };
     // cpp + 1 chunks of 16 B per pixel: its channels, then its padding, set to zeros (K past
     // the end reads the padding, so no select is needed)
@@ -230,11 +238,9 @@ __global__ __launch_bounds__(256) void k_conv3x3_split(ConvArgs a, uint32_t ntx,
     stage(0u, true);
     for (uint32_t i0 = 256u * kBatch; i0 < total; i0 += 256u * kBatch) stage(i0, false);
     __syncthreads();
-    f32x4 acc[MT][NG];
+    f32x4 acc[MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int j = 0; j < NG; ++j) acc[m][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     // k = 32 s + 8 g as (tap, channel): tap = (k * invc) >> 20, exact while k < 2^20 / Cin
     // (k < 9 Cin + 32 kDepth <= 2016)
     const uint32_t invc = ((1u << 20) + a.Cin - 1u) / a.Cin;
@@ -260,13 +266,9 @@ __global__ __launch_bounds__(256) void k_conv3x3_split(ConvArgs a, uint32_t ntx,
             const uint32_t ks = s0 + d, cur = (par + d) & 1u;
             load_a(ks + 1u, A[cur ^ 1u]);
             const bool kv = 32u * ks + 8u * g < K;
+            const bf16x8 w = __builtin_bit_cast(bf16x8, kv ? B[d] : u32x4{0u, 0u, 0u, 0u});
 #pragma unroll
-            for (int j = 0; j < NG; ++j) {
-                const bf16x8 w = __builtin_bit_cast(bf16x8, kv ? B[d][j] : u32x4{0u, 0u, 0u, 0u});
-#pragma unroll
-                for (int m = 0; m < MT; ++m)
-                    acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, A[cur][m], acc[m][j], 0, 0, 0);
-            }
+            for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, A[cur][m], acc[m], 0, 0, 0);
             fetch(ks + kDepth, B[d]);
         }
     };
@@ -276,286 +278,203 @@ __global__ __launch_bounds__(256) void k_conv3x3_split(ConvArgs a, uint32_t ntx,
         ring(s0, kDepth & 1u);
         if ((s0 += kDepth) >= S) break;
     }
-    // D layout: lane holds output channels 16j + 4g .. 16j + 4g + 3 of pixel r of its row m.
-    // BF16 outputs at 4-channel aligned strides and offsets go out as one 8-byte store per
-    // four channels (mask read the same way); otherwise one store per channel
-    const int x = tx0 + (int)r;
-    if constexpr (!OUTF && !MASK) {
-        if (a.pool) {
-            float bias[NG][4];
+    const uint32_t co0 = cobase + 4u * g;
+    float bias[4];
 #pragma unroll
-            for (int j = 0; j < NG; ++j)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t co = cobase + (uint32_t)j * 16u + 4u * g + (uint32_t)i;
-                    bias[j][i] = (a.bias && co < a.Cout) ? a.bias[co] : 0.0f;
-                }
-            epilogue_pool<NG, RELU>(a, acc, bias, cobase, n, x, ty0 + (int)rowbase, g, r);
-            return;
-        }
-    }
-    if (x >= (int)a.W) return;
-    const bool vec = !OUTF && a.Cout % 4u == 0 && a.out_stride % 4u == 0 && a.out_off % 4u == 0 &&
-                     (!MASK || a.mask_stride % 4u == 0);
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int y = ty0 + (int)rowbase + m;
-        if (y >= (int)a.H) continue;
-        const size_t p = img + (size_t)y * a.W + (size_t)x;
-#pragma unroll
-        for (int j = 0; j < NG; ++j) {
-            const uint32_t co0 = cobase + (uint32_t)j * 16u + 4u * g;
-            if (co0 >= a.Cout) continue;
-            if (vec) {
-                float v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    v[i] = acc[m][j][i] + (a.bias ? a.bias[co0 + i] : 0.0f);
-                    if (RELU) v[i] = v[i] > 0.0f ? v[i] : 0.0f;
-                }
-                if (MASK) {
-                    const uint2 mk = *reinterpret_cast<const uint2*>(a.mask + p * a.mask_stride + co0);
-                    if (!(bf2f(mk.x) > 0.0f)) v[0] = 0.0f;
-                    if (!(bf2f(mk.x >> 16) > 0.0f)) v[1] = 0.0f;
-                    if (!(bf2f(mk.y) > 0.0f)) v[2] = 0.0f;
-                    if (!(bf2f(mk.y >> 16) > 0.0f)) v[3] = 0.0f;
-                }
-                *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + p * a.out_stride + a.out_off + co0) =
-                    make_uint2(pk2bf(v[0], v[1]), pk2bf(v[2], v[3]));
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t co = co0 + (uint32_t)i;
-                    if (co >= a.Cout) continue;
-                    float v = acc[m][j][i] + (a.bias ? a.bias[co] : 0.0f);
-                    if (RELU) v = v > 0.0f ? v : 0.0f;
-                    if (MASK && !(bf2f(a.mask[p * a.mask_stride + co]) > 0.0f)) v = 0.0f;
-                    if (OUTF) reinterpret_cast<float*>(a.out)[p * a.out_stride + a.out_off + co] = v;
-                    else reinterpret_cast<uint16_t*>(a.out)[p * a.out_stride + a.out_off + co] = f2bf(v);
-                }
-            }
-        }
-    }
+    for (uint32_t i = 0; i < 4u; ++i) bias[i] = (a.bias && co0 + i < a.Cout) ? a.bias[co0 + i] : 0.0f;
+    put_rows<MT, RELU, OUTF, MASK>(a, acc, bias, co0, n, tx0, ty0 + (int)rowbase, r);
 }
 
-// Resident-weight form for layers whose weights fit in LDS next to one input tile: persistent
-// workgroups of NW waves load the layer's weights into LDS once, as rows of KP = 9 Cin rounded
-// up to 64 (zeros past Cout and past 9 Cin) at a pitch of KP + 8 elements (the 16 rows one
-// operand reads then start in different banks), and walk the kTileX x (NW MT) pixel tiles of
-// the grid.  The next tile's input is fetched into registers while the current tile is
-// computed, so the K loop reads only LDS and has no barrier; each K step's tap offset comes
-// from a small LDS table.  K chunks, operands and their order are those of k_conv3x3_split (steps
-// past 9 Cin add zero products), so every output is the same sum in the same order.
-template <int MT, int NW>
-constexpr uint32_t res_chunks() {   // 16-B chunks of a halo tile per thread, Cin <= 96 (12 + 1 pad)
-    return ((uint32_t)(NW * MT + 2) * (kTileX + 2) * 13u + 64u * NW - 1u) / (64u * NW);
-}
-inline uint32_t res_kp(uint32_t cin) { return (9u * cin + 63u) & ~63u; }
-template <int NT>
-inline size_t conv_res_lds(int rows, uint32_t cin) {
-    return ((size_t)NT * 16u * (res_kp(cin) + 8u) + (size_t)(rows + 2) * (kTileX + 2) * (cin + 8u)) * 2u +
-           4u * (res_kp(cin) / 32u + 2u) * 4u;
-}
+// Resident-weight form for the layers with tiles enough for every CU: persistent workgroups walk the
+// kTileX x res_y pixel tiles, each wave with the weights of 16 output channels in registers and ROWS
+// rows of 16 pixels, so the only operand it reads from LDS is the input.  Tiles with their halo are
+// double-buffered in LDS, the next one fetched into registers while the current one is computed: one
+// barrier a tile.
+// K is walked in steps of 32 as in the split form: k = tap CI + channel, 9 CI rounded up to whole steps
+// (CI: the input channels; a multiple of 16, fewer are padded with zeros), so every output is the same
+// sum in the same order there and here.  A pixel's neighbours in x follow it in LDS, so the 32 values
+// of a step that lies within one row of taps are at one offset for all of a row's pixels (CI an odd
+// multiple of 16: the second half of a step may lie in the next pixel, beyond its padding), and a
+// fragment read once feeds the steps of up to three output rows: ROWS + 2 reads for 3 ROWS MFMAs where
+// CI is a multiple of 32.  Otherwise steps of the middle row of taps start half a step off (reads of
+// their own), one step holds the end of the first row of taps and the start of the second, and
+// the last one ends in the padding.
+// Bound by the LDS reads and MFMAs where there are many channels (64 -> 64 at 1088 x 1920: 154 GFLOP and 535
+// MB in 141 us, 1.1 PFLOP/s and 3.8 TB/s; 80 -> 64: 223 us), by HBM where there are few (32 -> 32: 38 GFLOP and
+// 268 MB in 50 us).  The form before kept the weights in LDS and read (2 + Cout / 16) operands for
+// every 2 Cout / 16 MFMAs, more LDS time than MFMA time: 241, 291 and 112 us, and 64 -> 3 122 us (now 74).
+// Rows of a tile: 8, so that two workgroups or more share a CU and one's epilogue runs beside
+// another's MFMAs (64 -> 64 channels at 1088 x 1920 161 -> 148 us against 16 rows); 16 for 80 and 96 output
+// channels, whose five or six waves would leave SIMDs uneven (64 -> 80 channels of 8 images of 128 x
+// 128 27 -> 38 us with 8 rows).
+constexpr int res_y(int nt) { return nt <= 4 ? 8 : 16; }
+constexpr uint32_t res_pix(int nt) { return (uint32_t)(res_y(nt) + 2) * (kTileX + 2); }
+constexpr uint32_t res_waves(int nt) { return nt <= 2 ? 4u : nt == 3 ? 6u : nt == 4 ? 4u : 2u * (uint32_t)nt; }
+// waves per SIMD the registers are cut for, and the workgroups per CU they allow
+constexpr uint32_t res_simd(int nt, int ci) { return ci <= 32 ? 4u : (nt == 3 && ci <= 64) || nt >= 5 ? 3u : 2u; }
+constexpr uint32_t res_per_cu(int nt, int ci) { return 4u * res_simd(nt, ci) / res_waves(nt); }
+constexpr size_t res_lds(int nt, int ci) { return 2u * res_pix(nt) * ((uint32_t)ci + 8u) * 2u; }
 
-template <int MT, int NW, int NT, bool RELU, bool OUTF, bool MASK>
-__global__ __launch_bounds__(64 * NW) void k_conv3x3_res(ConvArgs a, uint32_t ntx, uint32_t nty, uint32_t ntiles) {
-    constexpr int TY = NW * MT;
-    constexpr uint32_t kThreads = 64u * NW;
-    constexpr uint32_t kPix = (uint32_t)(TY + 2) * (kTileX + 2);
-    constexpr uint32_t kCh = res_chunks<MT, NW>();
-    extern __shared__ __align__(16) uint16_t lds[];
-    const uint32_t K = 9u * a.Cin, KP = (K + 63u) & ~63u, WP = KP + 8u, KS = KP / 32u;
-    uint16_t* const wl = lds;                                  // NT*16 rows x WP
-    uint16_t* const tile = lds + (size_t)NT * 16u * WP;        // kPix pixels x cs
-    const uint32_t cs = a.Cin + 8u;
-    uint32_t* const offs = reinterpret_cast<uint32_t*>(tile + (size_t)kPix * cs);   // KS x 4 tap offsets
-    const uint32_t tid = threadIdx.x;
-    // weights -> LDS in batches of 8 pieces of 16 B per thread (row = piece / kq by a
-    // multiply-high with ceil(2^32 / kq), exact for these sizes)
-    {
-        const uint32_t kq = KP / 8u, np = (uint32_t)NT * 16u * kq;
-        const uint32_t magic = (uint32_t)(((1ull << 32) + kq - 1u) / kq);
-        for (uint32_t i0 = 0; i0 < np; i0 += kThreads * 8u) {
-            u32x4 v[8];
-#pragma unroll
-            for (uint32_t b = 0; b < 8u; ++b) {
-                const uint32_t i = i0 + tid + kThreads * b;
-                const uint32_t row = __umulhi(i, magic), kk = 8u * (i - row * kq);
-                v[b] = u32x4{0u, 0u, 0u, 0u};
-                if (i < np && row < a.Cout && kk < K) v[b] = *reinterpret_cast<const u32x4*>(a.w + (size_t)row * K + kk);
-            }
-#pragma unroll
-            for (uint32_t b = 0; b < 8u; ++b) {
-                const uint32_t i = i0 + tid + kThreads * b;
-                const uint32_t row = __umulhi(i, magic), kk = 8u * (i - row * kq);
-                if (i < np) *reinterpret_cast<u32x4*>(wl + (size_t)row * WP + kk) = v[b];
-            }
-        }
-    }
-    // tap offsets: entry 4 s + g is the tile offset (elements) of k = 32 s + 8 g relative to the
-    // centre tap's pixel; past 9 Cin (and for the two steps after the last, which the pipelined
-    // loop reads ahead) it points at the centre pixel's zero padding
-    if (tid < 4u * (KS + 2u)) {
-        const uint32_t k = 8u * tid;
-        const uint32_t tap = k / a.Cin;
-        const bool kv = tap < 9u;
-        const int dy = kv ? (int)(tap / 3u) - 1 : 0, dx = kv ? (int)(tap % 3u) - 1 : 0;
-        offs[tid] = (uint32_t)((dy * (kTileX + 2) + dx) * (int)cs) + (kv ? k - tap * a.Cin : a.Cin);
-    }
-    // input tiles: cpp = Cin / 8 + 1 chunks per pixel (channels, then the zero padding); chunk
-    // i -> pixel (i * inv) >> 20, exact for i < 2^20 / 13
-    const uint32_t cpp = a.Cin / 8u + 1u, total = kPix * cpp;
+template <int NT, int CI, bool RELU, bool OUTF, bool MASK>
+__global__ __launch_bounds__(64 * res_waves(NT)) __attribute__((amdgpu_waves_per_eu(res_simd(NT, CI)))) void k_conv3x3_res(
+    ConvArgs a, uint32_t ntx, uint32_t nty, uint32_t ntiles) {
+    constexpr uint32_t kWaves = res_waves(NT), kThreads = 64u * kWaves, kResPix = res_pix(NT);
+    constexpr int kResY = res_y(NT), ROWS = kResY * NT / (int)kWaves;
+    constexpr int cs = CI + 8;                             // LDS pixel stride (16 B of padding, zeros)
+    constexpr uint32_t kCh = (kResPix * (CI / 8u) + kThreads - 1u) / kThreads;
+    constexpr int kRow = 3 * CI, KS = (9 * CI + 31) / 32;   // K values of a row of taps, K steps
+    extern __shared__ __align__(16) uint16_t lds[];        // 2 x kResPix pixels x cs
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, g = lane >> 4, r = lane & 15u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t co16 = 16u * (wave % NT), rowbase = ROWS * (wave / NT);
+    for (uint32_t i = tid; i < 2u * kResPix * (cs / 8u); i += kThreads)
+        *reinterpret_cast<u32x4*>(lds + 8u * i) = u32x4{0u, 0u, 0u, 0u};
+    // input tiles: cpp chunks of 16 B per pixel; chunk i -> pixel (i * inv) >> 20, exact for i < 2^20 / 12
+    const uint32_t cpp = a.Cin / 8u, total = kResPix * cpp;
     const uint32_t inv = ((1u << 20) + cpp - 1u) / cpp;
     u32x4 pre[kCh];
+    uint32_t keep = 0;   // bit b: pre[b] lies in the image (else zeros)
+    // this thread's chunks: byte offsets from the tile's first halo pixel, in the tensor they come from
+    // (where registers are left for them: 64 -> 64 channels at 1088 x 1920 148 -> 138 us, 80 -> 64 223 -> 243)
+    constexpr bool kOff = CI <= 64 && NT <= 4;
+    uint32_t voff[kCh], from_up = 0;
+#pragma unroll
+    for (uint32_t b = 0; b < kCh && kOff; ++b) {
+        const uint32_t i = min(tid + kThreads * b, total - 1u), pix = (i * inv) >> 20, c = 8u * (i - pix * cpp);
+        const uint32_t ly = pix / (uint32_t)(kTileX + 2), lx = pix % (uint32_t)(kTileX + 2);
+        const bool up = c < a.up_C;
+        voff[b] = 2u * (up ? (((ly + 1u) >> 1) * (a.W >> 1) + ((lx + 1u) >> 1)) * a.up_C + c : (ly * a.W + lx) * a.in_stride + c);
+        from_up |= up ? 1u << b : 0u;
+    }
     auto origin = [&](uint32_t t, uint32_t& n, int& tx0, int& ty0) {
         const uint32_t tx = t % ntx, rest = t / ntx;
         tx0 = (int)(tx * (uint32_t)kTileX);
-        ty0 = (int)((rest % nty) * (uint32_t)TY);
+        ty0 = (int)((rest % nty) * (uint32_t)kResY);
         n = rest / nty;
     };
     auto fetch_tile = [&](uint32_t t) {
         uint32_t n;
         int tx0, ty0;
         origin(t, n, tx0, ty0);
-        const size_t img = (size_t)n * a.H * a.W;
+        if (kOff && tx0 > 0 && ty0 > 0 && tx0 + kTileX < (int)a.W && ty0 + kResY < (int)a.H) {   // the halo lies inside
+            const char* const pi = reinterpret_cast<const char*>(
+                a.in + (((size_t)n * a.H + (size_t)(ty0 - 1)) * a.W + (size_t)(tx0 - 1)) * a.in_stride);
+            const char* const pu = reinterpret_cast<const char*>(
+                a.up + (((size_t)n * (a.H >> 1) + (size_t)(ty0 / 2 - 1)) * (a.W >> 1) + (size_t)(tx0 / 2 - 1)) * a.up_C);
+            keep = ~0u;
+            if (a.up_C == 0u) {
+#pragma unroll
+                for (uint32_t b = 0; b < kCh; ++b) pre[b] = *reinterpret_cast<const u32x4*>(pi + voff[b]);
+            } else {
+#pragma unroll
+                for (uint32_t b = 0; b < kCh; ++b)
+                    pre[b] = *reinterpret_cast<const u32x4*>(((from_up >> b & 1u) ? pu : pi) + voff[b]);
+            }
+            return;
+        }
+        keep = 0u;
+#pragma unroll
+        for (uint32_t b = 0; b < kCh; ++b) {
+            const uint32_t i = min(tid + kThreads * b, total - 1u);
+            const uint32_t pix = (i * inv) >> 20;
+            bool ok = true;
+            pre[b] = halo_chunk(a, n, ty0 + (int)(pix / (uint32_t)(kTileX + 2)) - 1, tx0 + (int)(pix % (uint32_t)(kTileX + 2)) - 1,
+                                8u * (i - pix * cpp), ok);
+            keep |= ok ? 1u << b : 0u;
+        }
+    };
+    auto store_tile = [&](uint16_t* tile) {
 #pragma unroll
         for (uint32_t b = 0; b < kCh; ++b) {
             const uint32_t i = tid + kThreads * b;
             const uint32_t pix = (i * inv) >> 20, c8 = i - pix * cpp;
-            const int y = ty0 + (int)(pix / (uint32_t)(kTileX + 2)) - 1, x = tx0 + (int)(pix % (uint32_t)(kTileX + 2)) - 1;
-            pre[b] = u32x4{0u, 0u, 0u, 0u};
-            if (i < total && c8 + 1u < cpp && y >= 0 && y < (int)a.H && x >= 0 && x < (int)a.W)
-                pre[b] = *reinterpret_cast<const u32x4*>(
-                    8u * c8 < a.up_C
-                        ? a.up + (((size_t)n * (a.H >> 1) + (size_t)(y >> 1)) * (a.W >> 1) + (size_t)(x >> 1)) * a.up_C +
-                              8u * c8
-                        : a.in + (img + (size_t)y * a.W + (size_t)x) * a.in_stride + 8u * c8);
+            if (i < total)
+                *reinterpret_cast<u32x4*>(tile + pix * cs + 8u * c8) = (keep >> b & 1u) ? pre[b] : u32x4{0u, 0u, 0u, 0u};
         }
     };
     uint32_t t = blockIdx.x;
     if (t < ntiles) fetch_tile(t);
-    const uint32_t lane = tid & 63u, wave = tid >> 6;
-    const uint32_t g = lane >> 4, r = lane & 15u;
-    const uint32_t rowbase = (uint32_t)MT * wave;
-    // this lane's centre pixel of row 0 of its rows, and its weight row
-    const uint16_t* const abase = tile + (size_t)((rowbase + 1u) * (kTileX + 2) + r + 1u) * cs;
-    const uint32_t rstep = (uint32_t)(kTileX + 2) * cs;
-    const uint16_t* const wrow = wl + (size_t)r * WP + 8u * g;
-    const bool vec = !OUTF && a.Cout % 4u == 0 && a.out_stride % 4u == 0 && a.out_off % 4u == 0 &&
-                     (!MASK || a.mask_stride % 4u == 0);
-    // this lane's biases, loaded once: loads in the epilogue would also wait for the next
-    // tile's fetch (vector loads complete in order)
-    float bias[NT][4];
+    // this lane's weights (past Cout the last row again: outputs nobody stores) and biases
+    bf16x8 w[KS];
+    const uint16_t* const wrow = a.w + (size_t)min(co16 + r, a.Cout - 1u) * (9u * a.Cin);
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (uint32_t k = 0; k < (uint32_t)KS; ++k) {
+        const uint32_t kk = 32u * k + 8u * g, tap = kk / (uint32_t)CI, ci = kk % (uint32_t)CI;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(wrow + min(tap, 8u) * a.Cin + min(ci, a.Cin - 8u));
+        w[k] = __builtin_bit_cast(bf16x8, tap < 9u && ci < a.Cin ? v : u32x4{0u, 0u, 0u, 0u});
+    }
+    const uint32_t co0 = co16 + 4u * g;
+    float bias[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t co = (uint32_t)j * 16u + 4u * g + (uint32_t)i;
-            bias[j][i] = (a.bias && co < a.Cout) ? a.bias[co] : 0.0f;
+    for (uint32_t i = 0; i < 4u; ++i) bias[i] = (a.bias && co0 + i < a.Cout) ? a.bias[co0 + i] : 0.0f;
+    __syncthreads();   // the zeros
+    uint32_t buf = 0;
+    if (t < ntiles) store_tile(lds);
+    __syncthreads();
+    for (; t < ntiles; t += gridDim.x, buf ^= 1u) {
+        const bool more = t + gridDim.x < ntiles;
+        if (more) fetch_tile(t + gridDim.x);
+        const uint16_t* const base = lds + buf * (kResPix * cs) + (rowbase * (kTileX + 2) + r) * cs + 8u * g;
+        // of a step whose second half lies in the next pixel, of the one whose second half lies in the next
+        // row of taps (its first half is the end of this one), and of the one whose second half is padding
+        const bool up = g >= 2u;
+        const uint16_t* const cross = base + (up ? 8 : 0);
+        const uint16_t* const mixed = base + (up ? (kTileX + 2) * cs - 16 : 2 * cs + CI - 16);
+        const uint16_t* const last = base + 2 * cs + CI - 16 + (up ? 16 - 8 * (int)g : 0);
+        f32x4 acc[ROWS];
+#pragma unroll
+        for (int m = 0; m < ROWS; ++m) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if constexpr (CI == 64 && res_simd(NT, CI) == 2) {
+            // the next row's fragments are read while this row's MFMAs run (64 -> 64 channels at 1088 x 1920 149 ->
+            // 141 us; fewer channels gain nothing, more have no registers for it)
+            bf16x8 A[2][kRow / 32];
+            auto read_row = [&](int i, bf16x8 (&dst)[kRow / 32]) {
+#pragma unroll
+                for (int k = 0; k < kRow / 32; ++k) dst[k] = ld8(base + (i * (kTileX + 2) + 32 * k / CI) * cs + 32 * k % CI);
+            };
+            read_row(0, A[0]);
+#pragma unroll
+            for (int i = 0; i < ROWS + 2; ++i) {   // a row of the halo: dy of output row i - dy
+                if (i < ROWS + 1) read_row(i + 1, A[(i + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < kRow / 32; ++k)
+#pragma unroll
+                    for (int dy = 0; dy < 3; ++dy)
+                        if (i - dy >= 0 && i - dy < ROWS)
+                            acc[i - dy] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[dy * (kRow / 32) + k], A[i & 1][k],
+                                                                                 acc[i - dy], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < ROWS + 2; ++i) {   // a row of the halo: dy of output row i - dy
+                if (CI % 32 != 0 && i >= 1 && i - 1 < ROWS)
+                    acc[i - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[kRow / 32], ld8(mixed + (i - 1) * (kTileX + 2) * cs),
+                                                                         acc[i - 1], 0, 0, 0);
+#pragma unroll
+                for (int rel = 0; rel + 32 <= kRow; rel += 16) {   // a step's start within its row of taps
+                    const bool first = rel % 32 == 0;              // dy 0 and 2 (and 1 where CI is a multiple of 32)
+                    if (!first && CI % 32 == 0) continue;
+                    const uint16_t* const at = rel / CI != (rel + 31) / CI ? cross : base;
+                    const bf16x8 A = ld8(at + (i * (kTileX + 2) + rel / CI) * cs + rel % CI);
+#pragma unroll
+                    for (int dy = 0; dy < 3; ++dy) {
+                        if ((dy * kRow + rel) % 32 != 0 || i - dy < 0 || i - dy >= ROWS) continue;
+                        acc[i - dy] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[(dy * kRow + rel) / 32], A, acc[i - dy], 0, 0, 0);
+                    }
+                }
+                if (CI % 32 != 0 && i >= 2)
+                    acc[i - 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[KS - 1], ld8(last + i * (kTileX + 2) * cs), acc[i - 2], 0,
+                                                                         0, 0);
+            }
         }
-    for (; t < ntiles; t += gridDim.x) {
-        __syncthreads();   // the previous tile is no longer read (and weights and offsets are written)
-#pragma unroll
-        for (uint32_t b = 0; b < kCh; ++b) {
-            const uint32_t i = tid + kThreads * b;
-            const uint32_t pix = (i * inv) >> 20, c8 = i - pix * cpp;
-            if (i < total) *reinterpret_cast<u32x4*>(tile + (size_t)pix * cs + 8u * c8) = pre[b];
-        }
-        __syncthreads();
+        if (more) store_tile(lds + (buf ^ 1u) * (kResPix * cs));
         uint32_t n;
         int tx0, ty0;
         origin(t, n, tx0, ty0);
-        if (t + gridDim.x < ntiles) fetch_tile(t + gridDim.x);
-        f32x4 acc[MT][NT];
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int j = 0; j < NT; ++j) acc[m][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        // software-pipelined by hand: the operands of step s + 1 (and the offset of step s + 2)
-        // are read while the MFMAs of step s run; KS is even, reads past the last step hit the
-        // zero padding (A) or whatever follows the weight row (B, unused)
-        bf16x8 A0[MT], B0[NT], A1[MT], B1[NT];
-        auto load = [&](uint32_t ks, uint32_t o, bf16x8 (&A)[MT], bf16x8 (&B)[NT]) {
-            const uint16_t* const ap = abase + (int32_t)o;
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-                A[m] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(ap + (size_t)m * rstep));
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-                B[j] = __builtin_bit_cast(bf16x8,
-                                          *reinterpret_cast<const u32x4*>(wrow + (size_t)j * 16u * WP + 32u * ks));
-        };
-        auto mma = [&](const bf16x8 (&A)[MT], const bf16x8 (&B)[NT]) {
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-#pragma unroll
-                for (int m = 0; m < MT; ++m)
-                    acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[j], A[m], acc[m][j], 0, 0, 0);
-        };
-        load(0u, offs[g], A0, B0);
-        uint32_t o1 = offs[4u + g];
-        // (scheduling barriers keep each group of reads ahead of the MFMAs it overlaps)
-        for (uint32_t ks = 0; ks < KS; ks += 2u) {
-            load(ks + 1u, o1, A1, B1);
-            const uint32_t o2 = offs[4u * (ks + 2u) + g];
-            __builtin_amdgcn_sched_barrier(0);
-            mma(A0, B0);
-            __builtin_amdgcn_sched_barrier(0);
-            load(ks + 2u, o2, A0, B0);
-            o1 = offs[4u * (ks + 3u) + g];
-            __builtin_amdgcn_sched_barrier(0);
-            mma(A1, B1);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // D layout: lane holds output channels 16j + 4g .. 16j + 4g + 3 of pixel r of row m
-        const int x = tx0 + (int)r;
-        if constexpr (MT == 2 && !OUTF && !MASK) {
-            if (a.pool) {
-                epilogue_pool<NT, RELU>(a, acc, bias, 0u, n, x, ty0 + (int)rowbase, g, r);
-                continue;
-            }
-        }
-        if (x >= (int)a.W) continue;
-        const size_t img = (size_t)n * a.H * a.W;
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const int y = ty0 + (int)rowbase + m;
-            if (y >= (int)a.H) continue;
-            const size_t p = img + (size_t)y * a.W + (size_t)x;
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const uint32_t co0 = (uint32_t)j * 16u + 4u * g;
-                if (co0 >= a.Cout) continue;
-                if (vec) {
-                    float v[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        v[i] = acc[m][j][i] + bias[j][i];
-                        if (RELU) v[i] = v[i] > 0.0f ? v[i] : 0.0f;
-                    }
-                    if (MASK) {
-                        const uint2 mk = *reinterpret_cast<const uint2*>(a.mask + p * a.mask_stride + co0);
-                        if (!(bf2f(mk.x) > 0.0f)) v[0] = 0.0f;
-                        if (!(bf2f(mk.x >> 16) > 0.0f)) v[1] = 0.0f;
-                        if (!(bf2f(mk.y) > 0.0f)) v[2] = 0.0f;
-                        if (!(bf2f(mk.y >> 16) > 0.0f)) v[3] = 0.0f;
-                    }
-                    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + p * a.out_stride + a.out_off + co0) =
-                        make_uint2(pk2bf(v[0], v[1]), pk2bf(v[2], v[3]));
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const uint32_t co = co0 + (uint32_t)i;
-                        if (co >= a.Cout) continue;
-                        float v = acc[m][j][i] + bias[j][i];
-                        if (RELU) v = v > 0.0f ? v : 0.0f;
-                        if (MASK && !(bf2f(a.mask[p * a.mask_stride + co]) > 0.0f)) v = 0.0f;
-                        if (OUTF) reinterpret_cast<float*>(a.out)[p * a.out_stride + a.out_off + co] = v;
-                        else reinterpret_cast<uint16_t*>(a.out)[p * a.out_stride + a.out_off + co] = f2bf(v);
-                    }
-                }
-            }
-        }
+        put_rows<ROWS, RELU, OUTF, MASK>(a, acc, bias, co0, n, tx0, ty0 + (int)rowbase, r);
+        __syncthreads();   // this tile is no longer read, the next one is written
     }
 }
 
@@ -1203,29 +1122,41 @@ uint32_t device_cus() {
     return (uint32_t)n;
 }
 
-// resident-weight launch when the weights and a tile fit in LDS and every workgroup gets at
-// least two tiles; returns 1 when not applicable
-template <int MT, int NW, int NT, bool RELU, bool OUTF, bool MASK>
+// resident-weight launch when there are two tiles for every CU; returns 1 when not applicable.  Fewer
+// workgroups than the CUs hold where those would get less than two tiles each: the weights are read
+// once a workgroup.
+template <int NT, int CI, bool RELU, bool OUTF, bool MASK>
 int launch_res(const ConvArgs& a, hipStream_t s) {
-    constexpr uint32_t kMaxLds = 160u * 1024u;
-    if (a.Cin > kResMaxCin) return 1;
-    const size_t lds = conv_res_lds<NT>(NW * MT, a.Cin);
-    if (lds > kMaxLds) return 1;
-    const uint32_t ntx = (a.W + kTileX - 1) / kTileX, nty = (a.H + NW * MT - 1u) / (NW * MT);
+    const uint32_t ntx = (a.W + kTileX - 1u) / kTileX, nty = (a.H + (uint32_t)res_y(NT) - 1u) / (uint32_t)res_y(NT);
     const size_t ntiles = (size_t)ntx * nty * a.N;
-    const uint32_t per_cu = std::max<uint32_t>(1u, std::min<uint32_t>(8u / NW, (uint32_t)(kMaxLds / lds)));
-    const size_t grid = (size_t)device_cus() * per_cu;
-    if (ntiles < 2u * grid || ntiles > 0xFFFFFFFFu) return 1;
-    static size_t allowed = 65536;
-    if (lds > allowed) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conv3x3_res<MT, NW, NT, RELU, OUTF, MASK>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    size_t grid = (size_t)device_cus() * res_per_cu(NT, CI);
+    if (ntiles < 2u * device_cus() || ntiles > 0xFFFFFFFFu) return 1;
+    if (ntiles < 2u * grid) grid = std::max<size_t>(device_cus(), ntiles / 2u);
+    static bool allowed = false;
+    if (!allowed) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conv3x3_res<NT, CI, RELU, OUTF, MASK>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)res_lds(NT, CI)) != hipSuccess)
             return -1;
-        allowed = lds;
+        allowed = true;
     }
-    hipLaunchKernelGGL((k_conv3x3_res<MT, NW, NT, RELU, OUTF, MASK>), dim3((uint32_t)grid), dim3(64 * NW), lds, s, a,
-                       ntx, nty, (uint32_t)ntiles);
+    hipLaunchKernelGGL((k_conv3x3_res<NT, CI, RELU, OUTF, MASK>), dim3((uint32_t)grid), dim3(64u * res_waves(NT)), res_lds(NT, CI),
+                       s, a, ntx, nty, (uint32_t)ntiles);
     return 0;
+}
+template <int NT, bool RELU, bool OUTF, bool MASK>
+int launch_res(const ConvArgs& a, hipStream_t s) {
+    switch (a.Cin) {
+        case 16: return launch_res<NT, 16, RELU, OUTF, MASK>(a, s);
+        case 8: case 32: return launch_res<NT, 32, RELU, OUTF, MASK>(a, s);
+        case 48: return launch_res<NT, 48, RELU, OUTF, MASK>(a, s);
+        case 64: return launch_res<NT, 64, RELU, OUTF, MASK>(a, s);
+        default: break;
+    }
+    if constexpr (NT <= 4) {   // (more waves have no registers for the weights of 80 and 96 channels)
+        if (a.Cin == 80u) return launch_res<NT, 80, RELU, OUTF, MASK>(a, s);
+        if (a.Cin == 96u) return launch_res<NT, 96, RELU, OUTF, MASK>(a, s);
+    }
+    return 1;
 }
 
 // LDS above 64 KiB is allowed first (once per instantiation and size)
@@ -1248,15 +1179,15 @@ int launch_split(const ConvArgs& a, uint32_t groups, hipStream_t s) {
 // nt: 16-channel groups of the output
 template <bool RELU, bool OUTF, bool MASK>
 int launch_conv_nt(uint32_t nt, const ConvArgs& a, hipStream_t s) {
-    // resident weights where they fit and the grid has enough tiles, else split output channels
+    // resident weights where there are tiles enough, else split output channels
     int rc = 1;
     switch (nt) {
-        case 1: rc = launch_res<2, 8, 1, RELU, OUTF, MASK>(a, s); break;
-        case 2: rc = launch_res<2, 8, 2, RELU, OUTF, MASK>(a, s); break;
-        case 3: rc = launch_res<2, 8, 3, RELU, OUTF, MASK>(a, s); break;
-        case 4: rc = launch_res<2, 8, 4, RELU, OUTF, MASK>(a, s); break;
-        case 5: rc = launch_res<2, 8, 5, RELU, OUTF, MASK>(a, s); break;
-        case 6: rc = launch_res<2, 8, 6, RELU, OUTF, MASK>(a, s); break;
+        case 1: rc = launch_res<1, RELU, OUTF, MASK>(a, s); break;
+        case 2: rc = launch_res<2, RELU, OUTF, MASK>(a, s); break;
+        case 3: rc = launch_res<3, RELU, OUTF, MASK>(a, s); break;
+        case 4: rc = launch_res<4, RELU, OUTF, MASK>(a, s); break;
+        case 5: rc = launch_res<5, RELU, OUTF, MASK>(a, s); break;
+        case 6: rc = launch_res<6, RELU, OUTF, MASK>(a, s); break;
         default: break;
     }
     if (rc <= 0) return rc;
@@ -1390,8 +1321,9 @@ void prep_weights(hipStream_t s) {
 
 // forward pass on net.x0 (N x H x W, H and W multiples of 16) -> net.y
 // fuse_up: read the decoder's upsampled channels straight from the lower level in the
-// convolutions' staging instead of materialising them in cat[l] (inference; training keeps
-// cat[l] whole, its weight gradient reads it)
+// convolutions' staging instead of materialising them in cat[l], which then holds the skip alone, pixel
+// by pixel (half of each 160 B row of the level-0 concatenation lies in lines that the other half shares);
+// inference only, training keeps cat[l] whole, its weight gradient reads it
 int forward(uint32_t N, uint32_t H, uint32_t W, hipStream_t s, bool fuse_up = false) {
     prep_weights(s);
     int rc = 0;
@@ -1399,7 +1331,8 @@ int forward(uint32_t N, uint32_t H, uint32_t W, hipStream_t s, bool fuse_up = fa
     for (int l = 0; l < 4 && rc == 0; ++l) {
         const uint32_t h = H >> l, w = W >> l;
         rc |= conv_fwd(2 * l, in, net.a[l].p, net.a[l].C, 0, N, h, w, false, s);
-        rc |= conv_fwd(2 * l + 1, net.a[l], net.cat[l].p, net.cat[l].C, net.U[l], N, h, w, false, s, net.pool[l].p);
+        rc |= conv_fwd(2 * l + 1, net.a[l], net.cat[l].p, fuse_up ? net.E[l] : net.cat[l].C, fuse_up ? 0u : net.U[l], N, h,
+                       w, false, s, net.pool[l].p);
         in = net.pool[l];
     }
     const uint32_t h4 = H >> 4, w4 = W >> 4;
@@ -1410,7 +1343,9 @@ int forward(uint32_t N, uint32_t H, uint32_t W, hipStream_t s, bool fuse_up = fa
         const uint32_t h = H >> l, w = W >> l;
         const int li = 10 + 2 * (3 - l);
         if (fuse_up) {
-            rc |= conv_fwd(li, net.cat[l], net.d1[l].p, net.d1[l].C, 0, N, h, w, false, s, nullptr, &prev);
+            // (channel U of a pixel is the skip's first; those below are never read from here)
+            const Tensor skip{net.cat[l].p - net.U[l], net.E[l]};
+            rc |= conv_fwd(li, skip, net.d1[l].p, net.d1[l].C, 0, N, h, w, false, s, nullptr, &prev);
         } else {
             const size_t n8 = (size_t)N * h * w * (net.U[l] / 8);
             hipLaunchKernelGGL(k_up_fwd, dim3(blocks(n8)), dim3(256), 0, s, prev.p, net.cat[l].p, net.cat[l].C, 0u, N,

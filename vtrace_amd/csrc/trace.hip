@@ -40,6 +40,7 @@
 #include <cstddef>
 
 #include <cstring>
+#include <type_traits>
 
 #include "vt_internal.h"
 
@@ -951,13 +952,15 @@ __host__ __device__ __forceinline__ uint32_t* slot_counters(uint32_t* counters, 
 }
 
 // Parts and the work a launch hands out without atomics.  Workgroup b belongs to part
-// b % kParts; with own = 1 the waves of part p start on the part's first tiles, one each
+// b % kParts; in a launch with OWN the waves of part p start on the part's first tiles, one each
 // (wave i of the part on tile i), and only the tiles past those come from the part's counter.
 // A launch whose waves cover its items so needs no atomics at all, where every workgroup would
 // find each of the 8 counters exhausted before it ends: k_render0 on a 320 x 240 frame (1200 tiles)
 // 92 -> 59 us, k_secondary on a 640 x 480 frame's sun rays 81 -> 36 us.
-// own = 0 where the launch's workgroups may not all be resident at once (several streams): a tile
-// kept for a workgroup that starts late would be traced when everything else is done.
+// Without OWN where the launch's workgroups may not all be resident at once (several streams): a tile
+// kept for a workgroup that starts late would be traced when everything else is done.  Those
+// instantiations hold no shares: with shares in LDS and none kept, 13 small serving requests took
+// 1310 us instead of 1270.
 // One part's share, in LDS (registers are what the traversal kernels are short of):
 struct Part {
     uint32_t first;   // its first item, or (k_secondary) its number of bounce rays
@@ -969,11 +972,15 @@ struct Parts {
     Part part[kParts];
     uint32_t gone;    // parts whose counter this workgroup has seen exhausted
 };
+// a launch without OWN has no shares
+struct PartsGone {
+    uint32_t gone;
+};
 // (threads p < kParts, each for part p, before the workgroup's first barrier; unit: items per
 // counter step)
-__device__ __forceinline__ void put_part(Parts& P, uint32_t first, uint32_t count, uint32_t own, uint32_t unit) {
+__device__ __forceinline__ void put_part(Parts& P, uint32_t first, uint32_t count, uint32_t unit) {
     const uint32_t p = threadIdx.x;
-    const uint32_t kept = own ? (gridDim.x + kParts - 1u - p) / kParts * (uint32_t)kBlock : 0u;
+    const uint32_t kept = (gridDim.x + kParts - 1u - p) / kParts * (uint32_t)kBlock;
     P.part[p] = Part{first, count, kept, count > kept ? (count - kept + unit - 1u) / unit : 0u};
     if (p == 0) P.gone = 0u;
 }
@@ -996,17 +1003,42 @@ __device__ __forceinline__ uint32_t next_part(uint32_t open) {
 // Part p's counter has passed its end: no other wave of the workgroup asks it again.  (Reading all
 // eight counters here instead, to skip every empty part at once, cost 0.1 ms a launch: their lines
 // are then shared by all XCDs while the atomics still run.)
-__device__ __forceinline__ void mark_gone(Parts& P, uint32_t p) {
+template <typename P_>
+__device__ __forceinline__ void mark_gone(P_& P, uint32_t p) {
     if ((threadIdx.x & 63u) == 0) __hip_atomic_fetch_or(&P.gone, 1u << p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// OWN = false: each wave takes 64 consecutive of the items [0, nwork) at a time from the counters of the
+// parts, from part blockIdx.x % kParts on, until all parts are exhausted.
+template <typename Body>
+__device__ __forceinline__ void for_each_shared(uint32_t* fetch, uint32_t* gone, uint32_t nwork, Body&& body) {
+    const uint32_t lane = threadIdx.x & 63u, all = (nwork + 63u) / 64u;
+    for (uint32_t k = 0; k < kParts; ++k) {
+        const uint32_t p = (blockIdx.x + k) % kParts;
+        const uint32_t t0 = (uint32_t)((uint64_t)all * p / kParts), t1 = (uint32_t)((uint64_t)all * (p + 1u) / kParts);
+        const uint32_t first = t0 * 64u, count = min(t1 * 64u, nwork) - min(t0 * 64u, nwork), tiles = (count + 63u) / 64u;
+        for (;;) {
+            if (__hip_atomic_load(gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & (1u << p)) break;
+            uint32_t t = tiles;
+            if (tiles > 0 && lane == 0) t = atomicAdd(fetch + p * kPartStride, 1u);
+            t = __shfl(t, 0, 64);
+            if (t >= tiles) {
+                if (lane == 0) __hip_atomic_fetch_or(gone, 1u << p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                break;
+            }
+            const uint32_t i = t * 64u + lane;
+            if (i < count) body(first + i);
+        }
+    }
 }
 
 // Each wave takes 64 consecutive items of a part at a time until all parts are exhausted: its own
 // tile first, then tiles of its part from that part's counter (fetch + p * kPartStride), then of
 // the others in turn.  body(item): part p's items are P.part[p].first + [0, count).
 template <typename Body>
-__device__ __forceinline__ void for_each_item(uint32_t* fetch, Parts& P, uint32_t own, Body&& body) {
+__device__ __forceinline__ void for_each_item(uint32_t* fetch, Parts& P, Body&& body) {
     const uint32_t lane = threadIdx.x & 63u;
-    bool start = own != 0u;
+    bool start = true;
     for (;;) {
         uint32_t p = blockIdx.x % kParts, i;
         if (start) {
@@ -1031,10 +1063,10 @@ __device__ __forceinline__ void for_each_item(uint32_t* fetch, Parts& P, uint32_
 }
 
 // Items [0, nwork) in kParts contiguous ranges of whole 64-item tiles (threads p < kParts).
-__device__ __forceinline__ void put_static_part(Parts& P, uint32_t nwork, uint32_t own) {
+__device__ __forceinline__ void put_static_part(Parts& P, uint32_t nwork) {
     const uint32_t tiles = (nwork + 63u) / 64u, p = threadIdx.x;
     const uint32_t t0 = (uint32_t)((uint64_t)tiles * p / kParts), t1 = (uint32_t)((uint64_t)tiles * (p + 1u) / kParts);
-    put_part(P, t0 * 64u, min(t1 * 64u, nwork) - min(t0 * 64u, nwork), own, 64u);
+    put_part(P, t0 * 64u, min(t1 * 64u, nwork) - min(t0 * 64u, nwork), 64u);
 }
 
 // Wave-aggregated append to queue counters q (segments of `cap` slots): the wave's appending
@@ -1195,20 +1227,24 @@ struct TileMap {
     }
 };
 
-template <bool ST, bool DEEP>
+template <bool ST, bool DEEP, bool OWN>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_primary(const ReqGPU* __restrict__ reqs, const BatchGPU* __restrict__ B,
-                                                    const float* __restrict__ srgb_dec, WF wf, uint32_t own,
+                                                    const float* __restrict__ srgb_dec, WF wf,
                                                     unsigned long long* stats) {
     __shared__ uint32_t smem[(kStackLds + 16) * kBlock];
     __shared__ BvhNode tree_lds[kLdsNodes];
     const Lds stk{&smem[threadIdx.x]}, mslot{&smem[kStackLds * kBlock + threadIdx.x]};
-    __shared__ Parts parts;
-    const uint32_t nreq = B->nreq;
-    if (threadIdx.x < kParts) put_static_part(parts, B->work_base[nreq], own);
+    __shared__ std::conditional_t<OWN, Parts, PartsGone> parts;
+    if constexpr (OWN) {
+        if (threadIdx.x < kParts) put_static_part(parts, B->work_base[B->nreq]);
+    } else {
+        if (threadIdx.x == 0) parts.gone = 0u;
+    }
     const TreeLds tree = stage_tree(reqs, B, tree_lds);
     __syncthreads();
     Ctr<ST> ctr;
-    for_each_item(slot_counters(wf.counters, 2), parts, own, [&](uint32_t w) {
+    const uint32_t nreq = B->nreq;
+    auto item = [&](uint32_t w) {
         // the 64 items of a wave share a request (work ranges are 64-aligned)
         const uint32_t r = __builtin_amdgcn_readfirstlane(find_req(B->work_base, nreq, w));
         const ReqGPU& Rq = reqs[r];
@@ -1281,7 +1317,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
             wf.Ls[w] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(no_sun ? 1u : 0u));
         }
         wf.L[w] = L;
-    });
+    };
+    if constexpr (OWN) for_each_item(slot_counters(wf.counters, 2), parts, item);
+    else for_each_shared(slot_counters(wf.counters, 2), &parts.gone, B->work_base[nreq], item);
     if (ST) ctr.flush(stats);
 }
 
@@ -1310,23 +1348,29 @@ constexpr uint32_t kPoolLow = 8;
 // Each ray's query: the origin instance from the surface point first, then (if that walk
 // misses) the other instances the ray enters, in the tree's traversal order with the
 // closest-hit pruning of query(); a sun ray stops at its first hit.
-template <bool ST, bool DEEP, bool ONE>
+template <bool ST, bool DEEP, bool ONE, bool OWN>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_secondary(
     const ReqGPU* __restrict__ reqs, const BatchGPU* __restrict__ B, const float* __restrict__ srgb_dec, WF wf,
-    uint32_t q, uint32_t depth, uint32_t in_idx, uint32_t out_idx, uint32_t fetch_idx, uint32_t bounce, uint32_t own,
+    uint32_t q, uint32_t depth, uint32_t in_idx, uint32_t out_idx, uint32_t fetch_idx, uint32_t bounce,
     unsigned long long* stats) {
     __shared__ uint32_t smem[(kStackLds + 16) * kBlock];
     __shared__ BvhNode tree_lds[kLdsNodes];
     const Lds stk_lds{&smem[threadIdx.x]}, mslot{&smem[kStackLds * kBlock + threadIdx.x]};
     // part p: the bounce rays of segment p of this depth's queue, then the rays of its sun list (the
     // queue is complete, so its counts are read once)
-    __shared__ Parts parts;
+    __shared__ std::conditional_t<OWN, Parts, PartsGone> parts;
     const uint32_t cap = wf.seg_cap;
-    if (threadIdx.x < kParts) {
-        const uint32_t at = threadIdx.x * kPartStride;
-        const uint32_t cb = slot_counters(wf.counters, in_idx)[at], cs = slot_counters(wf.counters, sun_slot(in_idx))[at];
-        const uint32_t nb = bounce ? min(cb, cap) : 0u;
-        put_part(parts, nb, nb + min(cs, cap), own, 1u);
+    uint32_t* const qin = slot_counters(wf.counters, in_idx);
+    uint32_t* const qsun = slot_counters(wf.counters, sun_slot(in_idx));
+    if constexpr (OWN) {
+        if (threadIdx.x < kParts) {
+            const uint32_t at = threadIdx.x * kPartStride;
+            const uint32_t cb = qin[at], cs = qsun[at];
+            const uint32_t nb = bounce ? min(cb, cap) : 0u;
+            put_part(parts, nb, nb + min(cs, cap), 1u);
+        }
+    } else {
+        if (threadIdx.x == 0) parts.gone = 0u;
     }
     const TreeLds tree = stage_tree(reqs, B, tree_lds);
     __syncthreads();
@@ -1336,7 +1380,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     const uint32_t nreq = B->nreq;
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64u - lane));
-    bool start = own != 0u, more = true;   // more: the parts may hold items yet (uniform)
+    bool start = OWN, more = true;   // more: the parts may hold items yet (uniform)
+    uint32_t kp = 0;   // !OWN: parts this wave has found exhausted, from blockIdx.x % kParts on (uniform)
 
     // per-lane item and ray state
     bool busy = false, walking = false, is_bounce = false;
@@ -1359,41 +1404,70 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
         // -- take items for the idle lanes (consecutive items of one part in lane order) --
         const uint64_t idle = __ballot(!busy);
         bool fresh = false;
-        uint32_t item = 0, ipart = 0;
+        uint32_t item = 0, ipart = 0, inb = 0;
         if (idle != 0ull && more) {
             const uint32_t need = (uint32_t)__popcll(idle);
             const uint32_t rank = (uint32_t)__popcll(idle & below);
             uint32_t placed = 0;
-            while (placed < need) {
-                uint32_t p = blockIdx.x % kParts, base, end;
-                const bool kept = start;
-                if (kept) {   // the tile kept for this wave
-                    start = false;
-                    base = 64u * part_wave();
-                    end = parts.part[p].count;
-                } else {
-                    const uint32_t open = open_parts(parts);
-                    more = open != 0u;
-                    if (!more) break;
-                    p = next_part(open);
-                    base = 0;
-                    if (lane == 0) base = atomicAdd(fetch + p * kPartStride, need - placed);
-                    base = __builtin_amdgcn_readfirstlane(base) + parts.part[p].kept;
-                    end = parts.part[p].count;
+            if constexpr (!OWN)
+                while (placed < need && kp < kParts) {
+                    const uint32_t p = (blockIdx.x + kp) % kParts;
+                    const bool gone =
+                        (__hip_atomic_load(&parts.gone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & (1u << p)) != 0u;
+                    uint32_t take = 0;
+                    if (!gone) {
+                        // (both counts loaded before either is used: one round trip)
+                        const uint32_t cb = qin[p * kPartStride], cs = qsun[p * kPartStride];
+                        const uint32_t nb = bounce ? min(cb, cap) : 0u, count = nb + min(cs, cap);
+                        uint32_t base = 0;
+                        if (lane == 0 && count > 0) base = atomicAdd(fetch + p * kPartStride, need - placed);
+                        base = __shfl(base, 0, 64);
+                        take = base < count ? min(count - base, need - placed) : 0u;
+                        if (!busy && rank >= placed && rank < placed + take) {
+                            fresh = true;
+                            item = base + (rank - placed);
+                            ipart = p;
+                            inb = nb;
+                        }
+                        placed += take;
+                    }
+                    if (placed < need) {   // part p has no items left
+                        if (!gone) mark_gone(parts, p);
+                        more = ++kp < kParts;
+                    }
                 }
-                const uint32_t take = base < end ? min(end - base, need - placed) : 0u;
-                if (!busy && rank >= placed && rank < placed + take) {
-                    fresh = true;
-                    item = base + (rank - placed);
-                    ipart = p;
+            if constexpr (OWN)
+                while (placed < need) {
+                    uint32_t p = blockIdx.x % kParts, base, end;
+                    const bool kept = start;
+                    if (kept) {   // the tile kept for this wave
+                        start = false;
+                        base = 64u * part_wave();
+                        end = parts.part[p].count;
+                    } else {
+                        const uint32_t open = open_parts(parts);
+                        more = open != 0u;
+                        if (!more) break;
+                        p = next_part(open);
+                        base = 0;
+                        if (lane == 0) base = atomicAdd(fetch + p * kPartStride, need - placed);
+                        base = __builtin_amdgcn_readfirstlane(base) + parts.part[p].kept;
+                        end = parts.part[p].count;
+                    }
+                    const uint32_t take = base < end ? min(end - base, need - placed) : 0u;
+                    if (!busy && rank >= placed && rank < placed + take) {
+                        fresh = true;
+                        item = base + (rank - placed);
+                        ipart = p;
+                    }
+                    placed += take;
+                    if (!kept && placed < need) mark_gone(parts, p);
                 }
-                placed += take;
-                if (!kept && placed < need) mark_gone(parts, p);
-            }
         }
         // -- set up the new items' rays: the origin walk first --
         if (fresh) {
-            const uint32_t nb = parts.part[ipart].first;   // bounce items of part ipart
+            uint32_t nb = inb;   // bounce items of part ipart
+            if constexpr (OWN) nb = parts.part[ipart].first;
             is_bounce = item < nb;
             const uint32_t slot = is_bounce ? ipart * cap + item : wf.sun[q][ipart * cap + (item - nb)];
             const QueueRec sf = get_rec(&wf.rec[q][slot]);
@@ -1670,16 +1744,16 @@ __global__ void k_zero_counters(uint32_t* c) {
 template <bool ST, bool DEEP>
 __global__ __launch_bounds__(kBlock) void k_render0(const FrameGPU F, const SceneGPU S, const float* __restrict__ srgb_dec,
                                                     HitRecord* __restrict__ hits, float4* __restrict__ rad,
-                                                    uint32_t* fetch, uint32_t nwork, uint32_t own,
+                                                    uint32_t* fetch, uint32_t nwork,
                                                     unsigned long long* stats) {
     __shared__ uint32_t smem[(kStackLds + 16) * kBlock];
     const Lds stk{&smem[threadIdx.x]}, mslot{&smem[kStackLds * kBlock + threadIdx.x]};
     __shared__ Parts parts;
-    if (threadIdx.x < kParts) put_static_part(parts, nwork, own);
+    if (threadIdx.x < kParts) put_static_part(parts, nwork);
     __syncthreads();
     Ctr<ST> ctr;
     const uint32_t spp = F.spp ? F.spp : 1u;
-    for_each_item(fetch, parts, own, [&](uint32_t w) {
+    for_each_item(fetch, parts, [&](uint32_t w) {
         uint32_t px, py, s0;
         if (!work_pixel(F, w, 1u, &px, &py, &s0)) return;
         const uint32_t pix = py * F.width + px;
@@ -1855,18 +1929,15 @@ bool vt_batch_layout(const ReqGPU* reqs, uint32_t n, uint32_t npaths, BatchGPU& 
     return w <= npaths && px < 0xFFFFFFFFull;
 }
 
-template <bool ST, bool DEEP>
-static int launch_batch(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long long* stats, hipEvent_t* ev,
-                        uint8_t* kinds, uint32_t* nstages, hipStream_t s, hipEvent_t acc_after = nullptr,
-                        bool with_acc = true, uint32_t blocks = 0, bool allow_one = true) {
-    const uint32_t nblk = blocks ? blocks : g_persistent_blocks;
-    // Alone on the GPU (blocks = 0), every workgroup of a launch is resident, so its waves start on
-    // tiles of their own, and a launch has no more workgroups than its work has tiles for them: at
-    // most nwork items in the primary launch, one bounce and one sun ray of each in the others.  A
-    // captured launch sequence (nwork = 0 here) runs with any batch, so it keeps the full grid.
-    const uint32_t nwork = Bh.work_base[Bh.nreq], own = blocks == 0u && nwork != 0u ? 1u : 0u;
+template <bool ST, bool DEEP, bool OWN>
+static int launch_own(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long long* stats, hipEvent_t* ev,
+                      uint8_t* kinds, uint32_t* nstages, hipStream_t s, hipEvent_t acc_after, bool with_acc,
+                      uint32_t blocks, bool allow_one) {
+    const uint32_t nblk = blocks ? blocks : g_persistent_blocks, nwork = Bh.work_base[Bh.nreq];
+    // an OWN launch has no more workgroups than its work has tiles for them: at most nwork items in
+    // the primary launch, one bounce and one sun ray of each in the others
     auto grid_of = [&](uint64_t items) {
-        return dim3(own ? (uint32_t)std::min<uint64_t>(nblk, (items + kBlock - 1) / kBlock) : nblk);
+        return dim3(OWN ? (uint32_t)std::min<uint64_t>(nblk, (items + kBlock - 1) / kBlock) : nblk);
     };
     const dim3 grid = grid_of(nwork), grid2 = grid_of(2ull * nwork), block(kBlock);
     const ReqGPU* reqs = reinterpret_cast<const ReqGPU*>(wb.tables);
@@ -1884,19 +1955,18 @@ static int launch_batch(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long
     auto st_at = [&](uint32_t k) { return stats ? stats + (size_t)k * VT_STAT_COUNT : nullptr; };
     hipLaunchKernelGGL(k_zero_counters, dim3(kSlots * kParts / 256), dim3(256), 0, s, wb.counters);
     begin(VT_STAGE_PRIMARY);
-    hipLaunchKernelGGL((k_primary<ST, DEEP>), grid, block, 0, s, reqs, B, g_srgb_dec, wf, own,
-                       st_at(stage));
+    hipLaunchKernelGGL((k_primary<ST, DEEP, OWN>), grid, block, 0, s, reqs, B, g_srgb_dec, wf, st_at(stage));
     end();
     uint32_t fetch = 3, in_idx = 0;
     for (uint32_t d = 0; d <= Bh.max_bounces && fetch < kQueueCounters && kQueueCounters + d + 1 < kSlots; ++d) {
         const uint32_t out_idx = kQueueCounters + d + 1;
         begin(VT_STAGE_SECONDARY);
         if (allow_one && Bh.nreq == 1)
-            hipLaunchKernelGGL((k_secondary<ST, DEEP, true>), grid2, block, 0, s, reqs, B, g_srgb_dec, wf, d & 1u, d,
-                               in_idx, out_idx, fetch, d < Bh.max_bounces ? 1u : 0u, own, st_at(stage));
+            hipLaunchKernelGGL((k_secondary<ST, DEEP, true, OWN>), grid2, block, 0, s, reqs, B, g_srgb_dec, wf, d & 1u, d,
+                               in_idx, out_idx, fetch, d < Bh.max_bounces ? 1u : 0u, st_at(stage));
         else
-            hipLaunchKernelGGL((k_secondary<ST, DEEP, false>), grid2, block, 0, s, reqs, B, g_srgb_dec, wf, d & 1u, d,
-                               in_idx, out_idx, fetch, d < Bh.max_bounces ? 1u : 0u, own, st_at(stage));
+            hipLaunchKernelGGL((k_secondary<ST, DEEP, false, OWN>), grid2, block, 0, s, reqs, B, g_srgb_dec, wf, d & 1u, d,
+                               in_idx, out_idx, fetch, d < Bh.max_bounces ? 1u : 0u, st_at(stage));
         ++fetch;
         end();
         in_idx = out_idx;
@@ -1909,6 +1979,18 @@ static int launch_batch(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long
     }
     if (nstages) *nstages = stage;
     return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// Alone on the GPU (blocks = 0), every workgroup of a launch is resident, so its waves start on
+// tiles of their own.  A captured launch sequence (no work counted in Bh) runs with any batch, so it
+// keeps the full grid and hands out everything by its counters.
+template <bool ST, bool DEEP>
+static int launch_batch(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long long* stats, hipEvent_t* ev,
+                        uint8_t* kinds, uint32_t* nstages, hipStream_t s, hipEvent_t acc_after = nullptr,
+                        bool with_acc = true, uint32_t blocks = 0, bool allow_one = true) {
+    return blocks == 0u && Bh.work_base[Bh.nreq] != 0u
+               ? launch_own<ST, DEEP, true>(Bh, wb, stats, ev, kinds, nstages, s, acc_after, with_acc, blocks, allow_one)
+               : launch_own<ST, DEEP, false>(Bh, wb, stats, ev, kinds, nstages, s, acc_after, with_acc, blocks, allow_one);
 }
 
 // Uploads the request table (stream-ordered) and launches the batched pipeline.  host_tables
@@ -2000,7 +2082,7 @@ static int launch_render0(const FrameGPU& F, const SceneGPU& S, HitRecord* hits,
     if (kinds) kinds[0] = VT_STAGE_RENDER0;
     const uint32_t grid = std::min(g_persistent_blocks, (tiles * 64u + kBlock - 1) / kBlock);
     hipLaunchKernelGGL((k_render0<ST, DEEP>), dim3(grid), dim3(kBlock), 0, s, F, S, g_srgb_dec, hits, rad,
-                       slot_counters(wb.counters, 2), tiles * 64u, 1u, stats);
+                       slot_counters(wb.counters, 2), tiles * 64u, stats);
     if (ev) hipEventRecord(ev[1], s);
     if (nstages) *nstages = 1;
     return hipGetLastError() == hipSuccess ? 0 : -1;

@@ -774,8 +774,45 @@ __device__ __forceinline__ TreeLds stage_tree(const ReqGPU* reqs, const BatchGPU
     return t;
 }
 
+__device__ __forceinline__ BvhNode tree_node(const SceneGPU& S, const TreeLds& tree, uint32_t i) {
+    return tree.on ? lds_node(tree, i) : gld(S.nodes + i);
+}
+
+// The next leaf (instance index) that the ray's box tests leave to be entered, nearer subtrees first;
+// VT_EMPTY when there is none.  The stack holds subtrees to be tested (the root at first).  Both
+// children of a node are read and tested at once: one round trip a level, the farther one waits on
+// the stack and is tested again when it is taken, against what has been hit by then.
+template <bool DEEP>
+__device__ __forceinline__ uint32_t next_leaf(const SceneGPU& S, const TreeLds& tree, V3 O, V3 D, V3 inv_d, bool hit,
+                                              float hit_tn, TravStack<DEEP>& stk) {
+    auto reached = [&](const BvhNode& N, float* tn) {
+        float tf;
+        const bool crossed = slab_node(O, D, inv_d, N, tn, &tf);
+        return crossed & !(tf < 0.0f) & !(hit & (*tn > prune_bound(hit_tn)));
+    };
+    while (stk.sp > 0) {
+        BvhNode N = tree_node(S, tree, stk.pop());
+        float ta, tb;
+        bool in = reached(N, &ta);
+        while (in & (N.right != VT_EMPTY)) {
+            const BvhNode A = tree_node(S, tree, N.left), B = tree_node(S, tree, N.right);
+            const bool a = reached(A, &ta), b = reached(B, &tb);
+            const bool second = b & (!a | (tb < ta));
+            if (a & b) stk.push(second ? N.left : N.right);
+            in = a | b;
+            N = second ? B : A;
+        }
+        if (in) return N.left;
+    }
+    return VT_EMPTY;
+}
+
 // Primary ray: closest hit over all instances through the LBVH (nodes from `tree` in LDS when
 // given).  Secondary rays have their own traversal (in k_secondary).
+// Whatever the order, the closest entry of a box that is hit wins (ties to the lower index).  A counted
+// launch (ST) visits the nodes in the fixed order its counters are defined by; the others search for the
+// next leaf first and then walk all lanes' instances together, nearer ones first, so that lanes at
+// inner nodes do not wait for another's walk and instances behind a hit are not entered.
 template <bool ST, bool DEEP>
 __device__ HitG query(const SceneGPU& S, const FrameGPU& F, V3 O, V3 D, Ctr<ST>& ctr, const Lds& stk_lds,
                       const Lds& mslot, TreeLds tree) {
@@ -789,9 +826,17 @@ __device__ HitG query(const SceneGPU& S, const FrameGPU& F, V3 O, V3 D, Ctr<ST>&
     stk.lds = stk_lds;
     stk.sp = 0;
     stk.push(0u);
+    if constexpr (!ST) {
+        for (;;) {
+            const uint32_t i = next_leaf<DEEP>(S, tree, O, D, inv_d, best.hit, best.tn, stk);
+            if (i == VT_EMPTY) return best;
+            HitG h;
+            if (enter_instance<ST>(S, F, i, O, D, h, ctr, mslot) && better(h, best)) best = h;
+        }
+    }
     while (stk.sp > 0) {
         const uint32_t ni = stk.pop();
-        const BvhNode N = tree.on ? lds_node(tree, ni) : gld(S.nodes + ni);
+        const BvhNode N = tree_node(S, tree, ni);
         ctr.node();
         float tn, tf;
         if (!slab_node(O, D, inv_d, N, &tn, &tf) || tf < 0.0f) continue;

@@ -48,15 +48,15 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kStackLds = 16;   // LBVH stack entries per thread held in LDS
-// Wavefront counter slots: [0] queue of the primary vertices, [2] primary (and mode 0) fetch,
-// [3, 64) fetch counters of the secondary launches, [64 + d + 1] the queue built at depth d.
+// Wavefront counter slots: [0] queue of the primary vertices, [2] primary fetch, [3, 40) fetch counters of
+// the secondary launches, [40] and [41] mode 0, [64 + d + 1] the queue built at depth d.
 // Device-scope atomics on one address serialise (about 12 ns each on MI355X), which would bound
 // a launch at (items / 64) x 12 ns, so every slot holds one counter per part, kPartStride u32
 // apart: workgroups are dispatched round-robin over the 8 XCDs, workgroup b starts on part
 // b % kParts, and a launch's atomics spread over kParts addresses.  A queue is kParts
 // segments of seg_cap slots; part p of a queue's counters fills segment p.
 constexpr uint32_t kSlots = 128;
-constexpr uint32_t kQueueCounters = 64;
+constexpr uint32_t kRender0Slot = 40, kQueueCounters = 64;
 constexpr uint32_t kParts = 8;
 constexpr uint32_t kPartStride = 64;   // 256 B between the counters of one slot
 constexpr uint32_t kCounters = kSlots * kParts * kPartStride;
@@ -1776,8 +1776,11 @@ __device__ void accumulate_pixel(const ReqGPU* __restrict__ reqs, const BatchGPU
 __global__ void k_accumulate(const ReqGPU* __restrict__ reqs, const BatchGPU* __restrict__ B, WF wf) {
     const uint32_t nreq = B->nreq;
     const uint32_t total = B->pix_base[nreq];
-    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x)
-        accumulate_pixel(reqs, B, wf, t);
+    const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
+    // the next launch sequence's counters (a launch of their own was 2 us alone on the GPU and 20 us beside
+    // other streams' persistent workgroups)
+    for (uint32_t c = t0; c < kSlots * kParts; c += gridDim.x * blockDim.x) wf.counters[c * kPartStride] = 0u;
+    for (uint32_t t = t0; t < total; t += gridDim.x * blockDim.x) accumulate_pixel(reqs, B, wf, t);
 }
 
 __global__ void k_zero_counters(uint32_t* c) {
@@ -1789,12 +1792,13 @@ __global__ void k_zero_counters(uint32_t* c) {
 template <bool ST, bool DEEP>
 __global__ __launch_bounds__(kBlock) void k_render0(const FrameGPU F, const SceneGPU S, const float* __restrict__ srgb_dec,
                                                     HitRecord* __restrict__ hits, float4* __restrict__ rad,
-                                                    uint32_t* fetch, uint32_t nwork,
+                                                    uint32_t* fetch, uint32_t* next_fetch, uint32_t nwork,
                                                     unsigned long long* stats) {
     __shared__ uint32_t smem[(kStackLds + 16) * kBlock];
     const Lds stk{&smem[threadIdx.x]}, mslot{&smem[kStackLds * kBlock + threadIdx.x]};
     __shared__ Parts parts;
     if (threadIdx.x < kParts) put_static_part(parts, nwork);
+    if (blockIdx.x == 0 && threadIdx.x < kParts) next_fetch[threadIdx.x * kPartStride] = 0u;   // the next frame's
     __syncthreads();
     Ctr<ST> ctr;
     const uint32_t spp = F.spp ? F.spp : 1u;
@@ -1890,6 +1894,7 @@ int vt_wave_bind(WaveBuffers& wb, void* mem, uint32_t npaths) {
         return r;
     };
     wb.npaths = npaths;
+    wb.clean = false;
     wb.L = take((size_t)npaths * 16);
     wb.Ls = take((size_t)npaths * 16);
     wb.br = take((size_t)npaths * 16);
@@ -1901,6 +1906,12 @@ int vt_wave_bind(WaveBuffers& wb, void* mem, uint32_t npaths) {
     wb.counters = reinterpret_cast<uint32_t*>(take((size_t)kCounters * 4));
     wb.tables = take(sizeof(ReqGPU) * VT_MAX_BATCH + sizeof(BatchGPU));
     return 0;
+}
+
+// Zeroed counters for the launch sequence that follows on s (which leaves them in use until its end).
+static void zero_counters(const WaveBuffers& wb, hipStream_t s) {
+    if (!wb.clean) hipLaunchKernelGGL(k_zero_counters, dim3(kSlots * kParts / 256), dim3(256), 0, s, wb.counters);
+    wb.clean = false;
 }
 
 static WF to_wf(const WaveBuffers& wb) {
@@ -1998,12 +2009,11 @@ static int launch_own(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long l
         ++stage;
     };
     auto st_at = [&](uint32_t k) { return stats ? stats + (size_t)k * VT_STAT_COUNT : nullptr; };
-    hipLaunchKernelGGL(k_zero_counters, dim3(kSlots * kParts / 256), dim3(256), 0, s, wb.counters);
     begin(VT_STAGE_PRIMARY);
     hipLaunchKernelGGL((k_primary<ST, DEEP, OWN>), grid, block, 0, s, reqs, B, g_srgb_dec, wf, st_at(stage));
     end();
     uint32_t fetch = 3, in_idx = 0;
-    for (uint32_t d = 0; d <= Bh.max_bounces && fetch < kQueueCounters && kQueueCounters + d + 1 < kSlots; ++d) {
+    for (uint32_t d = 0; d <= Bh.max_bounces && fetch < kRender0Slot && kQueueCounters + d + 1 < kSlots; ++d) {
         const uint32_t out_idx = kQueueCounters + d + 1;
         begin(VT_STAGE_SECONDARY);
         if (allow_one && Bh.nreq == 1)
@@ -2023,7 +2033,9 @@ static int launch_own(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long l
         end();
     }
     if (nstages) *nstages = stage;
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    const bool ok = hipGetLastError() == hipSuccess;
+    if (with_acc) wb.clean = ok;
+    return ok ? 0 : -1;
 }
 
 // Alone on the GPU (blocks = 0), every workgroup of a launch is resident, so its waves start on
@@ -2069,6 +2081,7 @@ int vt_trace_batch(const ReqGPU* reqs, uint32_t n, const WaveBuffers& wb, unsign
     st = st && stats != nullptr;
     if (hipMemcpyAsync(wb.tables, h, kTableBytes, hipMemcpyHostToDevice, s) != hipSuccess) return -1;
     if (slot >= 0) hipEventRecord(g_ring.ev[slot], s);
+    zero_counters(wb, s);
     if (deep) return st ? launch_batch<true, true>(*Bh, wb, stats, ev, kinds, nstages, s, acc_after, true, blocks)
                         : launch_batch<false, true>(*Bh, wb, stats, ev, kinds, nstages, s, acc_after, true, blocks);
     return st ? launch_batch<true, false>(*Bh, wb, stats, ev, kinds, nstages, s, acc_after, true, blocks)
@@ -2098,10 +2111,12 @@ int vt_trace_accumulate(const WaveBuffers& wb, hipStream_t s, uint32_t blocks) {
     const ReqGPU* reqs = reinterpret_cast<const ReqGPU*>(wb.tables);
     const BatchGPU* B = reinterpret_cast<const BatchGPU*>(static_cast<const char*>(wb.tables) + sizeof(ReqGPU) * VT_MAX_BATCH);
     hipLaunchKernelGGL(k_accumulate, dim3(blocks ? blocks : g_persistent_blocks), dim3(256), 0, s, reqs, B, to_wf(wb));
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    wb.clean = hipGetLastError() == hipSuccess;
+    return wb.clean ? 0 : -1;
 }
 
-// Uploads a batch's request table only (for a captured graph launched afterwards).
+// Uploads a batch's request table only (for a captured graph launched afterwards, then
+// vt_trace_accumulate, which ends the sequence).
 int vt_trace_upload_tables(const ReqGPU* reqs, uint32_t n, const WaveBuffers& wb, hipStream_t s, BatchGPU* layout) {
     if (n == 0 || n > VT_MAX_BATCH || ring_init() != 0) return -1;
     const int slot = g_ring.next;
@@ -2114,6 +2129,7 @@ int vt_trace_upload_tables(const ReqGPU* reqs, uint32_t n, const WaveBuffers& wb
     if (layout) *layout = *Bh;
     if (hipMemcpyAsync(wb.tables, h, kTableBytes, hipMemcpyHostToDevice, s) != hipSuccess) return -1;
     hipEventRecord(g_ring.ev[slot], s);
+    zero_counters(wb, s);
     return 0;
 }
 
@@ -2122,15 +2138,19 @@ static int launch_render0(const FrameGPU& F, const SceneGPU& S, HitRecord* hits,
                           unsigned long long* stats, hipEvent_t* ev, uint8_t* kinds, uint32_t* nstages,
                           hipStream_t s) {
     const uint32_t tiles = ((F.width + 7u) / 8u) * ((F.height + 7u) / 8u);
-    hipLaunchKernelGGL(k_zero_counters, dim3(kSlots * kParts / 256), dim3(256), 0, s, wb.counters);
+    zero_counters(wb, s);
+    const uint32_t slot = wb.render0 & 1u;
+    wb.render0 ^= 1u;
     if (ev) hipEventRecord(ev[0], s);
     if (kinds) kinds[0] = VT_STAGE_RENDER0;
     const uint32_t grid = std::min(g_persistent_blocks, (tiles * 64u + kBlock - 1) / kBlock);
     hipLaunchKernelGGL((k_render0<ST, DEEP>), dim3(grid), dim3(kBlock), 0, s, F, S, g_srgb_dec, hits, rad,
-                       slot_counters(wb.counters, 2), tiles * 64u, stats);
+                       slot_counters(wb.counters, kRender0Slot + slot), slot_counters(wb.counters, kRender0Slot + 1u - slot),
+                       tiles * 64u, stats);
     if (ev) hipEventRecord(ev[1], s);
     if (nstages) *nstages = 1;
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    wb.clean = hipGetLastError() == hipSuccess;
+    return wb.clean ? 0 : -1;
 }
 
 size_t vt_trace_table_bytes() { return kTableBytes; }

@@ -78,6 +78,10 @@ struct WaveBuffers {
     void* tables = nullptr;                 // ReqGPU[VT_MAX_BATCH] then BatchGPU
     void* gsamp = nullptr;                  // optional, owned by the caller: 2 x float4 per path
                                             // (G-buffer of each sample, averaged per pixel)
+    // The counters are zero, but for those of the last mode-0 frame: every launch sequence ends with the
+    // accumulation, which zeroes them for the next one.  Without it they are zeroed first.
+    mutable bool clean = false;
+    mutable uint32_t render0 = 0;           // which of two counter slots the next mode-0 frame uses
 };
 size_t vt_wave_bytes(uint32_t npaths);
 int vt_wave_bind(WaveBuffers& wb, void* mem, uint32_t npaths);

@@ -628,14 +628,16 @@ __device__ __forceinline__ void wgrad_block(const WGradArgs& a, uint32_t chunk, 
 
 // Every layer's weight gradient in one launch at the end of the backward pass: a layer alone has
 // too little work to fill the GPU and to hide its start (19 launches: 175 us a step of 8 crops of 128 x
-// 128, this one 106).  The workgroups that share a chunk are consecutive.
+// 128, this one 92; 99 with the workgroups of a chunk on different XCDs).
 __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_conv3x3_wgrad(WGradTable T) {
     __shared__ __align__(16) uint16_t lds[kWgLds];
     uint32_t l = 0;
     while (l + 1u < (uint32_t)kLayers && blockIdx.x >= T.l[l + 1].first) ++l;
     const WGradArgs& a = T.l[l];
-    const uint32_t b = blockIdx.x - a.first, per = a.cib * a.cob, sub = b % per;
-    const uint32_t chunk = b / per, cib = sub % a.cib, cob = sub / a.cib;
+    // workgroups are dealt to the 8 XCDs in turn: the ones that share a chunk are 8 apart, on one L2
+    const uint32_t b = blockIdx.x - a.first, per = a.cib * a.cob, sub = b / 8u % per;
+    const uint32_t chunk = b / (8u * per) * 8u + b % 8u, cib = sub % a.cib, cob = sub / a.cib;
+    if (chunk * a.tiles_chunk >= a.tiles) return;   // (uniform: chunks come in eights)
     switch (a.nco * 4u + a.nci) {
         case 5: wgrad_block<1, 1>(a, chunk, cib, cob, lds); break;
         case 6: wgrad_block<1, 2>(a, chunk, cib, cob, lds); break;
@@ -1247,8 +1249,9 @@ int conv_bwd_data(int li, const Tensor& g, const Tensor& dx, const Tensor* mask,
 uint32_t layer_level(int li) { return li < 10 ? (uint32_t)li / 2u : li < 18 ? 3u - (uint32_t)(li - 10) / 2u : 0u; }
 
 // How the weight gradients of a batch of N x H x W are split over one launch's workgroups, and where
-// their partial sums lie: about kWgPerCu workgroups per CU in all (as many as are resident: fewer
-// leave CUs idle, more write and read more partial sums), each of about the same work (a tile
+// their partial sums lie: about kWgPerCu workgroups per CU in all (as many as are resident: more write and
+// read more partial sums: 8 fine-tuning steps 4.92 ms with 4, 4.94 with 3, 5.15 with 8; 2 with 64 output channels a
+// workgroup 5.18, 5 with 32 5.10), each of about the same work (a tile
 // costs its staging, about as much as 4 blocks of 16 x 16 channels, and its blocks).
 constexpr uint32_t kWgPerCu = 4;
 int plan_wgrad(uint32_t N, uint32_t H, uint32_t W) {
@@ -1279,7 +1282,7 @@ int plan_wgrad(uint32_t N, uint32_t H, uint32_t W) {
         a.tiles_chunk = (uint32_t)std::max<uint64_t>(1u, std::min<uint64_t>(a.tiles, (share + cost(a) - 1u) / cost(a)));
         const uint32_t chunks = (a.tiles + a.tiles_chunk - 1u) / a.tiles_chunk;
         a.first = first;
-        first += chunks * a.cob * a.cib;
+        first += (chunks + 7u) / 8u * 8u * a.cob * a.cib;
         net.parts.l[i].off = off;
         net.parts.l[i].chunks = chunks;
         net.parts.l[i].n = L.d.nw + L.cout;

@@ -30,7 +30,7 @@
 //   k_conv3x3_wgrad  dW[co][tap][ci] = sum_p dY[p][co] X[p+tap][ci] over a chunk of pixel tiles,
 //                    all nine taps of a block of input channels in registers, the operands
 //                    transposed on the way out of LDS; dbias in the same pass.
-//   pooling, upsampling, feature, loss, Adam and weight-layout kernels are element-wise.
+//   pooling (backward), feature, loss and weight-layout kernels are element-wise.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -83,16 +83,22 @@ struct ConvArgs {
     const uint16_t* up;      // input channels [0, up_C) read from this N x H/2 x W/2 x up_C tensor at
                              // (y/2, x/2) (nearest upsampling), the rest from `in`; up_C = 0: `in`
     uint32_t up_C;
+    // MASK: the mask of channels [0, low_C) is `low_mask`'s (N x H/2 x W/2 x low_C) at (y/2, x/2), and those
+    // channels of the output are summed over 2x2 pixels into `low_sum` (N x H/2 x W/2 x low_C): the gradient
+    // of the level whose upsampling they are.  H and W even; low_C = 0: none
+    const uint16_t* low_mask;
+    uint16_t* low_sum;
+    uint32_t low_C;
     uint32_t in_stride, out_stride, out_off, mask_stride;
     uint32_t N, H, W, Cin, Cout;
 };
 
-// The 2x2 mean pool of a layer whose output is also pooled (a.pool; H and W even): o0, o1 are the
-// BF16 outputs of this lane's pixels (x, y0) and (x, y0 + 1), y0 even, and lanes r, r ^ 1 an even/odd
-// column pair, so the pooled value comes from this lane and its neighbour: the four outputs
-// summed in row-major order, times 0.25, rounded to BF16.  Every lane reaches the shuffles.
-__device__ __forceinline__ void put_pool(const ConvArgs& a, const uint2& o0, const uint2& o1, uint32_t co0, uint32_t n,
-                                         int x, int y0, uint32_t r, bool in) {
+// Sums over 2x2 pixels, times `scale`, rounded to BF16: o0, o1 are this lane's outputs (4 channels) at pixels
+// (x, y0) and (x, y0 + 1), y0 even, and lanes r, r ^ 1 an even/odd column pair, so the sum comes from
+// this lane and its neighbour, in row-major order.  Every lane reaches the shuffles; the even ones store to
+// dst, N x H/2 x W/2 x C.
+__device__ __forceinline__ void put_quad(const ConvArgs& a, uint16_t* dst, uint32_t C, float scale, const uint2& o0,
+                                         const uint2& o1, uint32_t co0, uint32_t n, int x, int y0, uint32_t r, bool in) {
     const uint32_t own[2][2] = {{o0.x, o0.y}, {o1.x, o1.y}};
     uint32_t nb[2][2];
 #pragma unroll
@@ -105,10 +111,10 @@ __device__ __forceinline__ void put_pool(const ConvArgs& a, const uint2& o0, con
     for (int i = 0; i < 4; ++i) {
         const int t = i >> 1, sh = 16 * (i & 1);
         const float s = ((bf2f(own[0][t] >> sh) + bf2f(nb[0][t] >> sh)) + bf2f(own[1][t] >> sh)) + bf2f(nb[1][t] >> sh);
-        o[i] = 0.25f * s;
+        o[i] = scale * s;
     }
     const size_t q = ((size_t)n * (a.H / 2u) + (size_t)(y0 >> 1)) * (a.W / 2u) + (size_t)(x >> 1);
-    *reinterpret_cast<uint2*>(a.pool + q * a.Cout + co0) = make_uint2(pk2bf(o[0], o[1]), pk2bf(o[2], o[3]));
+    *reinterpret_cast<uint2*>(dst + q * C + co0) = make_uint2(pk2bf(o[0], o[1]), pk2bf(o[2], o[3]));
 }
 
 // Epilogue of the convolutions for a wave's ROWS rows of 16 pixels from (tx0, y0), y0 even: a lane holds
@@ -120,7 +126,9 @@ template <int ROWS, bool RELU, bool OUTF, bool MASK>
 __device__ __forceinline__ void put_rows(const ConvArgs& a, const f32x4 (&acc)[ROWS], const float (&bias)[4], uint32_t co0,
                                          uint32_t n, int tx0, int y0, uint32_t r) {
     const bool in_x = tx0 + (int)r < (int)a.W && co0 < a.Cout;
-    const uint32_t at = r * a.out_stride + co0, at_mask = r * a.mask_stride + co0;
+    // (a wave's 16 channels lie below low_C or at and above it: widths are multiples of 16)
+    const bool low = MASK && (uint32_t)__builtin_amdgcn_readfirstlane(co0) < a.low_C;
+    const uint32_t at = r * a.out_stride + co0, at_mask = low ? (r >> 1) * a.low_C + co0 : r * a.mask_stride + co0;
     uint2 o[2] = {make_uint2(0u, 0u), make_uint2(0u, 0u)};
 #pragma unroll
     for (int m = 0; m < ROWS; ++m) {
@@ -140,16 +148,19 @@ __device__ __forceinline__ void put_rows(const ConvArgs& a, const f32x4 (&acc)[R
                 if (in_x && co0 + i < a.Cout) row[at + i] = v[i];
         } else {
             if (MASK && in_x) {
-                const uint2 mk = *reinterpret_cast<const uint2*>(a.mask + p * a.mask_stride + at_mask);
+                const size_t pl = ((size_t)n * (a.H / 2u) + (size_t)(y >> 1)) * (a.W / 2u) + (size_t)(tx0 >> 1);
+                const uint2 mk = *reinterpret_cast<const uint2*>((low ? a.low_mask + pl * a.low_C : a.mask + p * a.mask_stride) + at_mask);
                 if (!(bf2f(mk.x) > 0.0f)) v[0] = 0.0f;
                 if (!(bf2f(mk.x >> 16) > 0.0f)) v[1] = 0.0f;
                 if (!(bf2f(mk.y) > 0.0f)) v[2] = 0.0f;
                 if (!(bf2f(mk.y >> 16) > 0.0f)) v[3] = 0.0f;
             }
             o[m & 1] = make_uint2(pk2bf(v[0], v[1]), pk2bf(v[2], v[3]));
-            if (in_x) *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + p * a.out_stride + a.out_off + at) = o[m & 1];
-            if constexpr (!MASK) {
-                if ((m & 1) && a.pool) put_pool(a, o[0], o[1], co0, n, tx0 + (int)r, y - 1, r, in_x);
+            if (in_x && !low) *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + p * a.out_stride + a.out_off + at) = o[m & 1];
+            if constexpr (MASK) {
+                if ((m & 1) && low) put_quad(a, a.low_sum, a.low_C, 1.0f, o[0], o[1], co0, n, tx0 + (int)r, y - 1, r, in_x);
+            } else {
+                if ((m & 1) && a.pool) put_quad(a, a.pool, a.Cout, 0.25f, o[0], o[1], co0, n, tx0 + (int)r, y - 1, r, in_x);
             }
         }
     }
@@ -480,7 +491,9 @@ __global__ __launch_bounds__(64 * res_waves(NT)) __attribute__((amdgpu_waves_per
 
 // ---- weight gradient ----------------------------------------------------------------------
 struct WGradArgs {
-    const uint16_t* in;   // forward input, N x H x W x in_stride, channels [0, Cin)
+    const uint16_t* in;   // forward input, N x H x W x in_stride, channels [up_C, Cin)
+    const uint16_t* up;   // its channels [0, up_C), N x H/2 x W/2 x up_C at (y/2, x/2)
+    uint32_t up_C;
     const uint16_t* g;    // gradient of the pre-activation output, N x H x W x g_stride (g_stride % 8 == 0)
     float* part;          // [chunks][Cout * 9 * Cin weights, then Cout biases]
     uint32_t in_stride, g_stride;
@@ -534,26 +547,58 @@ __device__ __forceinline__ void wgrad_block(const WGradArgs& a, uint32_t chunk, 
     const uint32_t ci0 = cib * 16u * NCI, co0 = cob * 16u * NCO;
     const uint32_t cout8 = (a.Cout + 7u) & ~7u;
     const uint32_t t1 = min(a.tiles, (chunk + 1u) * a.tiles_chunk);
+    // This thread's chunks: byte offsets from the tile's first pixel (gradient), from the halo's first pixel (input),
+    // and their place in the tile.  Chunks outside the image or the channels read the tile's first pixel and are
+    // zeros in LDS: every load is unconditional, with a wave-uniform base and a few instructions for its
+    // bounds (addresses made anew for each chunk: 92 us a step, or 125 with the upsampled channels read from
+    // below; this 76).
     u32x4 gpre[GB], xpre[XB];
+    uint32_t goff[GB], xoff[XB], gpos[GB], xpos[XB], from_up = 0, keep = 0;
+    const uint32_t gsafe = 2u * co0, xsafe = 2u * ((a.W + 1u) * a.in_stride);
+#pragma unroll
+    for (uint32_t b = 0; b < GB; ++b) {
+        const uint32_t i = tid + kWgThreads * b, pix = i / (2u * NCO), c = co0 + 8u * (i % (2u * NCO));
+        const bool ok = i < GCH && c < cout8;
+        gpos[b] = ok ? pix % kWgX | (pix / kWgX) << 16 : 0xFFFFFFFFu;   // (no such pixel)
+        goff[b] = ok ? 2u * ((pix / kWgX * a.W + pix % kWgX) * a.g_stride + c) : gsafe;
+    }
+#pragma unroll
+    for (uint32_t b = 0; b < XB; ++b) {
+        const uint32_t i = tid + kWgThreads * b, pix = i / (2u * NCI), c = ci0 + 8u * (i % (2u * NCI));
+        const uint32_t lx = pix % XW, ly = pix / XW;
+        const bool ok = i < XCH && c < a.Cin, up = ok && c < a.up_C;
+        xpos[b] = ok ? lx | ly << 16 : 0xFFFFFFFFu;
+        xoff[b] = up ? 2u * ((((ly + 1u) >> 1) * (a.W >> 1) + ((lx + 1u) >> 1)) * a.up_C + c) : 2u * ((ly * a.W + lx) * a.in_stride + c);
+        from_up |= up ? 1u << b : 0u;
+    }
     auto fetch = [&](uint32_t t) {
         const uint32_t tx = t % a.ntx, rest = t / a.ntx, ty = rest % a.nty, n = rest / a.nty;
-        const int x0 = (int)(tx * kWgX), y0 = (int)(ty * kWgY);
-        const size_t img = (size_t)n * a.H * a.W;
+        const uint32_t x0 = tx * kWgX, y0 = ty * kWgY;
+        const size_t p0 = ((size_t)n * a.H + y0) * a.W + x0;
+        const char* const pg = reinterpret_cast<const char*>(a.g + p0 * a.g_stride);
+        const char* const px = reinterpret_cast<const char*>(a.in + p0 * a.in_stride) - xsafe;
+        keep = 0u;
 #pragma unroll
         for (uint32_t b = 0; b < GB; ++b) {
-            const uint32_t i = tid + kWgThreads * b, pix = i / (2u * NCO), c = co0 + 8u * (i % (2u * NCO));
-            const uint32_t x = (uint32_t)x0 + pix % kWgX, y = (uint32_t)y0 + pix / kWgX;
-            gpre[b] = u32x4{0u, 0u, 0u, 0u};
-            if (i < GCH && c < cout8 && x < a.W && y < a.H)
-                gpre[b] = *reinterpret_cast<const u32x4*>(a.g + (img + (size_t)y * a.W + x) * a.g_stride + c);
+            const bool ok = x0 + (gpos[b] & 0xFFFFu) < a.W && y0 + (gpos[b] >> 16) < a.H;
+            gpre[b] = *reinterpret_cast<const u32x4*>(pg + (ok ? goff[b] : gsafe));
+            keep |= ok ? 1u << b : 0u;
         }
+        bool ok[XB];
 #pragma unroll
-        for (uint32_t b = 0; b < XB; ++b) {
-            const uint32_t i = tid + kWgThreads * b, pix = i / (2u * NCI), c = ci0 + 8u * (i % (2u * NCI));
-            const int x = x0 + (int)(pix % XW) - 1, y = y0 + (int)(pix / XW) - 1;
-            xpre[b] = u32x4{0u, 0u, 0u, 0u};
-            if (i < XCH && c < a.Cin && x >= 0 && x < (int)a.W && y >= 0 && y < (int)a.H)
-                xpre[b] = *reinterpret_cast<const u32x4*>(a.in + (img + (size_t)y * a.W + (uint32_t)x) * a.in_stride + c);
+        for (uint32_t b = 0; b < XB; ++b) {   // (the halo's first pixel is (x0 - 1, y0 - 1): unsigned, so outside is large)
+            ok[b] = x0 + (xpos[b] & 0xFFFFu) - 1u < a.W && y0 + (xpos[b] >> 16) - 1u < a.H;
+            keep |= ok[b] ? 1u << (GB + b) : 0u;
+        }
+        if (a.up_C == 0u) {
+#pragma unroll
+            for (uint32_t b = 0; b < XB; ++b) xpre[b] = *reinterpret_cast<const u32x4*>(px + (ok[b] ? xoff[b] : xsafe));
+        } else {
+            const size_t q0 = ((size_t)n * (a.H >> 1) + y0 / 2u) * (a.W >> 1) + x0 / 2u;
+            const char* const pu = reinterpret_cast<const char*>(a.up + q0 * a.up_C) - 2u * ((a.W >> 1) + 1u) * a.up_C;
+#pragma unroll
+            for (uint32_t b = 0; b < XB; ++b)
+                xpre[b] = *reinterpret_cast<const u32x4*>(ok[b] ? ((from_up >> b & 1u) ? pu : px) + xoff[b] : px + xsafe);
         }
     };
     // this lane's pixel and channels of a transposed read
@@ -577,12 +622,13 @@ __device__ __forceinline__ void wgrad_block(const WGradArgs& a, uint32_t chunk, 
 #pragma unroll
         for (uint32_t b = 0; b < GB; ++b) {
             const uint32_t i = tid + kWgThreads * b;
-            if (i < GCH) *reinterpret_cast<u32x4*>(gt + i / (2u * NCO) * GP + 8u * (i % (2u * NCO))) = gpre[b];
+            if (i < GCH) *reinterpret_cast<u32x4*>(gt + i / (2u * NCO) * GP + 8u * (i % (2u * NCO))) = (keep >> b & 1u) ? gpre[b] : u32x4{0u, 0u, 0u, 0u};
         }
 #pragma unroll
         for (uint32_t b = 0; b < XB; ++b) {
             const uint32_t i = tid + kWgThreads * b;
-            if (i < XCH) *reinterpret_cast<u32x4*>(xt + i / (2u * NCI) * XP + 8u * (i % (2u * NCI))) = xpre[b];
+            if (i < XCH) *reinterpret_cast<u32x4*>(xt + i / (2u * NCI) * XP + 8u * (i % (2u * NCI))) =
+                    (keep >> (GB + b) & 1u) ? xpre[b] : u32x4{0u, 0u, 0u, 0u};
         }
         __syncthreads();
         if (t + 1u < t1) fetch(t + 1u);
@@ -628,7 +674,7 @@ __device__ __forceinline__ void wgrad_block(const WGradArgs& a, uint32_t chunk, 
 
 // Every layer's weight gradient in one launch at the end of the backward pass: a layer alone has
 // too little work to fill the GPU and to hide its start (19 launches: 175 us a step of 8 crops of 128 x
-// 128, this one 92; 99 with the workgroups of a chunk on different XCDs).
+// 128, this one 76; 99 with the workgroups of a chunk on different XCDs and addresses made for each load).
 __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_conv3x3_wgrad(WGradTable T) {
     __shared__ __align__(16) uint16_t lds[kWgLds];
     uint32_t l = 0;
@@ -730,39 +776,6 @@ __global__ void k_pool_bwd(const uint16_t* __restrict__ gpool, const uint16_t* _
         o[t] = h2[0] | (h2[1] << 16);
     }
     *reinterpret_cast<u32x4*>(g + (size_t)p * C + c8 * 8u) = o;
-}
-
-// out (N x 2h x 2w, stride, off) = nearest upsampling of in (N x h x w x C)
-__global__ void k_up_fwd(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, uint32_t out_stride,
-                         uint32_t out_off, uint32_t N, uint32_t H, uint32_t W, uint32_t C) {
-    const uint32_t c8n = C / 8u;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N * H * W * c8n) return;
-    const uint32_t c8 = i % c8n, p = i / c8n;
-    const uint32_t x = p % W, y = (p / W) % H, n = p / (W * H);
-    const uint32_t parent = (n * (H / 2u) + y / 2u) * (W / 2u) + x / 2u;
-    *reinterpret_cast<u32x4*>(out + (size_t)p * out_stride + out_off + c8 * 8u) =
-        *reinterpret_cast<const u32x4*>(in + (size_t)parent * C + c8 * 8u);
-}
-
-// g (N x h x w x C) = sum over the 4 children of gcat (N x 2h x 2w, stride, channels [0, C))
-__global__ void k_up_bwd(const uint16_t* __restrict__ gcat, uint32_t stride, uint16_t* __restrict__ g, uint32_t N,
-                         uint32_t h, uint32_t w, uint32_t C) {
-    const uint32_t c8n = C / 8u;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N * h * w * c8n) return;
-    const uint32_t c8 = i % c8n, q = i / c8n;
-    const uint32_t x = q % w, y = (q / w) % h, n = q / (w * h);
-    const uint32_t W = 2u * w, H = 2u * h;
-    float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (uint32_t d = 0; d < 4; ++d) {
-        const uint32_t p = (n * H + 2u * y + (d >> 1)) * W + 2u * x + (d & 1u);
-        const u32x4 v = *reinterpret_cast<const u32x4*>(gcat + (size_t)p * stride + c8 * 8u);
-        for (int t = 0; t < 8; ++t) s[t] += bf2f(half16(v, t));
-    }
-    u32x4 o;
-    for (int t = 0; t < 4; ++t) o[t] = (uint32_t)f2bf(s[2 * t]) | ((uint32_t)f2bf(s[2 * t + 1]) << 16);
-    *reinterpret_cast<u32x4*>(g + (size_t)q * C + c8 * 8u) = o;
 }
 
 // features of an h x w frame into an hp x wp tensor (edge-replicated padding), 16 channels:
@@ -1225,8 +1238,10 @@ int conv_fwd(int li, const Tensor& in, void* out, uint32_t out_stride, uint32_t 
 
 // backward-data of layer li: g (Cout channels, stride g.C, g.C % 8 == 0) -> dX (Cin channels),
 // masked by the forward input X (> 0) when mask is given
+// low, low_g (optional, H and W even): X's channels [0, low.C) are the upsampling of `low`, whose gradient (masked
+// by it) goes to low_g instead of dX
 int conv_bwd_data(int li, const Tensor& g, const Tensor& dx, const Tensor* mask, uint32_t N, uint32_t H, uint32_t W,
-                  hipStream_t s) {
+                  hipStream_t s, const Tensor* low = nullptr, const Tensor* low_g = nullptr) {
     const Layer& L = net.L[li];
     ConvArgs a{};
     a.in = a.up = g.p;
@@ -1238,6 +1253,11 @@ int conv_bwd_data(int li, const Tensor& g, const Tensor& dx, const Tensor* mask,
     a.out_off = 0;
     a.mask = mask ? mask->p : nullptr;
     a.mask_stride = mask ? mask->C : 0;
+    if (low) {
+        a.low_mask = low->p;
+        a.low_sum = low_g->p;
+        a.low_C = low->C;
+    }
     a.N = N; a.H = H; a.W = W;
     a.Cin = L.d.cout8;
     a.Cout = L.cin;
@@ -1249,10 +1269,10 @@ int conv_bwd_data(int li, const Tensor& g, const Tensor& dx, const Tensor* mask,
 uint32_t layer_level(int li) { return li < 10 ? (uint32_t)li / 2u : li < 18 ? 3u - (uint32_t)(li - 10) / 2u : 0u; }
 
 // How the weight gradients of a batch of N x H x W are split over one launch's workgroups, and where
-// their partial sums lie: about kWgPerCu workgroups per CU in all (as many as are resident: more write and
-// read more partial sums: 8 fine-tuning steps 4.92 ms with 4, 4.94 with 3, 5.15 with 8; 2 with 64 output channels a
-// workgroup 5.18, 5 with 32 5.10), each of about the same work (a tile
-// costs its staging, about as much as 4 blocks of 16 x 16 channels, and its blocks).
+// their partial sums lie: about kWgPerCu workgroups per CU in all, as many as are resident (more write and
+// read more partial sums; 8 fine-tuning steps 4.92 ms with 4, 4.94 with 3, 5.15 with 8, with 64 output channels
+// a workgroup and 2 per CU 5.18, with 32 and 5 5.10), each of about the same work: a tile costs its staging,
+// about as much as 4 blocks of 16 x 16 channels, and its blocks.
 constexpr uint32_t kWgPerCu = 4;
 int plan_wgrad(uint32_t N, uint32_t H, uint32_t W) {
     uint64_t work = 0;
@@ -1304,9 +1324,12 @@ int plan_wgrad(uint32_t N, uint32_t H, uint32_t W) {
     return 0;
 }
 
-// the operands of layer li's weight gradient: its input x and its output's gradient g
-void wgrad_of(int li, const Tensor& x, const Tensor& g) {
+// the operands of layer li's weight gradient: its input x (channels [0, up.C) the upsampling of up) and its
+// output's gradient g
+void wgrad_of(int li, const Tensor& x, const Tensor& g, const Tensor* up = nullptr) {
     WGradArgs& a = net.wg.l[li];
+    a.up = up ? up->p : x.p;
+    a.up_C = up ? up->C : 0u;
     a.in = x.p;
     a.in_stride = x.C;
     a.g = g.p;
@@ -1323,18 +1346,17 @@ void prep_weights(hipStream_t s) {
 }
 
 // forward pass on net.x0 (N x H x W, H and W multiples of 16) -> net.y
-// fuse_up: read the decoder's upsampled channels straight from the lower level in the
-// convolutions' staging instead of materialising them in cat[l], which then holds the skip alone, pixel
-// by pixel (half of each 160 B row of the level-0 concatenation lies in lines that the other half shares);
-// inference only, training keeps cat[l] whole, its weight gradient reads it
-int forward(uint32_t N, uint32_t H, uint32_t W, hipStream_t s, bool fuse_up = false) {
+// The decoder's upsampled channels are read straight from the lower level wherever they are needed; cat[l]
+// holds the skip, in its channels of the concatenation, or (dense: inference) by itself, pixel by
+// pixel: half of each 160 B row of the level-0 concatenation lies in lines that the other half shares.
+int forward(uint32_t N, uint32_t H, uint32_t W, hipStream_t s, bool dense = false) {
     prep_weights(s);
     int rc = 0;
     Tensor in = net.x0;
     for (int l = 0; l < 4 && rc == 0; ++l) {
         const uint32_t h = H >> l, w = W >> l;
         rc |= conv_fwd(2 * l, in, net.a[l].p, net.a[l].C, 0, N, h, w, false, s);
-        rc |= conv_fwd(2 * l + 1, net.a[l], net.cat[l].p, fuse_up ? net.E[l] : net.cat[l].C, fuse_up ? 0u : net.U[l], N, h,
+        rc |= conv_fwd(2 * l + 1, net.a[l], net.cat[l].p, dense ? net.E[l] : net.cat[l].C, dense ? 0u : net.U[l], N, h,
                        w, false, s, net.pool[l].p);
         in = net.pool[l];
     }
@@ -1345,16 +1367,9 @@ int forward(uint32_t N, uint32_t H, uint32_t W, hipStream_t s, bool fuse_up = fa
     for (int l = 3; l >= 0 && rc == 0; --l) {
         const uint32_t h = H >> l, w = W >> l;
         const int li = 10 + 2 * (3 - l);
-        if (fuse_up) {
-            // (channel U of a pixel is the skip's first; those below are never read from here)
-            const Tensor skip{net.cat[l].p - net.U[l], net.E[l]};
-            rc |= conv_fwd(li, skip, net.d1[l].p, net.d1[l].C, 0, N, h, w, false, s, nullptr, &prev);
-        } else {
-            const size_t n8 = (size_t)N * h * w * (net.U[l] / 8);
-            hipLaunchKernelGGL(k_up_fwd, dim3(blocks(n8)), dim3(256), 0, s, prev.p, net.cat[l].p, net.cat[l].C, 0u, N,
-                               h, w, net.U[l]);
-            rc |= conv_fwd(li, net.cat[l], net.d1[l].p, net.d1[l].C, 0, N, h, w, false, s);
-        }
+        // (dense: channel U of a pixel is the skip's first; those below are never read from here)
+        const Tensor skip = dense ? Tensor{net.cat[l].p - net.U[l], net.E[l]} : net.cat[l];
+        rc |= conv_fwd(li, skip, net.d1[l].p, net.d1[l].C, 0, N, h, w, false, s, nullptr, &prev);
         rc |= conv_fwd(li + 1, net.d1[l], net.d2[l].p, net.d2[l].C, 0, N, h, w, false, s);
         prev = net.d2[l];
     }
@@ -1382,13 +1397,10 @@ int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, const float* l
         const int li = 10 + 2 * (3 - l);
         wgrad_of(li + 1, net.d1[l], net.gd2[l]);
         rc |= conv_bwd_data(li + 1, net.gd2[l], net.gd1[l], &net.d1[l], N, h, w, s);
-        wgrad_of(li, net.cat[l], net.gd1[l]);
-        rc |= conv_bwd_data(li, net.gd1[l], net.gcat[l], &net.cat[l], N, h, w, s);
-        // up part of the concatenation -> gradient of the coarser level's output
-        const Tensor& gprev = l < 3 ? net.gd2[l + 1] : net.gb2;
-        const size_t n8 = (size_t)N * (h / 2) * (w / 2) * (net.U[l] / 8);
-        hipLaunchKernelGGL(k_up_bwd, dim3(blocks(n8)), dim3(256), 0, s, net.gcat[l].p, net.gcat[l].C, gprev.p, N,
-                           h / 2, w / 2, net.U[l]);
+        // the up part of the concatenation: the coarser level's output and its gradient
+        const Tensor &prev = l < 3 ? net.d2[l + 1] : net.b2, &gprev = l < 3 ? net.gd2[l + 1] : net.gb2;
+        wgrad_of(li, net.cat[l], net.gd1[l], &prev);
+        rc |= conv_bwd_data(li, net.gd1[l], net.gcat[l], &net.cat[l], N, h, w, s, &prev, &gprev);
     }
     // bottleneck
     const uint32_t h4 = H >> 4, w4 = W >> 4;

@@ -1423,6 +1423,7 @@ int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, const float* l
         wgrad_of(2 * l, in, net.ga[l]);
         if (l > 0) rc |= conv_bwd_data(2 * l, net.ga[l], net.gpool[l - 1], nullptr, N, h, w, s);
     }
+    if (rc != 0) return -1;   // no step on gradients that are not there
     hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(net.wg_blocks), dim3(kWgThreads), 0, s, net.wg);
     AdamArgs o{};
     if (lr) {
@@ -1436,7 +1437,7 @@ int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, const float* l
         hipLaunchKernelGGL(k_wgrad_reduce<false>, dim3(blocks(net.nparam)), dim3(256), 0, s, net.part, net.parts,
                            (uint32_t)net.nparam, net.grads, o);
     }
-    return rc == 0 && hipGetLastError() == hipSuccess ? 0 : -1;
+    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int ensure_io(size_t bytes) {

@@ -72,6 +72,7 @@ struct State {
     HitRecord* hits = nullptr;
     float4* rad = nullptr;
     uint32_t* bgra = nullptr;
+    uint32_t* shown = nullptr;   // page-locked, kShownBytes: small frames are encoded straight into it
     float4* gbuf = nullptr;     // optional G-buffer, 2 x float4 per pixel
     float4* gsamp = nullptr;    // its per-sample state, 2 x float4 per path
     size_t gsamp_cap = 0;
@@ -259,6 +260,16 @@ int ensure_frame_buffers() {
     }
     g.frame_cap = n;
     return 0;
+}
+
+// Frames of up to kShownBytes go to the host as the encoding kernel's own stores, without a copy after it.
+constexpr size_t kShownBytes = (size_t)4 << 20;
+bool ensure_shown() {
+    if (!g.shown && hipHostMalloc(&g.shown, kShownBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        g.shown = nullptr;
+    }
+    return g.shown != nullptr;
 }
 
 int grow_instances(uint32_t n) {
@@ -675,7 +686,7 @@ void cleanup(void) {
     vt_lbvh_free(g.bvh);
     hipHostFree(g.inst_host);
     hipFree(g.vol_table); hipFree(g.staging);
-    hipFree(g.hits); hipFree(g.rad); hipFree(g.bgra); hipFree(g.gbuf); hipFree(g.gsamp); hipFree(g.stats); hipFree(g.srgb_dec); hipFree(g.srgb_thr);
+    hipFree(g.hits); hipFree(g.rad); hipFree(g.bgra); hipHostFree(g.shown); hipFree(g.gbuf); hipFree(g.gsamp); hipFree(g.stats); hipFree(g.srgb_dec); hipFree(g.srgb_thr);
     hipFree(g.wave_mem);
     for (uint32_t k = 0; k < kMaxChunks; ++k) {
         if (g.xstream[k]) hipStreamSynchronize(g.xstream[k]);
@@ -856,6 +867,14 @@ int32_t vt_read_bgra8(uint32_t* dst, uint64_t bytes) {
         Guard G;
         if (!g.inited || !g.have_frame) return -1;
         uint32_t n = g.last_frame.width * g.last_frame.height;
+        const size_t need = (size_t)n * 4;
+        if (need <= kShownBytes && dst && bytes >= need && ensure_shown()) {
+            if (vt_encode_srgb8(reinterpret_cast<const float4*>(g.rad), g.shown, n, g.stream) != 0 ||
+                hipStreamSynchronize(g.stream) != hipSuccess)
+                return -1;
+            std::memcpy(dst, g.shown, need);
+            return 0;
+        }
         if (vt_encode_srgb8(reinterpret_cast<const float4*>(g.rad), g.bgra, n, g.stream) != 0) return -1;
     }
     return read_frame(g.bgra, dst, bytes, 4);

@@ -1849,10 +1849,15 @@ __global__ __launch_bounds__(kBlock) void k_render0(const FrameGPU F, const Scen
     if (ST) ctr.flush(stats);
 }
 
-__global__ void k_encode_srgb8(const float4* rad, uint32_t* out, uint32_t n, const float* thr) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// Radiance -> B8G8R8A8, four pixels a thread.  Bound by the latency of the eight dependent steps of a search
+// (of thresholds in LDS, twelve searches side by side) and, where out is host memory, by the link.
+__global__ __launch_bounds__(256) void k_encode_srgb8(const float4* __restrict__ rad, uint32_t* __restrict__ out, uint32_t n,
+                                                      const float* __restrict__ thresholds) {
+    __shared__ float thr[256];
+    if (threadIdx.x < 255u) thr[threadIdx.x] = thresholds[threadIdx.x];
+    __syncthreads();
+    const uint32_t i = 4u * (blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= n) return;
-    float4 c = rad[i];
     auto enc = [&](float v) -> uint32_t {
         uint32_t lo = 0, hi = 255;  // smallest k with v < thr[k], thr has 255 entries
         while (lo < hi) {
@@ -1862,9 +1867,19 @@ __global__ void k_encode_srgb8(const float4* rad, uint32_t* out, uint32_t n, con
         }
         return lo;
     };
-    uint32_t a = (uint32_t)fminf(fmaxf(c.w * 255.0f + 0.5f, 0.0f), 255.0f);
-    // B8G8R8A8 byte order: b, g, r, a
-    out[i] = enc(c.z) | (enc(c.y) << 8) | (enc(c.x) << 16) | (a << 24);
+    uint32_t o[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+        const float4 c = rad[min(i + k, n - 1u)];
+        const uint32_t a = (uint32_t)fminf(fmaxf(c.w * 255.0f + 0.5f, 0.0f), 255.0f);
+        // B8G8R8A8 byte order: b, g, r, a
+        o[k] = enc(c.z) | (enc(c.y) << 8) | (enc(c.x) << 16) | (a << 24);
+    }
+    if (i + 3u < n) {
+        *reinterpret_cast<uint4*>(out + i) = make_uint4(o[0], o[1], o[2], o[3]);
+    } else {
+        for (uint32_t k = 0; i + k < n; ++k) out[i + k] = o[k];
+    }
 }
 
 }  // namespace
@@ -2185,6 +2200,6 @@ int vt_trace_launch(const FrameGPU& F, const SceneGPU& S, HitRecord* hits, float
 
 int vt_encode_srgb8(const float4* rad, uint32_t* bgra, uint32_t n, hipStream_t s) {
     if (!g_srgb_thr) return -1;
-    hipLaunchKernelGGL(k_encode_srgb8, dim3((n + 255) / 256), dim3(256), 0, s, rad, bgra, n, g_srgb_thr);
+    hipLaunchKernelGGL(k_encode_srgb8, dim3((n + 1023) / 1024), dim3(256), 0, s, rad, bgra, n, g_srgb_thr);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

@@ -1,4 +1,4 @@
-"""GPU: copies to and from ordinary host memory, at the sizes where they change form (4 MB out, 12 MB in,
+"""GPU: copies to and from ordinary host memory, at the sizes where they change form (4 MB out, 24 MB in,
 chunks of 512 KB to 2 MB over several threads): the bytes equal those of a copy through page-locked
 memory, also when two threads read at once and after the renderer was reset."""
 import threading
@@ -50,7 +50,7 @@ def test_two_threads_read_at_once():
     assert all(np.array_equal(g.view(np.uint32), want.view(np.uint32)) for g in got)
 
 
-@pytest.mark.parametrize("d", [191, 192, 211])   # 256 x 256 x d bytes around 12 MB
+@pytest.mark.parametrize("d", [191, 192, 211, 383, 384, 421])   # 256 x 256 x d bytes around 12 and 24 MB
 def test_volume_round_trip(d):
     r = R.reset_renderer()
     idx = scenes.gen_volume((256, 256, d), 3, 0.3)

@@ -19,17 +19,18 @@
 //                    from an LDS tile of the NHWC input with its halo, B fragments 8 channels of a
 //                    [co][tap][ci] weight row.  Weights are the first MFMA operand, so a lane's
 //                    outputs are 4 consecutive channels of one pixel.
-//   k_conv3x3_res    persistent workgroups of 8 waves with the layer's weights resident in LDS, 16 x 16
-//                    pixel tiles, the next tile fetched into registers during the current one, a
-//                    software-pipelined K loop with no barrier: inputs of up to 96 channels
-//                    where weights and a tile fit in 160 KiB and there are tiles enough.
+//   k_conv3x3_res    persistent workgroups, each wave with the weights of 16 output channels in registers,
+//                    16 x 8 (or 16 x 16) pixel tiles double-buffered in LDS: inputs of up to 96
+//                    channels (64 for 80 and 96 outputs) where every CU has two tiles.
 //   k_conv3x3_split  16 x 8 pixel tiles with the output channels split over workgroups, weights from L2
 //                    into registers several K steps ahead: everything else.
-//                    Both can pool their output (2x2 mean) in the epilogue and read the decoder's
-//                    upsampled channels from the lower level in their staging.
-//   k_conv3x3_wgrad  dW[co][tap][ci] = sum_p dY[p][co] X[p+tap][ci] over a chunk of pixel tiles,
-//                    all nine taps of a block of input channels in registers, the operands
+//                    Both can pool their output (2x2 mean) in the epilogue, read the decoder's
+//                    upsampled channels from the lower level in their staging, and sum the gradient
+//                    of an upsampling in their epilogue.
+//   k_conv3x3_wgrad  dW[co][tap][ci] = sum_p dY[p][co] X[p+tap][ci] of all layers, over chunks of pixel
+//                    tiles, all nine taps of a block of input channels in registers, the operands
 //                    transposed on the way out of LDS; dbias in the same pass.
+//   k_wgrad_reduce   the chunks' sums added up; in training with the Adam step and the BF16 weights.
 //   pooling (backward), feature, loss and weight-layout kernels are element-wise.
 #include <hip/hip_runtime.h>
 
@@ -49,7 +50,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kInCh = 16;       // input feature channels (10 used)
 constexpr int kOutCh = 3;
 constexpr int kLayers = 19;
-constexpr int kMaxWidth = 96;   // widest layer (accumulators of the weight-gradient kernel)
+constexpr int kMaxWidth = 96;   // widest layer (six groups of 16 output channels)
 constexpr float kAlbedoEps = 0.01f;  // demodulation: irradiance = radiance / (albedo + eps)
 constexpr float kLogMax = 16.0f;     // clamp of the predicted log irradiance
 

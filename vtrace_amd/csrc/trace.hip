@@ -1522,49 +1522,53 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
             const ReqGPU& Rq = reqs[ri];
             const SceneGPU& S = Rq.S;
             const FrameGPU& F = Rq.F;
-            const InstanceGPU* I = &S.inst[origin];
-            const VolumeDesc V0 = inst_vol(S, I);   // (its loads issued before the sampling below)
-            V3 X, n;
-            surface_frame(&S.inst[sf.inst], sf.p, sf.face, X, n);
-            Rng r{sf.rng};
-            w = V3{F.sun[0], F.sun[1], F.sun[2]};
-            if (is_bounce) {
-                if (depth == 0) {
-                    val[0] = 1.0f * srgb_dec[sf.rgba & 255u];
-                    val[1] = 1.0f * srgb_dec[(sf.rgba >> 8) & 255u];
-                    val[2] = 1.0f * srgb_dec[(sf.rgba >> 16) & 255u];
+            // a batch is launched as deep as its longest paths (a captured one as deep as the loop's): a
+            // request of fewer bounces has no ray here, its lane takes another item
+            busy = ONE || !is_bounce || depth < (F.mode == 2 ? F.max_bounces : 0u);
+            if (busy) {
+                const InstanceGPU* I = &S.inst[origin];
+                const VolumeDesc V0 = inst_vol(S, I);   // (its loads issued before the sampling below)
+                V3 X, n;
+                surface_frame(&S.inst[sf.inst], sf.p, sf.face, X, n);
+                Rng r{sf.rng};
+                w = V3{F.sun[0], F.sun[1], F.sun[2]};
+                if (is_bounce) {
+                    if (depth == 0) {
+                        val[0] = 1.0f * srgb_dec[sf.rgba & 255u];
+                        val[1] = 1.0f * srgb_dec[(sf.rgba >> 8) & 255u];
+                        val[2] = 1.0f * srgb_dec[(sf.rgba >> 16) & 255u];
+                    } else {
+                        const float4 b4 = wf.br[path];
+                        val[0] = b4.x; val[1] = b4.y; val[2] = b4.z;
+                    }
+                    cosine_dir(r, n, w);
                 } else {
-                    const float4 b4 = wf.br[path];
-                    val[0] = b4.x; val[1] = b4.y; val[2] = b4.z;
+                    val[0] = sf.c[0]; val[1] = sf.c[1]; val[2] = sf.c[2];
                 }
-                cosine_dir(r, n, w);
-            } else {
-                val[0] = sf.c[0]; val[1] = sf.c[1]; val[2] = sf.c[2];
-            }
-            rng = r.s;
-            O = X;
-            inv_d = V3{1.0f / w.x, 1.0f / w.y, 1.0f / w.z};
-            ctr.ray();
-            best.hit = false;
-            best.inst = VT_EMPTY;
-            best.tn = INFINITY;
-            stk.sp = 0;
-            inst = origin;
-            tn = 0.0f;
-            face0 = (uint8_t)sf.face;
-            const int fa0 = (int)(sf.face >> 1), off0 = (sf.face & 1u) == 0u ? -1 : 1;
-            const int v0[3] = {(int)sf.v[0] + (fa0 == 0 ? off0 : 0), (int)sf.v[1] + (fa0 == 1 ? off0 : 0),
-                               (int)sf.v[2] + (fa0 == 2 ? off0 : 0)};
-            float inv[12];
+                rng = r.s;
+                O = X;
+                inv_d = V3{1.0f / w.x, 1.0f / w.y, 1.0f / w.z};
+                ctr.ray();
+                best.hit = false;
+                best.inst = VT_EMPTY;
+                best.tn = INFINITY;
+                stk.sp = 0;
+                inst = origin;
+                tn = 0.0f;
+                face0 = (uint8_t)sf.face;
+                const int fa0 = (int)(sf.face >> 1), off0 = (sf.face & 1u) == 0u ? -1 : 1;
+                const int v0[3] = {(int)sf.v[0] + (fa0 == 0 ? off0 : 0), (int)sf.v[1] + (fa0 == 1 ? off0 : 0),
+                                   (int)sf.v[2] + (fa0 == 2 ? off0 : 0)};
+                float inv[12];
 #pragma unroll
-            for (int k = 0; k < 12; ++k) inv[k] = gld(&I->inv[k]);
-            mdir = xf34(inv, w, 0.0f);
-            ctr.instance();
-            box_walk_begin(V0, sf.p, v0, mdir, W);
-            busy = true;
-            walking = true;
+                for (int k = 0; k < 12; ++k) inv[k] = gld(&I->inv[k]);
+                mdir = xf34(inv, w, 0.0f);
+                ctr.instance();
+                box_walk_begin(V0, sf.p, v0, mdir, W);
+                walking = true;
+            }
         }
-        if (__ballot(busy) == 0ull) break;   // no items left and none in flight
+        if (__ballot(busy) == 0ull && (ONE || !more)) break;   // no items left and none in flight
         // -- the walk loop: every walking lane steps until too few walk --
         for (;;) {
             if (walking) walking = box_walk_step<ST>(W, ctr, mslot);

@@ -1424,8 +1424,10 @@ int backward(uint32_t N, uint32_t H, uint32_t W, float* loss_dev, const float* l
         wgrad_of(2 * l, in, net.ga[l]);
         if (l > 0) rc |= conv_bwd_data(2 * l, net.ga[l], net.gpool[l - 1], nullptr, N, h, w, s);
     }
-    if (rc != 0) return -1;   // no step on gradients that are not there
+    if (rc != 0) return -1;
     hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(net.wg_blocks), dim3(kWgThreads), 0, s, net.wg);
+    // no step on gradients that are not there: where a launch above failed, the partial sums are an earlier pass's
+    if (hipGetLastError() != hipSuccess) return -1;
     AdamArgs o{};
     if (lr) {
         net.adam_t += 1;

@@ -41,3 +41,40 @@ def train_with_a_failed_launch(hip, what, nth):
                                       ("k_conv3x3_split", 20), ("k_conv3x3_split", 37), ("k_conv3x3_wgrad", 1)])
 def test_no_update_after_a_failed_launch(fake, what, nth):
     fake_hip.child(fake, "test_host_calls", "train_with_a_failed_launch", what, nth)
+
+
+# ---- instance records: the GPU reads the caller's buffer in place, so it is handed out again when that is over ----
+def commit_and_reopen(hip, n, refit, fail):
+    from vtrace_amd import renderer
+    r = renderer.get_renderer()
+    recs = np.zeros((n, 16), np.float32)
+    r.set_instances(recs)
+    hip.clear()
+    if fail:
+        hip.fail(fail)
+    recs[:, 12] = 1 + np.arange(n)
+    if fail:
+        with pytest.raises(renderer.RendererError):
+            (r.refit_instances if refit else r.set_instances)(recs)
+        assert _count(hip, "FAILED") == 1
+    else:
+        (r.refit_instances if refit else r.set_instances)(recs)
+    calls = [c for c in hip.lines() if c.startswith(("launch", "record", "attribute"))]
+    hip.clear()
+    assert r.lib.start_update_instances(n)
+    waits = [c.split()[2] for c in hip.lines() if c.startswith("sync event")]
+    reads = [k for k, c in enumerate(calls) if "k_instance_prep" in c or "k_lbvh_one" in c]
+    assert len(reads) == 1 and len(waits) == 1
+    # behind the launch that reads them, right behind it where much follows
+    marks = [k for k, c in enumerate(calls) if f"record event {waits[0]}" in c]
+    assert len(marks) == 1 and marks[0] > reads[0], calls
+    assert marks[0] == reads[0] + 1 or (refit and n <= 8192), calls
+
+
+@pytest.mark.parametrize("n,refit,fail", [(1, False, None), (300, False, None), (3000, False, None), (9000, False, None),
+                                          (40000, False, None), (5, True, None), (3000, True, None), (9000, True, None),
+                                          # a later launch, or the permission for its LDS, fails
+                                          (3000, False, "k_karras"), (4000, False, "attribute"), (40000, False, "k_sort_hist"),
+                                          (3000, True, "k_refit"), (9000, True, "k_refit")])
+def test_records_are_free_once_they_are_read(fake, n, refit, fail):
+    fake_hip.child(fake, "test_host_calls", "commit_and_reopen", n, refit, fail)

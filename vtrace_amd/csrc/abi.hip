@@ -56,7 +56,7 @@ struct State {
     uint32_t* depth_host = nullptr;
     hipEvent_t depth_ready = nullptr;
     bool depth_pending = false;
-    hipEvent_t inst_copied = nullptr;
+    hipEvent_t inst_read = nullptr;   // the last build or refit has read inst_host
     std::vector<float> inst_prev;     // records of the last build
     size_t inst_prev_vols = 0;        // textures known at the last build (validity of the records)
     uint64_t lbvh_builds = 0;
@@ -276,7 +276,7 @@ int grow_instances(uint32_t n) {
     if (n <= g.inst_capacity && g.inst_host) return 0;
     uint32_t cap = 1;
     while (cap < n + 1) cap *= 2;  // round_up_p2(n + 1), lib/memory.c:191
-    if (g.inst_copied) hipEventSynchronize(g.inst_copied);
+    if (g.inst_read) hipEventSynchronize(g.inst_read);
     hipHostFree(g.inst_host);
     g.inst_host = nullptr;
     hipError_t e;
@@ -548,7 +548,7 @@ uint64_t entry(void) {
     if ((e = hipSetDevice(g.device)) != hipSuccess ||
         (e = hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipEventCreate(&g.ev0)) != hipSuccess || (e = hipEventCreate(&g.ev1)) != hipSuccess ||
-        (e = hipEventCreateWithFlags(&g.inst_copied, hipEventDisableTiming)) != hipSuccess ||
+        (e = hipEventCreateWithFlags(&g.inst_read, hipEventDisableTiming)) != hipSuccess ||
         (e = hipEventCreateWithFlags(&g.depth_ready, hipEventDisableTiming)) != hipSuccess ||
         (e = hipHostMalloc(&g.depth_host, sizeof(uint32_t), hipHostMallocDefault)) != hipSuccess ||
         (e = hipMalloc(&g.vol_table, (size_t)kMaxTextures * sizeof(VolumeDesc))) != hipSuccess ||
@@ -695,7 +695,7 @@ void cleanup(void) {
         if (g.xstream[k]) hipStreamDestroy(g.xstream[k]);
     }
     for (uint32_t k = 0; k < kMaxChunks; ++k) hipFree(g.xgsamp[k]);
-    hipEventDestroy(g.ev0); hipEventDestroy(g.ev1); hipEventDestroy(g.inst_copied); hipEventDestroy(g.depth_ready);
+    hipEventDestroy(g.ev0); hipEventDestroy(g.ev1); hipEventDestroy(g.inst_read); hipEventDestroy(g.depth_ready);
     hipHostFree(g.depth_host);
     hipStreamDestroy(g.stream);
     vt_trace_set_tables(nullptr, nullptr);
@@ -728,7 +728,7 @@ float* start_update_instances(uint32_t instance_count) {
     if (!g.inited) return nullptr;
     if (instance_count == 0) instance_count = 1;  // lib/memory.c:236
     if (instance_count > g.inst_capacity && grow_instances(instance_count) != 0) return nullptr;
-    hipEventSynchronize(g.inst_copied);  // previous commit has left the staging buffer
+    hipEventSynchronize(g.inst_read);  // the previous commit has been read
     return g.inst_host;
 }
 
@@ -747,11 +747,10 @@ int32_t end_update_instances(uint32_t instance_count) {
         std::memcmp(g.inst_prev.data(), g.inst_host, nrec * 4) == 0)
         return 0;
     g.inst_prev.clear();
-    if (vt_lbvh_build(g.bvh, g.inst_host, instance_count, g.vol_table, (uint32_t)g.vols.size(), g.stream) != 0) {
+    if (vt_lbvh_build(g.bvh, g.inst_host, instance_count, g.vol_table, (uint32_t)g.vols.size(), g.stream, g.inst_read) != 0) {
         set_err("lbvh build", hipGetLastError());
         return -1;
     }
-    hipEventRecord(g.inst_copied, g.stream);
     // the tree depth selects the traversal-stack variant (LDS stack or a deep private stack);
     // it is read by the next frame (scene_gpu), so the update does not wait for the build.  A tree of
     // n leaves is at most n - 1 deep: up to kFlatInstances that bound fits the LDS stack, and the
@@ -783,11 +782,10 @@ int32_t vt_refit_instances(uint32_t instance_count) {
         set_err("vt_refit_instances: the instance count differs from the last build");
         return -1;
     }
-    if (vt_lbvh_refit(g.bvh, g.inst_host, instance_count, g.vol_table, (uint32_t)g.vols.size(), g.stream) != 0) {
+    if (vt_lbvh_refit(g.bvh, g.inst_host, instance_count, g.vol_table, (uint32_t)g.vols.size(), g.stream, g.inst_read) != 0) {
         set_err("lbvh refit", hipGetLastError());
         return -1;
     }
-    hipEventRecord(g.inst_copied, g.stream);
     g.inst_prev.assign(g.inst_host, g.inst_host + (size_t)instance_count * 16);
     g.inst_prev_vols = g.vols.size();
     return 0;

@@ -38,6 +38,10 @@ constexpr int kRefitLeaves = 4;           // leaves per thread: kRefitOneMax / 1
 constexpr uint32_t kRankMax = 16384;
 constexpr uint32_t kRankKeys = 64;        // keys a workgroup ranks
 constexpr uint32_t kPrepThreads = 256;
+// The mark behind a refit's first launch costs 5 us (of 30 for 16 instances, of 100 for 8000), which a program
+// that draws a frame between refits has nothing for; three refits in a row without one take 112 us marked
+// late and 92 marked early for 16, 302 and 272 for 8000, 573 and 499 for 20000.
+constexpr uint32_t kMarkLateMax = 8192;
 
 __device__ inline float gmin(float x, float y) { return (y < x) ? y : x; }
 __device__ inline float gmax(float x, float y) { return (x < y) ? y : x; }
@@ -675,17 +679,19 @@ void vt_lbvh_free(LbvhWork& w) {
 // Refit: new records for the same n instances keep the last build's topology (leaf order and
 // parents); instance data and leaf boxes are recomputed, internal boxes rebuilt bottom-up.
 int vt_lbvh_refit(LbvhWork& w, const float* records_dev, uint32_t n, const VolumeDesc* vols_dev, uint32_t nvol,
-                  hipStream_t s) {
+                  hipStream_t s, hipEvent_t read) {
     if (n == 0 || n > w.cap || !w.inst) return -1;
     const uint32_t tb = kPrepThreads, nb = (n + tb - 1) / tb;
     BvhNode* leaves_tmp = reinterpret_cast<BvhNode*>(w.cen + 3 * (size_t)w.cap);
     hipLaunchKernelGGL(k_instance_prep, dim3(nb), dim3(tb), 0, s, records_dev, n, vols_dev, nvol, w.inst, leaves_tmp,
                        w.cen, static_cast<float*>(nullptr));
+    if (read && n > kMarkLateMax) hipEventRecord(read, s);
     hipLaunchKernelGGL(k_leaves, dim3(nb), dim3(tb), 0, s, w.vals[0], n, leaves_tmp, w.nodes);
     if (n > 1) {
         hipLaunchKernelGGL(k_zero_counters, dim3(nb), dim3(tb), 0, s, w.counters, n - 1);
         hipLaunchKernelGGL(k_refit, dim3(nb), dim3(tb), 0, s, n, w.nodes, w.parent, w.counters);
     }
+    if (read && n <= kMarkLateMax) hipEventRecord(read, s);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -712,7 +718,7 @@ static bool allow_lds(K kernel, size_t lds) {
 }
 
 int vt_lbvh_build(LbvhWork& w, const float* records_dev, uint32_t n, const VolumeDesc* vols_dev, uint32_t nvol,
-                  hipStream_t s) {
+                  hipStream_t s, hipEvent_t read) {
     if (n == 0) return 0;
     if (vt_lbvh_reserve(w, n) != 0) return -1;
     const uint32_t tb = kPrepThreads, nb = (n + tb - 1) / tb;
@@ -724,11 +730,13 @@ int vt_lbvh_build(LbvhWork& w, const float* records_dev, uint32_t n, const Volum
         if (!allow_lds(&k_lbvh_one, lds)) return -1;
         hipLaunchKernelGGL(k_lbvh_one, dim3(1), dim3(P), lds, s, records_dev, n, vols_dev, nvol, w.inst, leaves_tmp,
                            w.cen, w.vals[0], w.nodes, w.parent, w.depth);
+        if (read) hipEventRecord(read, s);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
     const bool rank = n <= kRankMax;
     hipLaunchKernelGGL(k_instance_prep, dim3(nb), dim3(tb), 0, s, records_dev, n, vols_dev, nvol, w.inst, leaves_tmp,
                        w.cen, rank ? w.bounds : static_cast<float*>(nullptr));
+    if (read) hipEventRecord(read, s);
     if (rank) {
         const size_t lds = ((size_t)n + 63) / 64 * 256;
         if (!allow_lds(&k_rank_sort, lds) || !allow_lds(&k_karras<true>, lds)) return -1;

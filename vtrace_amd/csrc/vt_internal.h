@@ -40,12 +40,12 @@ int vt_brick_volume(BrickWork& w, const uint8_t* dense_dev, uint32_t fmt, const 
 void vt_brick_free(BrickWork& w);
 int vt_debrick(const VolumeDesc& v, uint8_t* dense_dev, hipStream_t s);
 
-// lbvh.hip: builds InstanceGPU records and the LBVH from n ABI records on the device.
-// Copies to and from the caller's host memory (hostcopy.hip).
+// hostcopy.hip: copies to and from the caller's host memory.
 hipError_t vt_copy_in(void* dev, const void* host, size_t bytes, hipStream_t s);
 hipError_t vt_copy_out(void* host, const void* dev, size_t bytes, hipStream_t s);
 void vt_copy_release();
 
+// lbvh.hip: builds InstanceGPU records and the LBVH from n ABI records, in device or page-locked memory.
 struct LbvhWork {
     uint32_t cap = 0;           // instances the buffers hold
     InstanceGPU* inst = nullptr;
@@ -61,10 +61,12 @@ struct LbvhWork {
 };
 int vt_lbvh_reserve(LbvhWork& w, uint32_t n);
 void vt_lbvh_free(LbvhWork& w);
+// read (optional): recorded behind the launch that reads the records, the first (a small refit: behind its last),
+// also where a later one fails: passed, the records may be written anew
 int vt_lbvh_build(LbvhWork& w, const float* records_dev, uint32_t n, const VolumeDesc* vols_dev, uint32_t nvol,
-                  hipStream_t s);
+                  hipStream_t s, hipEvent_t read = nullptr);
 int vt_lbvh_refit(LbvhWork& w, const float* records_dev, uint32_t n, const VolumeDesc* vols_dev, uint32_t nvol,
-                  hipStream_t s);
+                  hipStream_t s, hipEvent_t read = nullptr);
 
 // trace.hip: wavefront path state and queues (one block of device memory, see vt_wave_bind)
 struct WaveBuffers {

@@ -78,3 +78,24 @@ def commit_and_reopen(hip, n, refit, fail):
                                           (3000, True, "k_refit"), (9000, True, "k_refit")])
 def test_records_are_free_once_they_are_read(fake, n, refit, fail):
     fake_hip.child(fake, "test_host_calls", "commit_and_reopen", n, refit, fail)
+
+
+# ---- a tree that could not be built is not traced ----------------------------------------------
+def commit_fails(hip, n, fail):
+    from vtrace_amd import renderer
+    r = renderer.get_renderer()
+    r.set_instances(np.ones((3, 16), np.float32))
+    assert r.lib.vt_instance_count() == 3
+    r.lib.start_update_instances(n)
+    hip.fail(fail)
+    assert r.lib.end_update_instances(n) == -1 and _count(hip, "FAILED") == 1
+    assert r.lib.vt_instance_count() == 0
+    assert r.lib.vt_read_lbvh(None, 0, None, 0) == -1
+    r.set_instances(np.ones((n, 16), np.float32))
+    assert r.lib.vt_instance_count() == n
+
+
+# memory for the larger tree, a launch in the middle of a build, the copy of the tree's depth behind it
+@pytest.mark.parametrize("n,fail", [(2000, "malloc"), (2000, "copy out"), (2000, "k_karras"), (40000, "k_sort_scan"), (2, "k_lbvh_one")])
+def test_no_instances_after_a_failed_build(fake, n, fail):
+    fake_hip.child(fake, "test_host_calls", "commit_fails", n, fail)

@@ -747,6 +747,7 @@ int32_t end_update_instances(uint32_t instance_count) {
         std::memcmp(g.inst_prev.data(), g.inst_host, nrec * 4) == 0)
         return 0;
     g.inst_prev.clear();
+    g.inst_count = 0;   // if this fails: the old tree may be overwritten or freed, nothing is traced until the next commit
     if (vt_lbvh_build(g.bvh, g.inst_host, instance_count, g.vol_table, (uint32_t)g.vols.size(), g.stream, g.inst_read) != 0) {
         set_err("lbvh build", hipGetLastError());
         return -1;

@@ -764,6 +764,7 @@ int32_t end_update_instances(uint32_t instance_count) {
         if (e == hipSuccess) e = hipEventRecord(g.depth_ready, g.stream);
         if (e != hipSuccess) {
             set_err("lbvh depth", e);
+            (void)hipGetLastError();   // (the next build would take it for its own)
             return -1;
         }
         g.depth_pending = true;

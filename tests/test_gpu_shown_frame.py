@@ -39,3 +39,31 @@ def test_shown_frame_bytes(width, height):
         assert np.array_equal(r.bgra8(), _encode(r.radiance()))
     small = np.zeros(width * height - 1, np.uint32)
     assert r.lib.vt_read_bgra8(small.ctypes.data, small.nbytes) != 0   # too small a buffer stays refused
+
+
+@pytest.mark.parametrize("width,height", [(3, 1), (67, 31), (1024, 1024), (1025, 1024)])
+def test_shown_frame_into_page_locked_memory(width, height):
+    """The same bytes as into ordinary memory, the memory behind them untouched."""
+    import torch
+
+    sc = scenes.multi_volume_scene(count=3, n=32, world=160, seed=8, width=width, height=height, spp=1, max_bounces=0)
+    r = R.reset_renderer()
+    R.load_scene(r, sc)
+    r.render(sc.P, sc.C)
+    n = width * height
+    mem = torch.full((n + 8,), -1, dtype=torch.int32, pin_memory=True).numpy()
+    print(f"case: shown frame {width}x{height} into page-locked memory", flush=True)
+    assert r.lib.vt_read_bgra8(mem.ctypes.data, 4 * n) == 0
+    assert np.array_equal(mem[:n].view(np.uint32).reshape(height, width), r.bgra8()) and np.all(mem[n:] == -1)
+
+
+@pytest.mark.parametrize("sky", [(float("nan"), float("inf"), -1.0), (0.0, -0.0, 1e30), (1.0, 0.99999994, float("-inf"))])
+def test_shown_frame_of_extreme_radiance(sky):
+    """NaN and what lies below the first threshold show as 0, what lies above the last as 255."""
+    r = R.reset_renderer()
+    r.set_params(scenes.RenderParams(6, 3, viewport_square=0, mode=1, sky=sky))
+    r.render(scenes.perspective(scenes.FOV, 2.0), scenes.look_at((0.0, 0.0, 9.0), (0.0, 0.0, 0.0)))
+    want = [0 if not v > 0.0 else 255 for v in sky]
+    print(f"case: shown frame, sky {sky}", flush=True)
+    got = r.bgra8()
+    assert np.all(got == np.uint32(want[2] | want[1] << 8 | want[0] << 16 | 0xFF000000)), hex(int(got[0, 0]))

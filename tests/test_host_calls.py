@@ -99,3 +99,31 @@ def commit_fails(hip, n, fail):
 @pytest.mark.parametrize("n,fail", [(2000, "malloc"), (2000, "copy out"), (2000, "k_karras"), (40000, "k_sort_scan"), (2, "k_lbvh_one")])
 def test_no_instances_after_a_failed_build(fake, n, fail):
     fake_hip.child(fake, "test_host_calls", "commit_fails", n, fail)
+
+
+# ---- reading the shown frame: into any memory that a copy takes -----------------------------------
+def read_shown(hip, kind, width, height):
+    import ctypes
+
+    from vtrace_amd import renderer, scenes
+    r = renderer.get_renderer()
+    r.set_params(scenes.RenderParams(width, height, mode=0))
+    r.render(scenes.perspective(1.0, 1.0), scenes.look_at((0.0, 0.0, 9.0), (0.0, 0.0, 0.0)))
+    n = width * height * 4
+    mem = np.zeros(n, np.uint8)
+    dst = {"ordinary": lambda: mem.ctypes.data, "page_locked": lambda: hip.page_locked(n),
+           "device": lambda: hip.device(n)}[kind]()
+    r.lib.vt_read_bgra8(dst, n)   # (what is allocated on first use)
+    hip.clear()
+    assert r.lib.vt_read_bgra8(dst, n) == 0
+    copies = [c for c in hip.lines() if c.startswith("copy")]
+    if kind == "ordinary" and n <= 4 << 20:
+        assert copies == [], copies
+    elif kind != "ordinary":   # by the copy engine, into the caller's memory
+        assert len(copies) == 1 and ctypes.c_void_p(dst).value == int(copies[0].split()[2], 16), copies
+
+
+@pytest.mark.parametrize("kind", ["ordinary", "page_locked", "device"])
+@pytest.mark.parametrize("width,height", [(64, 48), (1024, 1024), (1025, 1024)])
+def test_shown_frame_into_any_memory(fake, kind, width, height):
+    fake_hip.child(fake, "test_host_calls", "read_shown", kind, width, height)

@@ -262,7 +262,9 @@ int ensure_frame_buffers() {
     return 0;
 }
 
-// Frames of up to kShownBytes go to the host as the encoding kernel's own stores, without a copy after it.
+// Frames of up to kShownBytes go to ordinary host memory as the encoding kernel's own stores, without a transfer
+// after it: 640 x 480 119 -> 108 us, 1280 x 720 282 -> 268.  Into page-locked memory the transfer goes
+// straight to its place, where this would add a copy by the host (46 us against 85, and 95 against 222).
 constexpr size_t kShownBytes = (size_t)4 << 20;
 bool ensure_shown() {
     if (!g.shown && hipHostMalloc(&g.shown, kShownBytes, hipHostMallocDefault) != hipSuccess) {
@@ -868,7 +870,7 @@ int32_t vt_read_bgra8(uint32_t* dst, uint64_t bytes) {
         if (!g.inited || !g.have_frame) return -1;
         uint32_t n = g.last_frame.width * g.last_frame.height;
         const size_t need = (size_t)n * 4;
-        if (need <= kShownBytes && dst && bytes >= need && ensure_shown()) {
+        if (need <= kShownBytes && dst && bytes >= need && vt_copy_pageable(dst, need) && ensure_shown()) {
             if (vt_encode_srgb8(reinterpret_cast<const float4*>(g.rad), g.shown, n, g.stream) != 0 ||
                 hipStreamSynchronize(g.stream) != hipSuccess)
                 return -1;

@@ -203,19 +203,9 @@ Engine* engine() {
     return g_engine = e;
 }
 
-// ordinary host memory, at both ends of the range
-bool pageable(const void* p, size_t bytes) {
-    for (const char* q : {static_cast<const char*>(p), static_cast<const char*>(p) + bytes - 1}) {
-        hipPointerAttribute_t at;
-        if (hipPointerGetAttributes(&at, q) != hipSuccess) (void)hipGetLastError();
-        else if (at.type != hipMemoryTypeUnregistered) return false;
-    }
-    return true;
-}
-
 // Staged copy; false if it has to be done otherwise.
 bool staged(void* host, void* dev, size_t bytes, bool in, hipStream_t s, hipError_t* rc) {
-    if (bytes < (in ? kMinIn : kMinOut) || !pageable(host, bytes)) return false;
+    if (bytes < (in ? kMinIn : kMinOut) || !vt_copy_pageable(host, bytes)) return false;
     std::lock_guard<std::mutex> own(g_copy_lock);
     Engine* e = engine();
     if (!e) return false;
@@ -249,6 +239,16 @@ bool staged(void* host, void* dev, size_t bytes, bool in, hipStream_t s, hipErro
 }
 
 }  // namespace
+
+// Ordinary host memory at both ends of the range: neither page-locked nor known to the device.
+bool vt_copy_pageable(const void* p, size_t bytes) {
+    for (const char* q : {static_cast<const char*>(p), static_cast<const char*>(p) + bytes - 1}) {
+        hipPointerAttribute_t at;
+        if (hipPointerGetAttributes(&at, q) != hipSuccess) (void)hipGetLastError();
+        else if (at.type != hipMemoryTypeUnregistered) return false;
+    }
+    return true;
+}
 
 // Host to device in the order of stream s; pageable source memory may be reused on return, page-locked
 // memory when the stream has passed the copy (as hipMemcpyAsync).

@@ -1854,7 +1854,8 @@ __global__ __launch_bounds__(kBlock) void k_render0(const FrameGPU F, const Scen
 }
 
 // Radiance -> B8G8R8A8, four pixels a thread.  Bound by the latency of the eight dependent steps of a search
-// (of thresholds in LDS, twelve searches side by side) and, where out is host memory, by the link.
+// (of thresholds in LDS; a fixed number of steps without branches, so that the twelve searches run side by side:
+// one after another they took 4 us more) and, where out is host memory, by the link.
 __global__ __launch_bounds__(256) void k_encode_srgb8(const float4* __restrict__ rad, uint32_t* __restrict__ out, uint32_t n,
                                                       const float* __restrict__ thresholds) {
     __shared__ float thr[256];
@@ -1862,14 +1863,11 @@ __global__ __launch_bounds__(256) void k_encode_srgb8(const float4* __restrict__
     __syncthreads();
     const uint32_t i = 4u * (blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= n) return;
-    auto enc = [&](float v) -> uint32_t {
-        uint32_t lo = 0, hi = 255;  // smallest k with v < thr[k], thr has 255 entries
-        while (lo < hi) {
-            uint32_t mid = (lo + hi) >> 1;
-            if (v >= thr[mid]) lo = mid + 1;
-            else hi = mid;
-        }
-        return lo;
+    auto enc = [&](float v) -> uint32_t {   // thresholds that v reaches, of 255 (NaN: none)
+        uint32_t k = 0;
+#pragma unroll
+        for (uint32_t s = 128u; s > 0u; s >>= 1) k += v >= thr[k + s - 1u] ? s : 0u;
+        return k;
     };
     uint32_t o[4];
 #pragma unroll

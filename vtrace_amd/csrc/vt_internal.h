@@ -43,6 +43,7 @@ int vt_debrick(const VolumeDesc& v, uint8_t* dense_dev, hipStream_t s);
 // hostcopy.hip: copies to and from the caller's host memory.
 hipError_t vt_copy_in(void* dev, const void* host, size_t bytes, hipStream_t s);
 hipError_t vt_copy_out(void* host, const void* dev, size_t bytes, hipStream_t s);
+bool vt_copy_pageable(const void* p, size_t bytes);
 void vt_copy_release();
 
 // lbvh.hip: builds InstanceGPU records and the LBVH from n ABI records, in device or page-locked memory.

@@ -101,8 +101,8 @@ def test_no_instances_after_a_failed_build(fake, n, fail):
     fake_hip.child(fake, "test_host_calls", "commit_fails", n, fail)
 
 
-# ---- reading the shown frame: into any memory that a copy takes -----------------------------------
-def read_shown(hip, kind, width, height):
+# ---- reading the shown frame: into any memory that a copy takes, and every failure has a text ------
+def read_shown(hip, kind, width, height, fail=None):
     import ctypes
 
     from vtrace_amd import renderer, scenes
@@ -115,6 +115,13 @@ def read_shown(hip, kind, width, height):
            "device": lambda: hip.device(n)}[kind]()
     r.lib.vt_read_bgra8(dst, n)   # (what is allocated on first use)
     hip.clear()
+    if fail:
+        r.lib.vt_read_bgra8(None, n)
+        before = r.error()
+        hip.fail(fail)
+        assert r.lib.vt_read_bgra8(dst, n) == -1 and _count(hip, "FAILED") == 1
+        assert r.error() != before and r.error().startswith("read-back")
+        return
     assert r.lib.vt_read_bgra8(dst, n) == 0
     copies = [c for c in hip.lines() if c.startswith("copy")]
     if kind == "ordinary" and n <= 4 << 20:
@@ -127,3 +134,9 @@ def read_shown(hip, kind, width, height):
 @pytest.mark.parametrize("width,height", [(64, 48), (1024, 1024), (1025, 1024)])
 def test_shown_frame_into_any_memory(fake, kind, width, height):
     fake_hip.child(fake, "test_host_calls", "read_shown", kind, width, height)
+
+
+@pytest.mark.parametrize("kind,fail", [("ordinary", "k_encode_srgb8"), ("ordinary", "sync stream"),
+                                       ("page_locked", "k_encode_srgb8"), ("page_locked", "copy out")])
+def test_failed_read_of_the_shown_frame_says_so(fake, kind, fail):
+    fake_hip.child(fake, "test_host_calls", "read_shown", kind, 64, 48, fail)

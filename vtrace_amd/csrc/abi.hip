@@ -871,13 +871,22 @@ int32_t vt_read_bgra8(uint32_t* dst, uint64_t bytes) {
         uint32_t n = g.last_frame.width * g.last_frame.height;
         const size_t need = (size_t)n * 4;
         if (need <= kShownBytes && dst && bytes >= need && vt_copy_pageable(dst, need) && ensure_shown()) {
-            if (vt_encode_srgb8(reinterpret_cast<const float4*>(g.rad), g.shown, n, g.stream) != 0 ||
-                hipStreamSynchronize(g.stream) != hipSuccess)
+            if (vt_encode_srgb8(reinterpret_cast<const float4*>(g.rad), g.shown, n, g.stream) != 0) {
+                set_err("read-back: the frame could not be encoded");
                 return -1;
+            }
+            const hipError_t e = hipStreamSynchronize(g.stream);
+            if (e != hipSuccess) {
+                set_err("read-back", e);
+                return -1;
+            }
             std::memcpy(dst, g.shown, need);
             return 0;
         }
-        if (vt_encode_srgb8(reinterpret_cast<const float4*>(g.rad), g.bgra, n, g.stream) != 0) return -1;
+        if (vt_encode_srgb8(reinterpret_cast<const float4*>(g.rad), g.bgra, n, g.stream) != 0) {
+            set_err("read-back: the frame could not be encoded");
+            return -1;
+        }
     }
     return read_frame(g.bgra, dst, bytes, 4);
 }

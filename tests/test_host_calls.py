@@ -140,3 +140,38 @@ def test_shown_frame_into_any_memory(fake, kind, width, height):
                                        ("page_locked", "k_encode_srgb8"), ("page_locked", "copy out")])
 def test_failed_read_of_the_shown_frame_says_so(fake, kind, fail):
     fake_hip.child(fake, "test_host_calls", "read_shown", kind, 64, 48, fail)
+
+
+# ---- a captured launch sequence: nothing has run, so nothing counts as zeroed by it --------------------------
+def serve_from_a_graph(hip):
+    from vtrace_amd import renderer, scenes, serving
+    loop = serving.ServingLoop(renderer.get_renderer(), memory_budget=1 << 22, max_work=1 << 14, streams=1, pipeline=1)
+    loop.add_scene(np.ones((1, 16), np.float32))
+    q = serving.Request(0, 32, 32, 1, scenes.perspective(1.0, 1.0), scenes.look_at((0.0, 0.0, 9.0), (0.0, 0.0, 0.0)), seed=1)
+    for k in range(3):
+        loop.submit(q)
+        if k == 2:
+            hip.fail("graph ")   # a replay that could not be queued leaves the counters in doubt
+        hip.clear()
+        try:
+            loop.step()
+        except renderer.RendererError:
+            assert k == 2
+        calls = [c.split(" grid")[0] for c in hip.lines() if c.startswith(("launch", "capture", "graph"))]
+        names = ["graph" if c.startswith("graph") else c for c in calls]
+        assert not any("capture" in c and ("k_accumulate" in c or "k_zero_counters" in c) for c in names), names
+        run = [c for c in names if not c.startswith("capture")]
+        if k == 0:   # new counters are zeroed, then the sequence runs and ends with the accumulation
+            assert len(run) == 3 and "k_zero_counters" in run[0] and run[1] == "graph" and "k_accumulate" in run[2], run
+            assert sum(c.startswith("capture") for c in names) == 6
+        elif k == 1:
+            assert len(run) == 2 and run[0] == "graph" and "k_accumulate" in run[1], run
+    hip.lib.hipGetLastError()
+    loop.submit(q)
+    hip.clear()
+    loop.step()
+    assert _count(hip, "k_zero_counters") == 1
+
+
+def test_captured_sequences_leave_the_counters_to_the_launches(fake):
+    fake_hip.child(fake, "test_host_calls", "serve_from_a_graph")

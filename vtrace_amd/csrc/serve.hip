@@ -476,7 +476,7 @@ int32_t vt_serve_step(int64_t* completed, uint32_t max_completed) {
             hipEvent_t after = k == 0 ? nullptr : sv.acc_done[k - 1];
             if (c.use_graph) {
                 hipGraphExec_t& gx = nsub == 1 ? sv.graph[deep ? 1 : 0] : sv.sub_graph[k][deep ? 1 : 0][nsub - 1];
-                if (!gx) rc = vt_trace_capture(c.max_bounces, deep, wk, sk, &gx, false, blocks);
+                if (!gx) rc = vt_trace_capture(c.max_bounces, deep, wk, sk, &gx, blocks);
                 if (rc == 0) rc = vt_trace_upload_tables(batch[k].data(), (uint32_t)batch[k].size(), wk, sk, nullptr);
                 if (rc == 0) rc = hipGraphLaunch(gx, sk) == hipSuccess ? 0 : -1;
                 if (rc == 0 && after) hipStreamWaitEvent(sk, after, 0);

@@ -2106,17 +2106,16 @@ int vt_trace_batch(const ReqGPU* reqs, uint32_t n, const WaveBuffers& wb, unsign
 }
 
 // Captures the launch sequence of a batch (fixed grids, tables read from device memory)
-// into a graph; the table upload stays outside the graph.
+// into a graph; the table upload and the accumulation (vt_trace_accumulate) stay outside the graph.
 int vt_trace_capture(uint32_t max_bounces, bool deep, const WaveBuffers& wb, hipStream_t s, hipGraphExec_t* out,
-                     bool with_acc, uint32_t blocks) {
+                     uint32_t blocks) {
     BatchGPU Bh{};
     Bh.max_bounces = max_bounces;
     hipGraph_t graph;
     if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) return -1;
-    int rc = deep ? launch_batch<false, true>(Bh, wb, nullptr, nullptr, nullptr, nullptr, s, nullptr, with_acc, blocks,
-                                              false)
-                  : launch_batch<false, false>(Bh, wb, nullptr, nullptr, nullptr, nullptr, s, nullptr, with_acc, blocks,
-                                               false);
+    // (without the accumulation, which marks the counters zeroed: nothing runs here)
+    int rc = deep ? launch_batch<false, true>(Bh, wb, nullptr, nullptr, nullptr, nullptr, s, nullptr, false, blocks, false)
+                  : launch_batch<false, false>(Bh, wb, nullptr, nullptr, nullptr, nullptr, s, nullptr, false, blocks, false);
     if (hipStreamEndCapture(s, &graph) != hipSuccess || rc != 0) return -1;
     rc = hipGraphInstantiate(out, graph, nullptr, nullptr, 0) == hipSuccess ? 0 : -1;
     hipGraphDestroy(graph);

@@ -303,8 +303,11 @@ __global__ __launch_bounds__(256) void k_conv3x3_split(ConvArgs a, uint32_t ntx,
 // double-buffered in LDS, the next one fetched into registers while the current one is computed: one
 // barrier a tile.
 // K is walked in steps of 32 as in the split form: k = tap CI + channel, 9 CI rounded up to whole steps
-// (CI: the input channels; a multiple of 16, fewer are padded with zeros), so every output is the same
-// sum in the same order there and here.  A pixel's neighbours in x follow it in LDS, so the 32 values
+// (CI: the input channels; a multiple of 16), so every output is the same sum in the same order there and here.
+// 8 channels (the output layer's gradient) are padded to 32: a step holds one tap where the split form's holds
+// four.  An MFMA adds its four groups of 8 products one after another, so the zeros between the taps change
+// nothing and the bits are the same all the same (test_gpu_conv_forms.py, with taps that cancel).
+// A pixel's neighbours in x follow it in LDS, so the 32 values
 // of a step that lies within one row of taps are at one offset for all of a row's pixels (CI an odd
 // multiple of 16: the second half of a step may lie in the next pixel, beyond its padding), and a
 // fragment read once feeds the steps of up to three output rows: ROWS + 2 reads for 3 ROWS MFMAs where

@@ -61,3 +61,18 @@ def test_volume_round_trip(d):
     want = idx[np.ix_(*ax)]   # the texel a voxel samples (nearest)
     occ = want != 0
     assert dense.shape == idx.shape and np.array_equal(dense[occ], want[occ]) and not np.any(dense[~occ])
+
+
+# sizes whose last chunk, and whose last 64 bytes, are not whole
+@pytest.mark.parametrize("w,h,d", [(301, 293, 289), (5, 65535, 77), (4097, 4099, 3)])
+def test_volume_of_an_odd_size_round_trip(w, h, d):
+    r = R.reset_renderer()
+    rng = np.random.default_rng(w)
+    idx = rng.integers(0, 3, (d, h, w), dtype=np.uint8)
+    tid = r.upload(scenes.Volume(idx, scenes.gen_palette(3)))
+    dense = r.volume_dense(tid)
+    ax = [np.floor((np.arange(n, dtype=np.float32) / np.float32(n)) * np.float32(n)).astype(np.int64).clip(0, n - 1)
+          for n in idx.shape]
+    want = idx[np.ix_(*ax)]
+    occ = want != 0
+    assert dense.shape == idx.shape and np.array_equal(dense[occ], want[occ]) and not np.any(dense[~occ])

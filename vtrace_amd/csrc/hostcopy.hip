@@ -4,14 +4,20 @@
 // fresh destination, 10 GB/s out; the link does 57.  Here a large copy is cut into chunks that
 // several threads stage through page-locked slots of their own, on two streams: the host copies and
 // page faults run side by side and overlap the transfers, and so do the transfers' starts and ends.
-// Measured, hipMemcpyAsync -> this (4 threads, 2 MB slots; 6 and 8 threads were no faster, 1 MB slots
-// or one stream 15-25 % slower from 32 MB on):
-//   in:  4 MB 160 -> 188 us, 8 MB 307 -> 298, 16 MB 587 -> 474, 33 MB 1142 -> 761, 66 MB 2239 -> 1392
-//   out, fresh destination: 2 MB 262 -> 222 us, 4 MB 457 -> 312, 8 MB 785 -> 418, 33 MB 3400 -> 1076
-//   out, warm destination:  2 MB 145 -> 165 us, 4 MB 243 -> 244, 8 MB 512 -> 333, 33 MB 1921 -> 906
-// Out, that sets the size it starts at.  In, it starts at 24 MB, arrays the caches do not hold: the threads leave
-// lines of the program's memory in other cores' caches, and writing that memory anew then takes
-// 0.27 us a page (a 16 MB array made for each call 1.5 -> 2.6 ms, for 0.11 ms gained here).
+// A copy is paid for by the whole program: the threads also leave lines of its arrays in their own caches,
+// and writing such an array anew, or an array in the pages that it gave back, then takes longer.  So in
+// (fill_slot) the program's lines are prefetched past all but the first cache, and the sizes it starts at are
+// set by the copy and the next pass over the array together.  Measured, hipMemcpyAsync -> this, us (4 threads, 2 MB
+// slots, 32 MB of last-level cache; 6 and 8 threads were no faster, 1 MB slots or one stream 15-25 % slower):
+//   in, and the next array's writing before it (fresh pages):
+//     16 MB 586 + 270 -> 429 + 262, 24 MB 894 + 537 -> 580 + 424, 33 MB 1204 + 1126 -> 763 + 1042, 66 MB 2358 + 4569 -> 1572 + 4775
+//     (without the prefetch 434 + 286, 593 + 475, 754 + 1107, 1541 + 5468)
+//   out, and reading the result (fresh destination):
+//     2 MB 135 + 62 -> 155 + 55, 4 MB 252 + 134 -> 230 + 98, 8 MB 527 + 276 -> 357 + 265, 33 MB 2484 + 1112 -> 1305 + 1104
+// Out, it starts at 4 MB.  In, at 24 MB: a program that makes its 16 MB array out of others (a shifted 256^3
+// volume) writes it in 1.80 ms instead of 1.46, for 0.04 gained in the copy, while frames of 33 and 66 MB from the
+// device lose nothing (prepared in 17.9 ms, denoised in 5.85 ms without staging in, 4.58 with; 18.7 and 4.53 without
+// the prefetch).
 //
 // The threads are started by the first copy that is large enough, sleep between copies, and end with
 // vt_copy_release().  One copy runs at a time (the callers hold the runtime lock; the engine has its
@@ -76,12 +82,14 @@ struct Engine {
 std::mutex g_copy_lock;
 Engine* g_engine = nullptr;     // never destroyed at exit: its threads may be asleep in it
 
-// Into a slot, which the device reads next: stores past the caches, which the slots would push the program's
-// own data out of.
+// Into a slot, which the device reads next: stores past the caches, which the slots would push the program's own
+// data out of, and loads that leave its lines in none but the first (see above).
 void fill_slot(char* dst, const char* src, size_t n) {
     typedef long long v2 __attribute__((vector_size(16)));
+    constexpr size_t kAhead = 1024;
     size_t i = 0;
     for (; i + 64 <= n; i += 64) {
+        if (i + kAhead < n) __builtin_prefetch(src + i + kAhead, 0, 0);   // (non-temporal)
         v2 v[4];
         std::memcpy(v, src + i, 64);
         for (int k = 0; k < 4; ++k) __builtin_nontemporal_store(v[k], reinterpret_cast<v2*>(dst + i) + k);

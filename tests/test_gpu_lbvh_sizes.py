@@ -53,3 +53,10 @@ def test_lbvh_at_the_edges_of_its_forms(kind, n):
     r.refit_instances(sent)
     again, _ = r.lbvh()
     assert np.array_equal(again.view(np.uint32).reshape(-1, 8), o_nodes)
+
+
+@pytest.mark.parametrize("kind,n", [("scattered", 10239), ("scattered", 10240), ("scattered", 10241), ("equal", 10240),
+                                    ("equal", 10241)])
+def test_lbvh_where_counting_ends(kind, n):
+    """The codes of up to 10240 instances are sorted by counting, of more by the radix sort."""
+    test_lbvh_at_the_edges_of_its_forms(kind, n)

@@ -33,9 +33,9 @@ constexpr uint32_t kOneMax = 512;         // one thread per instance
 // k_refit_one: the boxes, links and counters of 4096 instances' inner nodes fill 144 of 160 KB of LDS
 constexpr uint32_t kRefitOneMax = 4096;
 constexpr int kRefitLeaves = 4;           // leaves per thread: kRefitOneMax / 1024
-// k_rank_sort compares every pair of codes: with bounds and codes 18 us for 4096, 64 us for 16384, against
-// 77 us in 14 launches for the radix sort's at 16384; four times as much at twice as many.
-constexpr uint32_t kRankMax = 16384;
+// k_rank_sort compares every pair of codes: an update (codes, tree and boxes) of 8000 instances takes 165 us with it
+// and 178 with the radix sort, of 10000 189 and 193, of 12000 212 and 209, of 16384 262 and 248.
+constexpr uint32_t kRankMax = 10240;
 constexpr uint32_t kRankKeys = 64;        // keys a workgroup ranks
 constexpr uint32_t kPrepThreads = 256;
 // The mark behind a refit's first launch costs 5 us (of 30 for 16 instances, of 100 for 8000), which a program

@@ -175,3 +175,27 @@ def serve_from_a_graph(hip):
 
 def test_captured_sequences_leave_the_counters_to_the_launches(fake):
     fake_hip.child(fake, "test_host_calls", "serve_from_a_graph")
+
+
+# ---- the BF16 weights are made anew until that has succeeded ------------------------------------------
+def prepared_weights_fail(hip):
+    from vtrace_amd import denoise, renderer
+    net = denoise.Denoiser(renderer.get_renderer(), seed=1)
+    rad, gbuf = np.ones((32, 32, 4), np.float32), np.ones((32, 32, 8), np.float32)
+    net.denoise(rad, gbuf, 1)
+    net.set_params(net.get_params())
+    hip.clear()
+    hip.fail("k_prep_weights")
+    with pytest.raises(renderer.RendererError):
+        net.denoise(rad, gbuf, 1)
+    assert _count(hip, "k_conv3x3") == 0
+    hip.clear()
+    net.denoise(rad, gbuf, 1)
+    assert _count(hip, "k_prep_weights") == 1 and _count(hip, "k_conv3x3") == 19
+    hip.clear()
+    net.denoise(rad, gbuf, 1)
+    assert _count(hip, "k_prep_weights") == 0
+
+
+def test_weights_are_prepared_again_after_a_failure(fake):
+    fake_hip.child(fake, "test_host_calls", "prepared_weights_fail")

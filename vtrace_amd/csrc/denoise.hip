@@ -1340,13 +1340,15 @@ void wgrad_of(int li, const Tensor& x, const Tensor& g, const Tensor* up = nullp
     a.g_stride = g.C;
 }
 
-void prep_weights(hipStream_t s) {
-    if (!net.weights_dirty) return;
+int prep_weights(hipStream_t s) {
+    if (!net.weights_dirty) return 0;
     uint32_t total = 0;
     for (auto& L : net.L) total += L.d.nw;
     hipLaunchKernelGGL(k_prep_weights, dim3(blocks(total)), dim3(256), 0, s, net.params, net.ldev, (uint32_t)kLayers,
                        net.wb, net.wt, total);
+    if (hipGetLastError() != hipSuccess) return -1;
     net.weights_dirty = false;
+    return 0;
 }
 
 // forward pass on net.x0 (N x H x W, H and W multiples of 16) -> net.y
@@ -1354,7 +1356,7 @@ void prep_weights(hipStream_t s) {
 // holds the skip, in its channels of the concatenation, or (dense: inference) by itself, pixel by
 // pixel: half of each 160 B row of the level-0 concatenation lies in lines that the other half shares.
 int forward(uint32_t N, uint32_t H, uint32_t W, hipStream_t s, bool dense = false) {
-    prep_weights(s);
+    if (prep_weights(s) != 0) return -1;
     int rc = 0;
     Tensor in = net.x0;
     for (int l = 0; l < 4 && rc == 0; ++l) {

@@ -107,12 +107,20 @@ struct Ctr<true> {
     }
     __device__ __forceinline__ void hit() { c[VT_STAT_HITS]++; }
     __device__ __forceinline__ void steps(uint32_t n) { c[VT_STAT_STEPS] += n; }
+    // Called by every thread of the workgroup at the kernel's end.  The waves' sums meet in LDS, so that a
+    // workgroup adds to memory once: waves that start together end together, and their atomics on one
+    // address wait for each other (a counted mode-0 frame at 1920 x 1080 217 us; 490 with one add per wave and counter).
     __device__ void flush(unsigned long long* out) {
+        __shared__ unsigned long long sum[VT_STAT_COUNT];
+        if (threadIdx.x < VT_STAT_COUNT) sum[threadIdx.x] = 0ull;
+        __syncthreads();
         for (int k = 0; k < VT_STAT_COUNT; ++k) {
             unsigned long long v = c[k];
             for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-            if ((threadIdx.x & 63) == 0 && v) atomicAdd(&out[k], v);
+            if ((threadIdx.x & 63) == 0 && v) atomicAdd(&sum[k], v);
         }
+        __syncthreads();
+        if (threadIdx.x < VT_STAT_COUNT && sum[threadIdx.x]) atomicAdd(&out[threadIdx.x], sum[threadIdx.x]);
     }
 };
 

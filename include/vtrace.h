@@ -181,8 +181,10 @@ int32_t vt_bench_frames(uint32_t warmup, uint32_t iters, float* kernel_ms, float
 int32_t vt_read_volume(int32_t id, void* dst, uint64_t bytes);
 int32_t vt_volume_info(int32_t id, uint32_t* info8);
 /* The volume's brick map (one u32 per 8^3 brick, x-fastest brick order): a non-empty brick's
- * id, or 0xFFFFFF00 | r for an empty brick, r = radius of the cube of empty bricks around it
- * (L-inf brick distance to the nearest non-empty brick - 1, at most 31). */
+ * id (below 0xE0000000), or for an empty brick 0xE0000000 | r << 24 | (K_o - 1) << 3 o, o = 0..7:
+ * r = radius of the cube of empty bricks around it (L-inf brick distance to the nearest non-empty
+ * brick - 1, at most 31), K_o = side in bricks of the largest empty cube that has it as its corner
+ * towards octant o (bit a of o: towards -axis a), at most 8. */
 int32_t vt_read_brick_map(int32_t id, uint32_t* dst, uint64_t bytes);
 /* LBVH of the current instances: (2n-1) x 32 B nodes and n x 128 B instance records. */
 int32_t vt_read_lbvh(void* nodes, uint64_t node_bytes, void* instances, uint64_t inst_bytes);

@@ -917,8 +917,8 @@ int32_t vt_read_stage_stats(uint64_t* dst, uint32_t max_stages, uint8_t* kinds) 
 
 float vt_last_frame_ms(void) { return g.last_ms; }
 
-// Whole frames as render_tick renders them (two streams for path-traced frames of 2+ samples,
-// each frame complete before the next starts): kernel_ms = mean GPU time per frame (HIP events
+// Whole frames as render_tick renders them (large path-traced ones in chunks of tile rows, each frame
+// complete before the next starts): kernel_ms = mean GPU time per frame (HIP events
 // around each frame), wall_ms = mean host time per frame including the per-frame wait.
 int32_t vt_bench_frames(uint32_t warmup, uint32_t iters, float* kernel_ms, float* wall_ms) {
     Guard G;

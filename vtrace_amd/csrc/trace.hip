@@ -2064,8 +2064,8 @@ static int launch_own(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long l
 }
 
 // Alone on the GPU (blocks = 0), every workgroup of a launch is resident, so its waves start on
-// tiles of their own.  A captured launch sequence (no work counted in Bh) runs with any batch, so it
-// keeps the full grid and hands out everything by its counters.
+// tiles of their own.  A captured launch sequence (no work counted in Bh: the serving loop's default) runs with any
+// batch, so it keeps the full grid and hands out everything by its counters.
 template <bool ST, bool DEEP>
 static int launch_batch(const BatchGPU& Bh, const WaveBuffers& wb, unsigned long long* stats, hipEvent_t* ev,
                         uint8_t* kinds, uint32_t* nstages, hipStream_t s, hipEvent_t acc_after = nullptr,
